@@ -50,36 +50,36 @@ def listed():
     return [
         # the 10x10 lattice, 1e5 humans, one year: the smallest simulation a
         # user runs (a first look, a unit test), bound by launches
-        _sim("lattice 10x10, 365 d", "lattice", 1, 10, 1000, 365),
+        _sim("lattice 10x10", "lattice", 1, 10, 1000, 365),
         # the reference's own parameter set (one serotype, introductions,
         # stochastic-rounding counts) on ragged communities with every output
         # file's data kept and the census read back, launched day by day
-        _sim("reference set, outputs kept", "reference", 1, 17, 300, 200, graph=False, keep=True),
+        _sim("reference set kept", "reference", 1, 17, 300, 200, graph=False, keep=True),
         # a fit of the climate coefficients: 16 chains' proposals, one year of
         # days whose parameters and lifetimes change daily
-        _sim("climate fit, 16 chains", "climate", 16, 12, 400, 363),
+        _sim("climate fit", "climate", 16, 12, 400, 363),
         # one iteration of the 64-chain fit: 1e6 humans in 32x32 communities
         # per chain, 260 weeks
-        _sim("fit iteration, 64 chains", "fit", 64, 32, 977, 1819),
+        _sim("fit iteration", "fit", 64, 32, 977, 1819),
         # the 100x100 lattice, 1e7 humans, prior immunity, ten years
-        _sim("lattice 100x100, 3650 d", "lattice", 1, 100, 1000, 3650),
+        _sim("lattice 100x100", "lattice", 1, 100, 1000, 3650),
         # a batch of simulations of uneven lattices and communities, through
         # its epidemic: the training data of the surrogate and the benchmark
-        _sim("batch of 64 uneven", "batch", 64, 53, 1100, 150, graph=False),
+        _sim("uneven batch", "batch", 64, 53, 1100, 150, graph=False),
         # few large communities (cities of 3,000 to 21,000 humans), whose
         # bitmaps need several waves each
-        _sim("cities 7x7", "cities", 1, 7, 9000, 180),
+        _sim("cities", "cities", 1, 7, 9000, 180),
         # surrogate: a serving loop's device-buffer call, 64 rows
-        _mlp("forward, device, 64 rows", "noalloc", 64),
+        _mlp("device forward 64", "noalloc", 64),
         # the first stage of screened delayed acceptance, 64 chains
-        _mlp("forward, 64 rows", "forward", 64),
+        _mlp("forward 64", "forward", 64),
         # a Langevin step's gradient, 64 chains
-        _mlp("input gradient, 64 rows", "input_grad", 64),
+        _mlp("input gradient 64", "input_grad", 64),
         # validation of a trained network, the largest batch train_surrogate
         # allows
-        _mlp("forward, 4096 rows", "forward", 4096),
+        _mlp("forward 4096", "forward", 4096),
         # training on 50,000 runs in minibatches of 512 (the last one ragged)
-        _mlp("training, 2 epochs", "train", 50000, epochs=2),
+        _mlp("training", "train", 50000, epochs=2),
     ]
 
 
