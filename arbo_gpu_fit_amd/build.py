@@ -22,7 +22,7 @@ LIB = os.path.join(OUT_DIR, "libarbo_hip.so")
 
 SOURCES = ["arbo_kernels.hip", "arbo_engine.cpp", "arbo_tables.cpp", "arbo_mcmc.cpp", "arbo_surrogate.hip", "arbo_output.cpp",
            "arbo_data.cpp"]
-HEADERS = ["arbo_rng.h", "arbo_device.h", "arbo_tables.h"]
+HEADERS = ["arbo_rng.h", "arbo_device.h", "arbo_tables.h", "arbo_surrogate_fused.h"]
 
 ARCH = os.environ.get("ARBO_OFFLOAD_ARCH", "gfx950")
 

@@ -1,11 +1,15 @@
 // arbo_surrogate.hip — the surrogate MLP on gfx950: matrix products on the
 // bfloat16 MFMA units with float32 accumulation, fused bias / GELU / GELU
-// gradient / bias-gradient epilogues, the Poisson loss, and Adam.
+// gradient epilogues, the Poisson loss, and Adam.
 //
-// One kernel does every matrix product of the forward and backward passes:
-// C[i, j] = sum_k A(i, k) B(j, k), each operand float32 in memory with its
-// own strides (one of them 1), so X W^T (forward), dZ W (input gradients)
-// and dZ^T X (weight gradients over the batch) are the same code.
+// Networks whose layers are at most 512 wide and whose row tile fits a CU's
+// LDS (fits_tile; the fit's 6-256^4-260 among them) run the row-tile kernels
+// of arbo_surrogate_fused.h: a pass is one launch, a training step two.
+//
+// The others run a product a launch, C[i, j] = sum_k A(i, k) B(j, k), each
+// operand float32 in memory with its own strides (one of them 1), so X W^T
+// (forward), dZ W (input gradients) and dZ^T X (weight gradients over the
+// batch) are the same code.
 //  * A workgroup of four wave64s computes a 64 x 64 block of C; each wave one
 //    32 x 32 tile with v_mfma_f32_32x32x16_bf16 (16-deep k-steps, float32
 //    accumulators, 16 per lane).
@@ -23,11 +27,9 @@
 //  * The weight-gradient product appends a column of ones to its B operand,
 //    so the bias gradient (the batch sum of dZ) comes out of the same launch,
 //    and the weight gradients of all layers, independent once the input
-//    gradients are known, share one launch (k_gemm_group): a training step
-//    is then 5 forward products, 4 input-gradient products and one grouped
-//    launch, where each launch costs about 5 us whatever its size.
-// Parameters stay float32 and are read by the products directly, so an
-// Adam step needs no repacking.
+//    gradients are known, share one launch (k_gemm_group).
+// Parameters stay float32; k_gemm reads them directly, k_mlp reads the packed
+// halves that set_params and every Adam update write.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -67,10 +69,34 @@ __host__ __device__ inline float bf2f(uint16_t h) {
     return f;
 }
 
-__device__ inline float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-__device__ inline float gelu_grad(float z) {
-    return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+// GELU z Phi(z) and, where wanted, its derivative Phi(z) + z phi(z), from
+// erfc(x) = exp(-x^2) t P(t), t = 1 / (1 + p x), x = |z| / sqrt(2): the form
+// of Cody (1969) and of Press et al.'s erfc, P of degree 8 fitted here to
+// exp(x^2) erfc(x) on [0, 7] by iteratively reweighted least squares
+// (relative error 1.0e-8 before rounding).  About 25 operations for both and
+// no branch, where erff and expf take some 150 on both sides of a divergent
+// one, which a row tile's 4,096 activations a layer made 1.7 us of; against
+// 64 bits over [-9, 9] at most 3.8e-7 (with erff 4.5e-7), rms 4.7e-8 (5.4e-8).
+struct Gelu { float h, grad; };
+__device__ __forceinline__ Gelu gelu_pair(float z) {
+    const float x = fabsf(z) * 0.70710678118654752f;
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(x, 0.475f, 1.0f));
+    float q = -0.053407583385705948f;
+    q = __builtin_fmaf(q, t, 0.29242432117462158f);
+    q = __builtin_fmaf(q, t, -0.59631341695785522f);
+    q = __builtin_fmaf(q, t, 0.48363786935806274f);
+    q = __builtin_fmaf(q, t, -0.13959354162216187f);
+    q = __builtin_fmaf(q, t, 0.25286203622817993f);
+    q = __builtin_fmaf(q, t, 0.22282379865646362f);
+    q = __builtin_fmaf(q, t, 0.26965680718421936f);
+    q = __builtin_fmaf(q, t, 0.26790973544120789f);
+    const float e = __builtin_amdgcn_exp2f(-0.5f * z * z * 1.4426950408889634f);   // exp(-z^2 / 2)
+    const float c = 0.5f * q * t * e;                                              // Phi(-|z|)
+    const float cdf = z >= 0.0f ? 1.0f - c : c;
+    return Gelu{z * cdf, __builtin_fmaf(z * 0.39894228040143268f, e, cdf)};
 }
+__device__ inline float gelu(float z) { return gelu_pair(z).h; }
+__device__ inline float gelu_grad(float z) { return gelu_pair(z).grad; }
 
 enum : uint32_t {
     EPI_STORE = 0,       // outf = acc (with ones: column N - 1 to outb)
@@ -323,6 +349,14 @@ __global__ void k_zero_f32(float* __restrict__ p, uint64_t n) {
     if (i < n) p[i] = 0.0f;
 }
 
+}  // namespace
+}  // namespace arbo
+
+#include "arbo_surrogate_fused.h"
+
+namespace arbo {
+namespace {
+
 template <class T>
 struct Buf {
     T* p = nullptr;
@@ -377,6 +411,13 @@ struct ArboSurrogate {
     Buf<double> epoch_sum;          // the loss summed over one training epoch
     Buf<float> data_x, data_y;
     Buf<uint32_t> idx;
+    // networks that fit k_mlp (fits_tile): the weights' packed halves and the
+    // arrays between k_mlp and k_wgrad; H[0] and Z[L-1] hold the rows' inputs
+    // and outputs, the other layers' H, Z and dZ are not there
+    bool fused = false;
+    Buf<uint16_t> pack;
+    std::vector<uint32_t> foff, boffk;   // each layer's forward and backward fragments (bytes)
+    std::vector<Buf<uint16_t>> HT, DT;   // layer inputs and dZ as operands of k_wgrad
     float* scratch = nullptr;       // this device's no-allocation activation buffers
     uint64_t adam_t = 0;
     std::string err;
@@ -529,8 +570,152 @@ int backward(ArboSurrogate* s, uint32_t B, bool want_w, bool want_x) {
     return ARBO_OK;
 }
 
+// Whether k_mlp takes a network: every layer within its column tiles, and a
+// row tile's two activation buffers, biases and gelu'(z) within a CU's 160 KB
+// of LDS.  Wider or deeper networks run a product a launch (k_gemm).
+bool fits_tile(const std::vector<uint32_t>& w) {
+    uint32_t widest = 0, floats = 0;
+    for (size_t l = 0; l < w.size(); ++l) {
+        widest = std::max(widest, w[l]);
+        if (l > 0) floats += blocks(w[l], 32) * 32;
+        if (l > 0 && l + 1 < w.size()) floats += kFuseRows * gg_row(w[l]);
+    }
+    if (widest > kFuseWidth) return false;
+    const uint32_t ldk = blocks(widest, kGroupK) * kGroupK + 8;
+    return 4 * kFuseRows * ldk * sizeof(uint16_t) + 4 * floats + 1024 <= 160 * 1024;
+}
+
+// The row-tile pass of a fused network over n rows: forward stages, then the
+// backward ones (down to the inputs, or to layer 1 when only the dZ are
+// wanted).
+PassArgs pass_args(const ArboSurrogate* s, uint32_t mode, uint32_t n) {
+    PassArgs a{};
+    const uint32_t L = s->L;
+    a.n = n;
+    a.L = L;
+    a.w0 = s->w[0];
+    a.pack = s->pack.p;
+    a.pack_bytes = (uint32_t)(s->pack.n * sizeof(uint16_t));
+    a.x = s->H[0].p;
+    uint32_t k = 0, widest = 0, buf = 0, lds = 0;   // lds: floats behind the activations
+    // the stages of one layer's product; its result becomes the next one's input
+    auto product = [&](uint32_t kind, uint32_t off, uint32_t K, uint32_t N, uint32_t bias_at, uint32_t gg_at, uint16_t* t) {
+        const uint32_t tiles = blocks(N, 16);
+        for (uint32_t t0 = 0; t0 < tiles; t0 += kFuseCols / 16) {
+            Stage& g = a.st[k++];
+            g.off = off;
+            g.K = K;
+            g.N = N;
+            g.steps = blocks(K, 32);
+            g.groups = blocks(g.steps, kGroup);
+            g.tiles = tiles;
+            g.tile0 = t0;
+            g.buf = buf;
+            g.bias_at = bias_at;
+            g.gg_at = gg_at;
+            g.t = t0 == 0 ? t : nullptr;
+            g.kind = kind;
+        }
+        buf ^= 1u;
+        widest = std::max(widest, K);
+        if (mode != PASS_FORWARD && kind != STAGE_INPUT) widest = std::max(widest, N);
+    };
+    for (uint32_t l = 0; l < L; ++l) {   // biases, padded to the 32 columns a stage's end reads
+        a.bias[l] = Bias{s->P.p + s->boff[l], lds, s->w[l + 1]};
+        lds += blocks(s->w[l + 1], 32) * 32;
+    }
+    uint32_t gg[ARBO_SUR_MAX_LAYERS] = {};
+    for (uint32_t l = 0; l + 1 < L && mode != PASS_FORWARD; ++l) {
+        gg[l] = lds;
+        lds += kFuseRows * gg_row(s->w[l + 1]);
+    }
+    for (uint32_t l = 0; l < L; ++l)
+        product(l + 1 < L ? STAGE_HIDDEN : STAGE_OUTPUT, s->foff[l], s->w[l], s->w[l + 1], a.bias[l].at, gg[l],
+                s->HT[l].p);
+    if (mode != PASS_FORWARD) {
+        for (uint32_t l = L - 1; l > 0; --l)
+            product(STAGE_BACK, s->boffk[l], s->w[l + 1], s->w[l], 0, gg[l - 1], s->DT[l].p);
+        if (mode == PASS_INPUT) product(STAGE_INPUT, s->boffk[0], s->w[1], s->w[0], 0, 0, nullptr);
+    }
+    a.stages = k;
+    a.tz = s->DT[0].p;
+    a.tzn = s->w[1];
+    a.ldk = blocks(widest, kGroupK) * kGroupK + 8;   // rows 4 LDS words apart mod 64: a wave's 16-byte operand
+                                                     // reads touch every bank once
+    a.lds = 4 * kFuseRows * a.ldk * (uint32_t)sizeof(uint16_t) + 4 * lds;
+    return a;
+}
+
+template <uint32_t MODE>
+hipError_t launch_pass(const PassArgs& a, hipStream_t st) {
+    uint32_t tiles = 1;
+    for (uint32_t k = 0; k < a.stages; ++k) tiles = std::max(tiles, a.st[k].tiles);
+    const dim3 grid(blocks(a.n, kFuseRows)), block(kFuseThreads);
+    if (tiles <= kFuseWaves) hipLaunchKernelGGL((k_mlp<MODE, 1>), grid, block, a.lds, st, a);   // one tile a wave
+    else hipLaunchKernelGGL((k_mlp<MODE, 2>), grid, block, a.lds, st, a);
+    return hipGetLastError();
+}
+
+// Weight and bias gradients of the last PASS_LOSS pass of n rows; adam: the
+// update instead of the gradients.
+hipError_t launch_wgrad(ArboSurrogate* s, uint32_t n, bool adam, float lr, float c1, float c2) {
+    GradArgs g{};
+    g.L = s->L;
+    g.steps = blocks(n, kFuseRows);
+    g.P = s->P.p;
+    g.G = s->G.p;
+    g.M = s->Mo.p;
+    g.V = s->Vo.p;
+    g.pack = s->pack.p;
+    g.lr = lr;
+    g.c1 = c1;
+    g.c2 = c2;
+    uint32_t wg = 0;
+    for (uint32_t l = 0; l < s->L; ++l) {
+        GradLayer& y = g.l[l];
+        y.N = s->w[l + 1];
+        y.K = s->w[l];
+        y.first = wg;
+        y.tx = blocks(y.K, 32);
+        wg += y.tx * blocks(y.N, 32);
+        y.dz = s->DT[l].p;
+        y.h = s->HT[l].p;
+        y.w = s->woff[l];
+        y.b = s->boff[l];
+        y.foff = s->foff[l];
+        y.boff = s->boffk[l];
+        y.ftiles = (y.N + 15) / 16;
+        y.btiles = (y.K + 15) / 16;
+    }
+    if (adam) hipLaunchKernelGGL((k_wgrad<true>), dim3(wg), dim3(64 * kGradWaves), 0, s->stream, g);
+    else hipLaunchKernelGGL((k_wgrad<false>), dim3(wg), dim3(64 * kGradWaves), 0, s->stream, g);
+    return hipGetLastError();
+}
+
+// The packed halves of every layer's weights from the parameters.
+hipError_t launch_pack(ArboSurrogate* s) {
+    for (uint32_t l = 0; l < s->L; ++l) {
+        const uint32_t N = s->w[l + 1], K = s->w[l];
+        hipLaunchKernelGGL(k_pack, dim3(blocks((uint64_t)N * ((K + 1) / 2), 256)), dim3(256), 0, s->stream, s->P.p + s->woff[l], N,
+                           K, s->foff[l], (N + 15) / 16, s->boffk[l], (K + 15) / 16, s->pack.p);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
+}
+
 int upload_x(ArboSurrogate* s, uint32_t n, const float* x) {
     SUR_TRY(s, hipMemcpyAsync(s->H[0].p, x, (size_t)n * s->w[0] * 4, hipMemcpyHostToDevice, s->stream));
+    return ARBO_OK;
+}
+
+// Sum of the loss's nb per-workgroup sums (synchronises).
+int sum_parts(ArboSurrogate* s, uint32_t nb, double* loss) {
+    std::vector<double> h(nb);
+    SUR_TRY(s, hipMemcpyAsync(h.data(), s->part.p, nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    SUR_TRY(s, hipStreamSynchronize(s->stream));
+    double t = 0.0;
+    for (double v : h) t += v;
+    *loss = t;
     return ARBO_OK;
 }
 
@@ -544,20 +729,19 @@ int poisson(ArboSurrogate* s, uint32_t B, const float* y, float scale, double* l
     hipLaunchKernelGGL(k_poisson, dim3(nb), dim3(256), 0, s->stream, s->Z[s->L - 1].p, y, rows, out, n, scale,
                        s->dZ[s->L - 1].p, s->part.p, acc);
     SUR_TRY(s, hipGetLastError());
-    if (loss) {
-        std::vector<double> h(nb);
-        SUR_TRY(s, hipMemcpyAsync(h.data(), s->part.p, nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-        SUR_TRY(s, hipStreamSynchronize(s->stream));
-        double t = 0.0;
-        for (double v : h) t += v;
-        *loss = t;
-    }
-    return ARBO_OK;
+    return loss ? sum_parts(s, nb, loss) : (int)ARBO_OK;
+}
+
+// Advances the Adam step and gives its bias corrections.
+void adam_next(ArboSurrogate* s, float* c1, float* c2) {
+    s->adam_t++;
+    *c1 = 1.0f - std::pow(0.9f, (float)s->adam_t);
+    *c2 = 1.0f - std::pow(0.999f, (float)s->adam_t);
 }
 
 int adam_step(ArboSurrogate* s, float lr) {
-    s->adam_t++;
-    const float c1 = 1.0f - std::pow(0.9f, (float)s->adam_t), c2 = 1.0f - std::pow(0.999f, (float)s->adam_t);
+    float c1, c2;
+    adam_next(s, &c1, &c2);
     hipLaunchKernelGGL(k_adam, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->P.p, s->G.p, s->Mo.p,
                        s->Vo.p, (uint64_t)s->n_params, lr, c1, c2);
     SUR_TRY(s, hipGetLastError());
@@ -603,14 +787,38 @@ ARBO_API int arbo_sur_create(int32_t device, uint32_t n_widths, const uint32_t* 
     if (!rc) rc = alloc(s, s->G, off);
     if (!rc) rc = alloc(s, s->Mo, off);
     if (!rc) rc = alloc(s, s->Vo, off);
+    s->fused = fits_tile(s->w);
     for (uint32_t l = 0; l < s->L && !rc; ++l) {
-        rc = alloc(s, s->Z[l], (size_t)max_batch * s->w[l + 1]);
-        if (!rc) rc = alloc(s, s->H[l], (size_t)max_batch * s->w[l]);
-        if (!rc) rc = alloc(s, s->dZ[l], (size_t)max_batch * s->w[l + 1]);
+        if (l + 1 == s->L || !s->fused) rc = alloc(s, s->Z[l], (size_t)max_batch * s->w[l + 1]);
+        if (!rc && (l == 0 || !s->fused)) rc = alloc(s, s->H[l], (size_t)max_batch * s->w[l]);
+        if (!rc && !s->fused) rc = alloc(s, s->dZ[l], (size_t)max_batch * s->w[l + 1]);
+    }
+    if (s->fused) {
+        const size_t bpad = (size_t)blocks(max_batch, kFuseRows) * kFuseRows;
+        s->HT.resize(s->L);
+        s->DT.resize(s->L);
+        uint32_t pk = 0;   // bytes: a few MB within the LDS limit on widths and depth
+        for (uint32_t l = 0; l < s->L && !rc; ++l) {
+            const uint32_t K = s->w[l], N = s->w[l + 1];
+            s->foff.push_back(pk);
+            pk += blocks(K, 32) * blocks(N, 16) * (4 * kFrag);
+            s->boffk.push_back(pk);
+            pk += blocks(N, 32) * blocks(K, 16) * (4 * kFrag);
+            rc = alloc(s, s->HT[l], 2 * bpad * 32 * blocks(K, 32));
+            if (!rc) rc = alloc(s, s->DT[l], 2 * bpad * 32 * blocks(N, 32));
+        }
+        // a stage's offsets run up to 15 tiles past a layer's last one (not read: kNoFrag), and stay inside
+        pk += 32 * (4 * kFrag);
+        if (!rc) rc = alloc(s, s->pack, pk / 2);
+        if (!rc) {   // fragments past a layer's last row or column stay zero
+            hipLaunchKernelGGL(k_zero_f32, dim3(blocks(pk / 4, 256)), dim3(256), 0, s->stream,
+                               reinterpret_cast<float*>(s->pack.p), (uint64_t)pk / 4);
+            if (hipGetLastError() != hipSuccess) rc = ARBO_E_DEVICE;
+        }
     }
     if (!rc) rc = alloc(s, s->dxin, (size_t)max_batch * s->w[0]);
     if (!rc) rc = alloc(s, s->yin, (size_t)max_batch * s->w[s->L]);
-    if (!rc) rc = alloc(s, s->part, blocks((uint64_t)max_batch * s->w[s->L], 256));
+    if (!rc) rc = alloc(s, s->part, std::max(blocks((uint64_t)max_batch * s->w[s->L], 256), blocks(max_batch, kFuseRows)));
     if (!rc) rc = alloc(s, s->epoch_sum, 1);
     if (rc) {
         arbo_sur_destroy(s);
@@ -669,6 +877,7 @@ ARBO_API int arbo_sur_set_params(ArboSurrogate* s, const float* in) {
     hipLaunchKernelGGL(k_zero_f32, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->Vo.p,
                        (uint64_t)s->n_params);
     SUR_TRY(s, hipGetLastError());
+    if (s->fused) SUR_TRY(s, launch_pack(s));
     s->adam_t = 0;
     SUR_TRY(s, hipStreamSynchronize(s->stream));
     return ARBO_OK;
@@ -679,7 +888,13 @@ ARBO_API int arbo_sur_forward(ArboSurrogate* s, uint32_t n, const float* x, floa
     if (n > s->max_batch) return fail(s, ARBO_E_CAPACITY, "more rows than max_batch");
     SUR_TRY(s, hipSetDevice(s->device));
     if (int rc = upload_x(s, n, x)) return rc;
-    if (int rc = forward(s, n)) return rc;
+    if (s->fused) {
+        PassArgs a = pass_args(s, PASS_FORWARD, n);
+        a.out = s->Z[s->L - 1].p;
+        SUR_TRY(s, launch_pass<PASS_FORWARD>(a, s->stream));
+    } else if (int rc = forward(s, n)) {
+        return rc;
+    }
     SUR_TRY(s, hipMemcpyAsync(out, s->Z[s->L - 1].p, (size_t)n * s->w[s->L] * 4, hipMemcpyDeviceToHost, s->stream));
     SUR_TRY(s, hipStreamSynchronize(s->stream));
     return ARBO_OK;
@@ -694,6 +909,13 @@ ARBO_API int arbo_sur_forward_noalloc(ArboSurrogate* s, uint32_t n, const float*
     if (!s->scratch) return fail(s, ARBO_E_STATE, "no scratch address on this device");
     SUR_TRY(s, hipSetDevice(s->device));
     const hipStream_t st = stream ? static_cast<hipStream_t>(stream) : s->stream;
+    if (s->fused) {   // the activations stay on chip
+        PassArgs a = pass_args(s, PASS_FORWARD, n);
+        a.x = x;
+        a.out = out;
+        SUR_TRY(s, launch_pass<PASS_FORWARD>(a, st));
+        return ARBO_OK;
+    }
     float* buf[2] = {s->scratch, s->scratch + kScratchElems};
     for (uint32_t l = 0; l < s->L; ++l) {   // the products of forward(), activations ping-ponged in the scratch
         const uint32_t K = s->w[l], N = s->w[l + 1];
@@ -724,10 +946,19 @@ ARBO_API int arbo_sur_input_grad(ArboSurrogate* s, uint32_t n, const float* x, c
     if (n > s->max_batch) return fail(s, ARBO_E_CAPACITY, "more rows than max_batch");
     SUR_TRY(s, hipSetDevice(s->device));
     if (int rc = upload_x(s, n, x)) return rc;
-    if (int rc = forward(s, n)) return rc;
     const uint64_t no = (uint64_t)n * s->w[s->L];
-    SUR_TRY(s, hipMemcpyAsync(s->dZ[s->L - 1].p, dout, no * 4, hipMemcpyHostToDevice, s->stream));
-    if (int rc = backward(s, n, false, true)) return rc;
+    if (s->fused) {
+        SUR_TRY(s, hipMemcpyAsync(s->yin.p, dout, no * 4, hipMemcpyHostToDevice, s->stream));
+        PassArgs a = pass_args(s, PASS_INPUT, n);
+        a.y = s->yin.p;
+        a.out = out ? s->Z[s->L - 1].p : nullptr;
+        a.dx = s->dxin.p;
+        SUR_TRY(s, launch_pass<PASS_INPUT>(a, s->stream));
+    } else {
+        if (int rc = forward(s, n)) return rc;
+        SUR_TRY(s, hipMemcpyAsync(s->dZ[s->L - 1].p, dout, no * 4, hipMemcpyHostToDevice, s->stream));
+        if (int rc = backward(s, n, false, true)) return rc;
+    }
     if (out) SUR_TRY(s, hipMemcpyAsync(out, s->Z[s->L - 1].p, no * 4, hipMemcpyDeviceToHost, s->stream));
     SUR_TRY(s, hipMemcpyAsync(dx, s->dxin.p, (size_t)n * s->w[0] * 4, hipMemcpyDeviceToHost, s->stream));
     SUR_TRY(s, hipStreamSynchronize(s->stream));
@@ -742,11 +973,21 @@ ARBO_API int arbo_sur_loss_grad(ArboSurrogate* s, uint32_t n, const float* x, co
     if (int rc = upload_x(s, n, x)) return rc;
     const uint64_t no = (uint64_t)n * s->w[s->L];
     SUR_TRY(s, hipMemcpyAsync(s->yin.p, y, no * 4, hipMemcpyHostToDevice, s->stream));
-    if (int rc = forward(s, n)) return rc;
     double l = 0.0;
-    if (int rc = poisson(s, n, s->yin.p, 1.0f / (float)no, &l)) return rc;
+    if (s->fused) {
+        PassArgs a = pass_args(s, PASS_LOSS, n);
+        a.y = s->yin.p;
+        a.scale = 1.0f / (float)no;
+        a.part = s->part.p;
+        SUR_TRY(s, launch_pass<PASS_LOSS>(a, s->stream));
+        SUR_TRY(s, launch_wgrad(s, n, false, 0.0f, 1.0f, 1.0f));
+        if (int rc = sum_parts(s, blocks(n, kFuseRows), &l)) return rc;
+    } else {
+        if (int rc = forward(s, n)) return rc;
+        if (int rc = poisson(s, n, s->yin.p, 1.0f / (float)no, &l)) return rc;
+        if (int rc = backward(s, n, true, false)) return rc;
+    }
     if (loss) *loss = l / (double)no;
-    if (int rc = backward(s, n, true, false)) return rc;
     if (grad) SUR_TRY(s, hipMemcpyAsync(grad, s->G.p, s->n_params * 4, hipMemcpyDeviceToHost, s->stream));
     SUR_TRY(s, hipStreamSynchronize(s->stream));
     return ARBO_OK;
@@ -784,6 +1025,20 @@ ARBO_API int arbo_sur_train(ArboSurrogate* s, uint32_t n, const float* x, const 
         }
         for (uint32_t b0 = 0; b0 < n; b0 += batch) {
             const uint32_t B = std::min(batch, n - b0);
+            if (s->fused) {   // rows and targets are read through the batch's row indices
+                PassArgs a = pass_args(s, PASS_LOSS, B);
+                a.x = s->data_x.p;
+                a.y = s->data_y.p;
+                a.rows = s->idx.p + b0;
+                a.scale = 1.0f / ((float)B * out);
+                a.part = s->part.p;
+                a.acc = epoch_loss ? s->epoch_sum.p : nullptr;
+                SUR_TRY(s, launch_pass<PASS_LOSS>(a, s->stream));
+                float c1, c2;
+                adam_next(s, &c1, &c2);
+                SUR_TRY(s, launch_wgrad(s, B, true, lr, c1, c2));
+                continue;
+            }
             hipLaunchKernelGGL(k_gather, dim3(blocks((uint64_t)B * in, 256)), dim3(256), 0, s->stream, s->data_x.p,
                                s->idx.p + b0, s->H[0].p, B, in);
             SUR_TRY(s, hipGetLastError());
@@ -825,6 +1080,9 @@ ARBO_API void arbo_sur_destroy(ArboSurrogate* s) {
     release(s->data_x);
     release(s->data_y);
     release(s->idx);
+    release(s->pack);
+    for (auto& b : s->HT) release(b);
+    for (auto& b : s->DT) release(b);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
 }
