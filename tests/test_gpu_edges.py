@@ -1,0 +1,42 @@
+"""Day kernels where their waves' shares of work end (GPU), bit for bit
+against the oracle."""
+import numpy as np
+import pytest
+
+from arbo_gpu_fit_amd import abi, configs
+from arbo_gpu_fit_amd.engine import Engine, SimSpec
+from tests.test_gpu_parity import _compare_series, _compare_state
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(hip_lib, oracle_lib, specs, days, flags=0, checks=()):
+    """Runs specs on the GPU and the oracle and compares census, series and
+    kept outputs at the days in `checks` and at the end."""
+    gpu, orc = Engine(hip_lib, flags=flags), Engine(oracle_lib, flags=flags & ~abi.F_GRAPH, threads=8)
+    for e in (gpu, orc):
+        e.init(specs, days)
+    for day in sorted({*checks, days}):
+        for e in (gpu, orc):
+            e.step(day - e.day)
+        for i in range(len(specs)):
+            _compare_state(gpu.state(i), orc.state(i), f"day {day} sim {i}")
+            _compare_series(gpu.series(i), orc.series(i), f"day {day} sim {i}")
+            if flags & abi.F_AOI:
+                assert np.array_equal(gpu.history(i), orc.history(i)), day
+                assert np.array_equal(gpu.aoi(i), orc.aoi(i)), day
+    gpu.close()
+    orc.close()
+
+
+@pytest.mark.parametrize("humans,per_day,serotypes", [(1, 3.0, 1), (40, 90.0, 2), (64, 1.5, 4), (700, 200.0, 3),
+                                                      (5000, 700.5, 1)])
+def test_introductions_use_their_tries_in_order(hip_lib, oracle_lib, humans, per_day, serotypes):
+    """More introductions than the community has susceptible humans (every
+    try is used and most repeat a human), and between one and several per
+    wave's 64 tries."""
+    print(f"[edges] introductions {humans} {per_day} {serotypes}", flush=True)
+    p = configs.reference_params(n_serotypes=serotypes, external_infection=per_day, seed_frac_h=0.01, seed_frac_m=0.01)
+    specs = [SimSpec(1, 1, np.array([humans], np.uint32), p, 5),
+             SimSpec(2, 1, np.array([humans, humans + 3], np.uint32), p, 6)]
+    _both(hip_lib, oracle_lib, specs, 40, flags=abi.F_AOI, checks=(1, 2, 15))
