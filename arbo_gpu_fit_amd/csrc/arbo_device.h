@@ -29,6 +29,7 @@ constexpr uint32_t kAoiRecord = 5000;     // ages per age-of-infection ring
 constexpr uint32_t kPartWords = 24;
 constexpr uint32_t kMaxReduceSplit = 64;  // workgroups per simulation of k_day_reduce: about one
                                           // community per thread, 1..64, about 2,048 in all
+constexpr uint32_t kAoiBlock = 256;       // communities of a workgroup of k_day_aoi
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this
 
 struct CommDesc {
@@ -71,7 +72,8 @@ struct SimDesc {
     float no_distance;            // fraction of events staying at the source (communities with kCommStay)
     uint64_t series_off;          // this simulation's block in the series array
     uint64_t spatial_off;         // its block [(T+1)][S][C] of the per-community series (if kept)
-    uint64_t h_begin, h_end;      // its humans: [h_begin, h_end) of the padded census, h_end a multiple of 4
+    uint32_t aoi_block;           // its first block of kAoiBlock communities (age-of-infection rings)
+    uint32_t aoi_blocks;
     uint32_t climate;             // 1: per-day beta/eip at clim_off and per-birth-day lifetime rows
     uint32_t clim_off;            // [max_days][3] beta_hm, beta_mh, eip in the dens pool
 };
@@ -135,10 +137,15 @@ struct EngineView {
                                    // mosquitoes), summed over days by k_day_reduce
     uint32_t* spatial;             // per-community infectious humans [(T+1)][S][C] per simulation, or null
     int32_t* hist;                 // per human 4 infection-history words (one per serotype), or null
-    uint8_t* aoi_mark;             // per human: 1 when a mosquito event infected it today (age-of-infection
-                                   // rings kept), else null
+    uint8_t* aoi_mark;             // per human: 1 + ring when a mosquito event infected it today
+                                   // (age-of-infection rings kept), else null
+    uint32_t* aoi_cnt;             // [G][4] a community's infections of a day: day + 1, then the four
+                                   // rings' counts as two 16-bit pairs (another day's: none today)
+    uint32_t* aoi_sum;             // [2 parity][blocks][4] their sums over blocks of kAoiBlock communities
+    const uint32_t* aoi_map;       // [blocks] simulation of each block
     uint32_t* aoi;                 // [n_sims][4][kAoiRecord] age-of-infection rings
-    uint32_t* aoi_pos;             // [n_sims][4] next position of each ring
+    uint32_t* aoi_pos;             // [2 parity][n_sims][4] next position of each ring on days of that parity
+    uint32_t aoi_nblocks;
     uint32_t aoi_from;             // first day whose infections enter the rings
     const uint32_t* csr_inbox;     // per CSR entry: inbox row (destination * 9 + in-edge index)
     const uint32_t* csr_thr;       // bits 0..24 threshold, 27..31 alias slot

@@ -1122,6 +1122,7 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
     // ---- onto humans: uniform target, success iff S and never infected by s ----
     const uint32_t N = cd.n;
     bool infected = false;
+    uint32_t aoi01 = 0, aoi23 = 0;   // infections by events per age-of-infection ring
 
     // One claim sequence: mosquito quads [m_lo, m_hi) of their direction's
     // list, then human quads [h_lo, h_hi) of theirs.  Mosquito slots and
@@ -1185,8 +1186,15 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
                     const uint64_t gi = cd.h_off + h;
                     v.h_word[gi] = (w & ~0xFu) | (1u << (4 + s)) | (s << 2) | 1u;
                     if (HIST) {
+                        if (v.aoi_mark && t >= v.aoi_from) {
+                            // the ring: the other serotypes its history holds
+                            const int4 o = reinterpret_cast<const int4*>(v.hist)[gi];
+                            const uint32_t ring = (uint32_t)(s != 0 && o.x != -1) + (uint32_t)(s != 1 && o.y != -1) +
+                                                  (uint32_t)(s != 2 && o.z != -1) + (uint32_t)(s != 3 && o.w != -1);
+                            v.aoi_mark[gi] = (uint8_t)(1u + ring);
+                            add_pair(aoi01, aoi23, ring);
+                        }
                         v.hist[4 * gi + s] = (int32_t)t - v.h_birth[gi];   // age at infection
-                        if (v.aoi_mark && t >= v.aoi_from) v.aoi_mark[gi] = 1;
                     }
                     const U4 r2 = draw(key, cd.h_base + h, t, P_H_IIP, 0);
                     v.h_next[gi] = (uint16_t)(t + sd.iip_min + mulhi(r2.x, sd.iip_span));
@@ -1258,6 +1266,18 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
             for (uint32_t att = kWave; x > 0 && att < kIntroTries; att += 4 * kWave)
                 introduce(att, std::integral_constant<uint32_t, 4>{});
             __syncthreads();
+        }
+    }
+    if (HIST && v.aoi_mark) {   // the community's records of the day, for k_day_aoi
+        aoi01 = wave_sum(aoi01);
+        aoi23 = wave_sum(aoi23);
+        if (aoi01 | aoi23) {
+            if (lane == 0) reinterpret_cast<uint4*>(v.aoi_cnt)[g] = make_uint4(t + 1u, aoi01, aoi23, 0u);
+            if (lane < 4) {
+                const uint32_t n = unpack_pair(aoi01, aoi23, lane);
+                const size_t b = (size_t)(t & 1u) * v.aoi_nblocks + sd.aoi_block + cd.c / kAoiBlock;
+                if (n) atomicAdd(&v.aoi_sum[4 * b + lane], n);
+            }
         }
     }
     // a human exposed today turns infectious on day t + iip + 1 at the earliest
@@ -1393,114 +1413,143 @@ __global__ __launch_bounds__(256) void k_day_reduce(EngineView v, uint32_t split
     if (tid >= 64 && tid < 66 && s_scan[tid - 64]) atomicAdd(&v.scanned[2 * (size_t)sim + (tid - 64)], s_scan[tid - 64]);
 }
 
-// Age-of-infection rings (nepidemic.cu:229-243), one workgroup per
-// simulation after the event kernel.  The reference appends each novel
+// Age-of-infection rings (nepidemic.cu:229-243), one workgroup per kAoiBlock
+// communities after the event kernel.  The reference appends each novel
 // infection by a mosquito event to ring k (k = serotypes the human had been
 // infected with before) at atomicInc positions, in whatever order threads
 // arrive.  Here a day's infections enter in human order, which makes the
-// rings deterministic: a counting pass gives the day's total per ring, and
-// the writing pass stores only the day's last kAoiRecord records of each
-// ring, so no slot is written twice in one launch.
+// rings deterministic, and only the day's last kAoiRecord records of each
+// ring are stored, so no slot is written twice in one launch.
+// A record's place is the ring's position, plus the records of the
+// simulation's earlier blocks (the event kernel's sums), of the block's
+// earlier communities (a scan of the event kernel's counts) and of the
+// community's earlier humans (a wave walks the marks of a community that has
+// any).  One workgroup per simulation that walked every human's mark twice
+// took 155 us a day on 86,700 humans, this 5.
 __global__ __launch_bounds__(256) void k_day_aoi(EngineView v) {
     const uint32_t t = *v.day + v.day_offset;
     if (t < v.aoi_from) return;
-    const uint32_t sim = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-    constexpr uint32_t kWaves = 256 / kWave, kChunk = 4 * 256;
+    const uint32_t sim = v.aoi_map[blockIdx.x], tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    constexpr uint32_t kWaves = 256 / kWave;
+    static_assert(kAoiBlock == 256, "a community per thread");
     const SimDesc& sd = v.sims[sim];
-    __shared__ uint32_t s_part[kWaves][4];
-    __shared__ uint32_t s_tot[4], s_pos[4];
-    // previous infections of the human infected today: its history words
-    // other than today's (one infection per human and day)
-    auto ring_of = [&](uint64_t gi) -> uint32_t {
-        const int4 h = reinterpret_cast<const int4*>(v.hist)[gi];
-        const uint32_t n = (uint32_t)(h.x != -1) + (uint32_t)(h.y != -1) + (uint32_t)(h.z != -1) + (uint32_t)(h.w != -1);
-        return n ? n - 1u : 0u;   // n >= 1: today's word is set
-    };
-    // counting pass
-    uint32_t c[4] = {0, 0, 0, 0};
-    for (uint64_t base = sd.h_begin; base < sd.h_end; base += kChunk) {
-        const uint64_t gi = base + 4 * tid;
-        if (gi >= sd.h_end) continue;
-        const uint32_t m = *reinterpret_cast<const uint32_t*>(v.aoi_mark + gi);
-        if (!m) continue;
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-            if (!((m >> (8 * e)) & 0xFFu)) continue;
-            const uint32_t r = ring_of(gi + e);
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) c[k] += r == k;   // constant indices: the counters stay in registers
-        }
+    const uint32_t blk = blockIdx.x - sd.aoi_block;
+    const uint4* sums = reinterpret_cast<const uint4*>(v.aoi_sum) + (size_t)(t & 1u) * v.aoi_nblocks + sd.aoi_block;
+    __shared__ uint32_t s_part[kWaves][8];
+    __shared__ uint32_t s_at[kAoiBlock][4];     // first record of each community and ring
+    __shared__ uint32_t s_list[kWaves][kWave];  // the communities with records, a quarter of the block each
+    __shared__ uint32_t s_n[kWaves];
+    // the day's records of the simulation and of its earlier blocks
+    uint32_t tot[4] = {0, 0, 0, 0}, pre[4] = {0, 0, 0, 0};
+    for (uint32_t b = tid; b < sd.aoi_blocks; b += 256) {
+        const uint4 n = sums[b];
+        const uint32_t e = b < blk ? 0xFFFFFFFFu : 0u;
+        tot[0] += n.x; tot[1] += n.y; tot[2] += n.z; tot[3] += n.w;
+        pre[0] += n.x & e; pre[1] += n.y & e; pre[2] += n.z & e; pre[3] += n.w & e;
     }
+    // this thread's community
+    const uint32_t c = blk * kAoiBlock + tid;
+    uint4 mine = make_uint4(0, 0, 0, 0);
+    if (c < sd.C) mine = reinterpret_cast<const uint4*>(v.aoi_cnt)[sd.comm_off + c];
+    const bool any = mine.x == t + 1u;   // counted today
+    const uint32_t cnt[4] = {any ? mine.y & 0xFFFFu : 0u, any ? mine.y >> 16 : 0u, any ? mine.z & 0xFFFFu : 0u,
+                             any ? mine.z >> 16 : 0u};
+    uint32_t at[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t w = wave_sum(c[k]);
-        if (lane == 0) s_part[wv][k] = w;
+        uint32_t n;
+        at[k] = wave_exclusive_scan(cnt[k], n);
+        const uint32_t a = wave_sum(tot[k]), p = wave_sum(pre[k]);
+        if (lane == 0) {
+            s_part[wv][k] = a;
+            s_part[wv][4 + k] = n;
+        }
+        tot[k] = a;
+        pre[k] = p;
+    }
+    __shared__ uint32_t s_pre[kWaves][4];
+    if (lane < 4) s_pre[wv][lane] = lane == 0 ? pre[0] : lane == 1 ? pre[1] : lane == 2 ? pre[2] : pre[3];
+    const uint64_t have = __builtin_amdgcn_ballot_w64(any);
+    if (any) s_list[wv][__builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0u))] = tid;
+    if (lane == 0) s_n[wv] = (uint32_t)__popcll(have);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        tot[k] = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kWaves; ++w) {
+            tot[k] += s_part[w][k];
+            at[k] += s_pre[w][k] + (w < wv ? s_part[w][4 + k] : 0u);
+        }
+        s_at[tid][k] = at[k];
+    }
+    uint32_t* pos = v.aoi_pos + 4 * (size_t)sim;
+    uint32_t base[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) base[k] = pos[(size_t)(t & 1u) * 4 * v.n_sims + k];
+    if (tid < 4) {   // tomorrow's position and sums
+        const uint32_t n = tid == 0 ? tot[0] : tid == 1 ? tot[1] : tid == 2 ? tot[2] : tot[3];
+        const uint32_t p = tid == 0 ? base[0] : tid == 1 ? base[1] : tid == 2 ? base[2] : base[3];
+        if (blk == 0) pos[(size_t)((t + 1) & 1u) * 4 * v.n_sims + tid] = (p + n) % kAoiRecord;
+        v.aoi_sum[4 * ((size_t)((t + 1) & 1u) * v.aoi_nblocks + blockIdx.x) + tid] = 0u;
     }
     __syncthreads();
-    if (tid < 4) {
-        uint32_t n = 0;
-        for (uint32_t w = 0; w < kWaves; ++w) n += s_part[w][tid];
-        s_tot[tid] = n;
-        s_pos[tid] = v.aoi_pos[4 * sim + tid];
-    }
-    __syncthreads();
-    if ((s_tot[0] | s_tot[1] | s_tot[2] | s_tot[3]) == 0) return;
-    // writing pass: record j of the day (per ring) goes to slot (pos + j) mod kAoiRecord
     uint32_t* ring = v.aoi + (uint64_t)sim * 4 * kAoiRecord;
-    uint32_t done[4] = {0, 0, 0, 0};   // records of the ring in earlier chunks (same in every thread)
-    for (uint64_t base = sd.h_begin; base < sd.h_end; base += kChunk) {
-        const uint64_t gi = base + 4 * tid;
-        uint32_t m = 0;
-        if (gi < sd.h_end) m = *reinterpret_cast<const uint32_t*>(v.aoi_mark + gi);
-        uint32_t k4[4] = {4, 4, 4, 4};
-        uint32_t mine[4] = {0, 0, 0, 0};
+    // the block's listed communities, dealt to the waves in turn
+    uint32_t before = 0;
+    for (uint32_t q = 0; q < kWaves; ++q) {
+        const uint32_t n = s_n[q];
+        for (uint32_t i = (wv + kWaves - before % kWaves) % kWaves; i < n; i += kWaves) {
+            const uint32_t l = s_list[q][i];
+            const CommDesc& cd = v.comm[sd.comm_off + blk * kAoiBlock + l];
+            const uint64_t h_off = cd.h_off;
+            const uint32_t nh = cd.n;
+            uint32_t next[4];
 #pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-            if (!((m >> (8 * e)) & 0xFFu)) continue;
-            k4[e] = ring_of(gi + e);
+            for (uint32_t k = 0; k < 4; ++k) next[k] = s_at[l][k];
+            constexpr uint32_t kStep = 4 * kWave, kAhead = 4;
+            for (uint32_t h0 = 0; h0 < nh; h0 += kAhead * kStep) {
+                uint32_t m[kAhead];   // communities start on multiples of four humans
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) mine[k] += k4[e] == k;
-        }
-        uint32_t before[4];
+                for (uint32_t u = 0; u < kAhead; ++u) {
+                    const uint32_t h = h0 + u * kStep + 4 * lane;
+                    m[u] = h < nh ? *reinterpret_cast<const uint32_t*>(v.aoi_mark + h_off + h) : 0u;
+                }
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {   // exclusive prefix over the workgroup
-            uint32_t x = mine[k];
+                for (uint32_t u = 0; u < kAhead; ++u) {
+                    if (!__builtin_amdgcn_ballot_w64(m[u] != 0u)) continue;
+                    const uint64_t gi = h_off + h0 + u * kStep + 4 * lane;
+                    uint32_t r[4], my[4] = {0, 0, 0, 0}, off[4];
 #pragma unroll
-            for (uint32_t d = 1; d < kWave; d <<= 1) {
-                const uint32_t y = __shfl_up(x, d, kWave);
-                if (lane >= d) x += y;
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        r[e] = (m[u] >> (8 * e)) & 0xFFu;
+#pragma unroll
+                        for (uint32_t k = 0; k < 4; ++k) my[k] += r[e] == k + 1u;
+                    }
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        uint32_t n4;
+                        off[k] = next[k] + wave_exclusive_scan(my[k], n4);
+                        next[k] += n4;
+                    }
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) {
+#pragma unroll
+                        for (uint32_t k = 0; k < 4; ++k) {
+                            if (r[e] != k + 1u) continue;
+                            const uint32_t j = off[k]++;
+                            if (j + kAoiRecord >= tot[k])   // among the day's last kAoiRecord records of ring k
+                                ring[k * kAoiRecord + (base[k] + j) % kAoiRecord] =
+                                    (uint32_t)((int32_t)t - v.h_birth[gi + e]);
+                        }
+                    }
+                    if (m[u]) *reinterpret_cast<uint32_t*>(v.aoi_mark + gi) = 0u;
+                }
             }
-            if (lane == kWave - 1) s_part[wv][k] = x;
-            before[k] = x - mine[k];
         }
-        __syncthreads();
-        uint32_t chunk_tot[4];
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            uint32_t off = 0, all = 0;
-            for (uint32_t w = 0; w < kWaves; ++w) {
-                off += w < wv ? s_part[w][k] : 0u;
-                all += s_part[w][k];
-            }
-            before[k] += off + done[k];
-            chunk_tot[k] = all;
-        }
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                if (k4[e] != k) continue;
-                const uint32_t j = before[k]++;
-                if (j + kAoiRecord >= s_tot[k])   // among the day's last kAoiRecord records of ring k
-                    ring[k * kAoiRecord + (s_pos[k] + j) % kAoiRecord] = (uint32_t)((int32_t)t - v.h_birth[gi + e]);
-            }
-        }
-        if (m) *reinterpret_cast<uint32_t*>(v.aoi_mark + gi) = 0u;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) done[k] += chunk_tot[k];
-        __syncthreads();   // s_part is rewritten by the next chunk
+        before += n;
     }
-    if (tid < 4) v.aoi_pos[4 * sim + tid] = (s_pos[tid] + s_tot[tid]) % kAoiRecord;
 }
 
 __global__ void k_advance_day(uint32_t* day, uint32_t n) {
@@ -1600,7 +1649,7 @@ hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st) 
         if (v.hist) hipLaunchKernelGGL((k_day_events<false, true, 1>), grid, block, 0, st, v);
         else hipLaunchKernelGGL((k_day_events<false, false, 1>), grid, block, 0, st, v);
     }
-    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, dim3(v.n_sims), dim3(256), 0, st, v);
+    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, dim3(v.aoi_nblocks), dim3(256), 0, st, v);
     return hipGetLastError();
 }
 

@@ -40,3 +40,32 @@ def test_introductions_use_their_tries_in_order(hip_lib, oracle_lib, humans, per
     specs = [SimSpec(1, 1, np.array([humans], np.uint32), p, 5),
              SimSpec(2, 1, np.array([humans, humans + 3], np.uint32), p, 6)]
     _both(hip_lib, oracle_lib, specs, 40, flags=abi.F_AOI, checks=(1, 2, 15))
+
+
+@pytest.mark.parametrize("grid,humans", [((1, 1), 3), ((16, 16), 40), ((257, 1), 30), ((23, 23), 30), ((2, 2), 9000)])
+def test_age_of_infection_records_across_blocks(hip_lib, oracle_lib, grid, humans):
+    """Communities below, at and above the rings' 256-community blocks, and
+    communities of several waves' marks; rings that wrap; a resumed day of
+    either parity."""
+    print(f"[edges] rings {grid} {humans}", flush=True)
+    p = configs.base_params(beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.05, seed_frac_m=0.05, external_infection=3.0)
+    small = configs.base_params(n_serotypes=2, beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.05)
+    specs = [SimSpec(3, 2, np.full(6, 50, np.uint32), small, 8),
+             SimSpec(*grid, np.full(grid[0] * grid[1], humans, np.uint32), p, 9)]
+    _both(hip_lib, oracle_lib, specs, 40, flags=abi.F_AOI, checks=(1, 5, 12, 25))
+    gpu, orc = Engine(hip_lib, flags=abi.F_AOI), Engine(oracle_lib, flags=abi.F_AOI, threads=8)
+    for e in (gpu, orc):
+        e.init(specs, 40)
+        e.step(11)
+        st = [e.state(i) for i in range(2)]
+        e.step(3)
+        e.set_day(11)
+        for i in range(2):
+            e.write_state(i, st[i])
+        e.step(6)
+        e.set_day(20)
+        e.step(5)
+    for i in range(2):
+        assert np.array_equal(gpu.aoi(i), orc.aoi(i)) and np.array_equal(gpu.history(i), orc.history(i))
+    gpu.close()
+    orc.close()
