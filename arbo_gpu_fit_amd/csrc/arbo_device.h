@@ -29,7 +29,7 @@ constexpr uint32_t kAoiRecord = 5000;     // ages per age-of-infection ring
 constexpr uint32_t kPartWords = 24;
 constexpr uint32_t kMaxReduceSplit = 64;  // workgroups per simulation of k_day_reduce: about one
                                           // community per thread, 1..64, about 2,048 in all
-constexpr uint32_t kAoiBlock = 256;       // communities of a workgroup of k_day_aoi
+constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this
 
 struct CommDesc {
@@ -142,7 +142,6 @@ struct EngineView {
     uint32_t* aoi_cnt;             // [G][4] a community's infections of a day: day + 1, then the four
                                    // rings' counts as two 16-bit pairs (another day's: none today)
     uint32_t* aoi_sum;             // [2 parity][blocks][4] their sums over blocks of kAoiBlock communities
-    const uint32_t* aoi_map;       // [blocks] simulation of each block
     uint32_t* aoi;                 // [n_sims][4][kAoiRecord] age-of-infection rings
     uint32_t* aoi_pos;             // [2 parity][n_sims][4] next position of each ring on days of that parity
     uint32_t aoi_nblocks;

@@ -62,7 +62,7 @@ struct ArboEngine {
     DevBuf<uint16_t> h_next, m_word, m_next;
     DevBuf<int32_t> h_birth, hist;
     DevBuf<uint8_t> aoi_mark;
-    DevBuf<uint32_t> aoi, aoi_pos, aoi_cnt, aoi_sum, aoi_map;
+    DevBuf<uint32_t> aoi, aoi_pos, aoi_cnt, aoi_sum;
     DevBuf<unsigned long long> lam, scanned;
     DevBuf<uint32_t> part;   // per-community partials of the day
     DevBuf<float> dens;
@@ -128,7 +128,7 @@ void free_batch(ArboEngine* e) {
     dev_free(e->comm); dev_free(e->simd);
     dev_free(e->h_word); dev_free(e->alive); dev_free(e->cnt); dev_free(e->nld); dev_free(e->active); dev_free(e->hsum); dev_free(e->series); dev_free(e->spatial); dev_free(e->csr_thr); dev_free(e->csr_inbox);
     dev_free(e->in_edge); dev_free(e->in_slot); dev_free(e->tables); dev_free(e->day_ctr);
-    dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum); dev_free(e->aoi_map);
+    dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum);
     dev_free(e->lam); dev_free(e->scanned); dev_free(e->dens); dev_free(e->part);
     e->ready = false;
 }
@@ -299,11 +299,12 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     e->sims.assign(n_sims, SimHost());
     e->sim_desc.assign(n_sims, SimDesc());
     std::vector<CommDesc> comm;
-    std::vector<uint32_t> csr_thr, csr_inbox, in_edge, in_slot, table_pool, aoi_map;
+    std::vector<uint32_t> csr_thr, csr_inbox, in_edge, in_slot, table_pool;
     std::vector<float> dens_pool;
     std::map<std::vector<uint32_t>, uint32_t> seen_u32;
     std::map<std::vector<float>, uint32_t> seen_f32;
     uint64_t h_tot = 0, m_tot = 0, ser_tot = 0, spa_tot = 0;
+    uint32_t aoi_blocks = 0;
     uint32_t max_n = 0, max_cap = 0, death_m_lds = 1;
     for (uint32_t i = 0; i < n_sims; ++i) {
         const SimTables& t = tabs[i];
@@ -406,9 +407,9 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
             max_n = std::max(max_n, cd.n);
             max_cap = std::max(max_cap, cd.cap);
         }
-        sd.aoi_block = (uint32_t)aoi_map.size();
+        sd.aoi_block = aoi_blocks;
         sd.aoi_blocks = (t.C + kAoiBlock - 1) / kAoiBlock;
-        if (e->flags & ARBO_F_AOI) aoi_map.insert(aoi_map.end(), sd.aoi_blocks, i);
+        aoi_blocks += sd.aoi_blocks;
     }
     h_tot = align_up(h_tot, kHumanAlign) + kHumanAlign;
     m_tot = align_up(m_tot, kMosqAlign) + ARBO_MAX_COMMUNITY_SLOTS;  // room for whole-workgroup vector reads
@@ -425,7 +426,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         (rc = dev_alloc(e, e->aoi, (e->flags & ARBO_F_AOI) ? (size_t)n_sims * 4 * kAoiRecord : 0)) ||
         (rc = dev_alloc(e, e->aoi_pos, (e->flags & ARBO_F_AOI) ? (size_t)n_sims * 8 : 0)) ||
         (rc = dev_alloc(e, e->aoi_cnt, (e->flags & ARBO_F_AOI) ? comm.size() * 4 : 0)) ||
-        (rc = dev_alloc(e, e->aoi_sum, aoi_map.size() * 8)) || (rc = dev_alloc(e, e->aoi_map, aoi_map.size())) || (rc = dev_alloc(e, e->m_word, m_tot)) ||
+        (rc = dev_alloc(e, e->aoi_sum, (e->flags & ARBO_F_AOI) ? (size_t)aoi_blocks * 8 : 0)) || (rc = dev_alloc(e, e->m_word, m_tot)) ||
         (rc = dev_alloc(e, e->m_next, m_tot)) || (rc = dev_alloc(e, e->alive, m_tot / 32)) || (rc = dev_alloc(e, e->cnt, comm.size() * kInboxEdges * 8)) || (rc = dev_alloc(e, e->nld, comm.size() * 8)) ||
         (rc = dev_alloc(e, e->hsum, comm.size() * 4)) || (rc = dev_alloc(e, e->active, comm.size())) ||
         (rc = dev_alloc(e, e->lam, (size_t)2 * n_sims * 8)) || (rc = dev_alloc(e, e->scanned, (size_t)2 * n_sims)) || (rc = dev_alloc(e, e->part, comm.size() * kPartWords)) || (rc = dev_alloc(e, e->series, ser_tot)) || (rc = dev_alloc(e, e->spatial, spa_tot)) ||
@@ -461,8 +462,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         HIP_TRY(e, launch_fill(e->aoi.p, (uint64_t)n_sims * 4 * kAoiRecord, 0u, e->stream));
         HIP_TRY(e, launch_fill(e->aoi_pos.p, (uint64_t)n_sims * 8, 0u, e->stream));
         HIP_TRY(e, launch_fill(e->aoi_cnt.p, (uint64_t)comm.size() * 4, 0u, e->stream));
-        HIP_TRY(e, launch_fill(e->aoi_sum.p, (uint64_t)aoi_map.size() * 8, 0u, e->stream));
-        HIP_TRY(e, hipMemcpy(e->aoi_map.p, aoi_map.data(), aoi_map.size() * 4, hipMemcpyHostToDevice));
+        HIP_TRY(e, launch_fill(e->aoi_sum.p, (uint64_t)aoi_blocks * 8, 0u, e->stream));
     }
     HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->m_word.p), m_tot / 2, 0x00030003u, e->stream));
 
@@ -490,8 +490,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     v.aoi_pos = e->aoi_pos.p;
     v.aoi_cnt = e->aoi_cnt.p;
     v.aoi_sum = e->aoi_sum.p;
-    v.aoi_map = e->aoi_map.p;
-    v.aoi_nblocks = (uint32_t)aoi_map.size();
+    v.aoi_nblocks = aoi_blocks;
     v.aoi_from = max_days > kAoiWindow ? max_days - kAoiWindow : 0u;
     v.csr_inbox = e->csr_inbox.p;
     v.csr_thr = e->csr_thr.p;

@@ -1413,142 +1413,102 @@ __global__ __launch_bounds__(256) void k_day_reduce(EngineView v, uint32_t split
     if (tid >= 64 && tid < 66 && s_scan[tid - 64]) atomicAdd(&v.scanned[2 * (size_t)sim + (tid - 64)], s_scan[tid - 64]);
 }
 
-// Age-of-infection rings (nepidemic.cu:229-243), one workgroup per kAoiBlock
-// communities after the event kernel.  The reference appends each novel
-// infection by a mosquito event to ring k (k = serotypes the human had been
-// infected with before) at atomicInc positions, in whatever order threads
-// arrive.  Here a day's infections enter in human order, which makes the
-// rings deterministic, and only the day's last kAoiRecord records of each
-// ring are stored, so no slot is written twice in one launch.
+// Age-of-infection rings (nepidemic.cu:229-243), a wave per community after
+// the event kernel.  The reference appends each novel infection by a mosquito
+// event to ring k (k = serotypes the human had been infected with before) at
+// atomicInc positions, in whatever order threads arrive.  Here a day's
+// infections enter in human order, which makes the rings deterministic, and
+// only the day's last kAoiRecord records of each ring are stored, so no slot
+// is written twice in one launch.
 // A record's place is the ring's position, plus the records of the
-// simulation's earlier blocks (the event kernel's sums), of the block's
-// earlier communities (a scan of the event kernel's counts) and of the
-// community's earlier humans (a wave walks the marks of a community that has
-// any).  One workgroup per simulation that walked every human's mark twice
-// took 155 us a day on 86,700 humans, this 5.
-__global__ __launch_bounds__(256) void k_day_aoi(EngineView v) {
-    const uint32_t t = *v.day + v.day_offset;
+// simulation's earlier blocks of communities (the event kernel's sums), of the
+// block's earlier communities (its counts) and of the community's earlier
+// humans (the marks, 1,024 requested at a time).  A community without records
+// leaves at once.  What bounds it is the chain of those three loads: 8 us a
+// day on 289 communities of 300, where one workgroup per simulation that
+// walked every human's mark twice took 155, and a workgroup per block of
+// communities 40.
+__global__ __launch_bounds__(kWave) void k_day_aoi(EngineView v) {
+    const uint32_t t = *v.day + v.day_offset, g = blockIdx.x, lane = threadIdx.x;
     if (t < v.aoi_from) return;
-    const uint32_t sim = v.aoi_map[blockIdx.x], tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-    constexpr uint32_t kWaves = 256 / kWave;
-    static_assert(kAoiBlock == 256, "a community per thread");
-    const SimDesc& sd = v.sims[sim];
-    const uint32_t blk = blockIdx.x - sd.aoi_block;
+    const uint4* cnt = reinterpret_cast<const uint4*>(v.aoi_cnt);
+    const CommDesc cd = v.comm[g];
+    const bool any = cnt[g].x == t + 1u;
+    if (!any && cd.c % kAoiBlock != 0) return;
+    const SimDesc& sd = v.sims[cd.sim];
+    const uint32_t blk = cd.c / kAoiBlock;
+    if (cd.c % kAoiBlock == 0 && lane < 4)   // tomorrow's sums
+        v.aoi_sum[4 * ((size_t)((t + 1) & 1u) * v.aoi_nblocks + sd.aoi_block + blk) + lane] = 0u;
+    if (!any && cd.c != 0) return;
+    // the day's records per ring: of the simulation, and before this community
     const uint4* sums = reinterpret_cast<const uint4*>(v.aoi_sum) + (size_t)(t & 1u) * v.aoi_nblocks + sd.aoi_block;
-    __shared__ uint32_t s_part[kWaves][8];
-    __shared__ uint32_t s_at[kAoiBlock][4];     // first record of each community and ring
-    __shared__ uint32_t s_list[kWaves][kWave];  // the communities with records, a quarter of the block each
-    __shared__ uint32_t s_n[kWaves];
-    // the day's records of the simulation and of its earlier blocks
-    uint32_t tot[4] = {0, 0, 0, 0}, pre[4] = {0, 0, 0, 0};
-    for (uint32_t b = tid; b < sd.aoi_blocks; b += 256) {
+    uint32_t tot[4] = {0, 0, 0, 0}, next[4] = {0, 0, 0, 0};
+    for (uint32_t b = lane; b < sd.aoi_blocks; b += kWave) {
         const uint4 n = sums[b];
         const uint32_t e = b < blk ? 0xFFFFFFFFu : 0u;
         tot[0] += n.x; tot[1] += n.y; tot[2] += n.z; tot[3] += n.w;
-        pre[0] += n.x & e; pre[1] += n.y & e; pre[2] += n.z & e; pre[3] += n.w & e;
+        next[0] += n.x & e; next[1] += n.y & e; next[2] += n.z & e; next[3] += n.w & e;
     }
-    // this thread's community
-    const uint32_t c = blk * kAoiBlock + tid;
-    uint4 mine = make_uint4(0, 0, 0, 0);
-    if (c < sd.C) mine = reinterpret_cast<const uint4*>(v.aoi_cnt)[sd.comm_off + c];
-    const bool any = mine.x == t + 1u;   // counted today
-    const uint32_t cnt[4] = {any ? mine.y & 0xFFFFu : 0u, any ? mine.y >> 16 : 0u, any ? mine.z & 0xFFFFu : 0u,
-                             any ? mine.z >> 16 : 0u};
-    uint32_t at[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        uint32_t n;
-        at[k] = wave_exclusive_scan(cnt[k], n);
-        const uint32_t a = wave_sum(tot[k]), p = wave_sum(pre[k]);
-        if (lane == 0) {
-            s_part[wv][k] = a;
-            s_part[wv][4 + k] = n;
-        }
-        tot[k] = a;
-        pre[k] = p;
+    for (uint32_t u = 0; u < kAoiBlock / kWave; ++u) {
+        const uint32_t o = blk * kAoiBlock + u * kWave + lane;
+        if (o >= cd.c) continue;
+        const uint4 n = cnt[sd.comm_off + o];
+        if (n.x != t + 1u) continue;
+        next[0] += n.y & 0xFFFFu; next[1] += n.y >> 16; next[2] += n.z & 0xFFFFu; next[3] += n.z >> 16;
     }
-    __shared__ uint32_t s_pre[kWaves][4];
-    if (lane < 4) s_pre[wv][lane] = lane == 0 ? pre[0] : lane == 1 ? pre[1] : lane == 2 ? pre[2] : pre[3];
-    const uint64_t have = __builtin_amdgcn_ballot_w64(any);
-    if (any) s_list[wv][__builtin_amdgcn_mbcnt_hi((uint32_t)(have >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)have, 0u))] = tid;
-    if (lane == 0) s_n[wv] = (uint32_t)__popcll(have);
-    __syncthreads();
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        tot[k] = 0;
-#pragma unroll
-        for (uint32_t w = 0; w < kWaves; ++w) {
-            tot[k] += s_part[w][k];
-            at[k] += s_pre[w][k] + (w < wv ? s_part[w][4 + k] : 0u);
-        }
-        s_at[tid][k] = at[k];
-    }
-    uint32_t* pos = v.aoi_pos + 4 * (size_t)sim;
+    const uint32_t* pos = v.aoi_pos + 4 * ((size_t)(t & 1u) * v.n_sims + cd.sim);
     uint32_t base[4];
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) base[k] = pos[(size_t)(t & 1u) * 4 * v.n_sims + k];
-    if (tid < 4) {   // tomorrow's position and sums
-        const uint32_t n = tid == 0 ? tot[0] : tid == 1 ? tot[1] : tid == 2 ? tot[2] : tot[3];
-        const uint32_t p = tid == 0 ? base[0] : tid == 1 ? base[1] : tid == 2 ? base[2] : base[3];
-        if (blk == 0) pos[(size_t)((t + 1) & 1u) * 4 * v.n_sims + tid] = (p + n) % kAoiRecord;
-        v.aoi_sum[4 * ((size_t)((t + 1) & 1u) * v.aoi_nblocks + blockIdx.x) + tid] = 0u;
+    for (uint32_t k = 0; k < 4; ++k) {
+        tot[k] = wave_sum(tot[k]);
+        next[k] = wave_sum(next[k]);
+        base[k] = pos[k];
     }
-    __syncthreads();
-    uint32_t* ring = v.aoi + (uint64_t)sim * 4 * kAoiRecord;
-    // the block's listed communities, dealt to the waves in turn
-    uint32_t before = 0;
-    for (uint32_t q = 0; q < kWaves; ++q) {
-        const uint32_t n = s_n[q];
-        for (uint32_t i = (wv + kWaves - before % kWaves) % kWaves; i < n; i += kWaves) {
-            const uint32_t l = s_list[q][i];
-            const CommDesc& cd = v.comm[sd.comm_off + blk * kAoiBlock + l];
-            const uint64_t h_off = cd.h_off;
-            const uint32_t nh = cd.n;
-            uint32_t next[4];
+    if (cd.c == 0 && lane < 4) {   // tomorrow's position
+        const uint32_t n = lane == 0 ? tot[0] : lane == 1 ? tot[1] : lane == 2 ? tot[2] : tot[3];
+        const uint32_t p = lane == 0 ? base[0] : lane == 1 ? base[1] : lane == 2 ? base[2] : base[3];
+        v.aoi_pos[4 * ((size_t)((t + 1) & 1u) * v.n_sims + cd.sim) + lane] = (p + n) % kAoiRecord;
+    }
+    if (!any) return;
+    uint32_t* ring = v.aoi + (uint64_t)cd.sim * 4 * kAoiRecord;
+    constexpr uint32_t kStep = 4 * kWave, kAhead = 4;
+    for (uint32_t h0 = 0; h0 < cd.n; h0 += kAhead * kStep) {
+        uint32_t m[kAhead];   // communities start on multiples of four humans
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) next[k] = s_at[l][k];
-            constexpr uint32_t kStep = 4 * kWave, kAhead = 4;
-            for (uint32_t h0 = 0; h0 < nh; h0 += kAhead * kStep) {
-                uint32_t m[kAhead];   // communities start on multiples of four humans
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            const uint32_t h = h0 + u * kStep + 4 * lane;
+            m[u] = h < cd.n ? *reinterpret_cast<const uint32_t*>(v.aoi_mark + cd.h_off + h) : 0u;
+        }
 #pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    const uint32_t h = h0 + u * kStep + 4 * lane;
-                    m[u] = h < nh ? *reinterpret_cast<const uint32_t*>(v.aoi_mark + h_off + h) : 0u;
-                }
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            if (!__builtin_amdgcn_ballot_w64(m[u] != 0u)) continue;
+            const uint64_t gi = cd.h_off + h0 + u * kStep + 4 * lane;
+            uint32_t r[4], my[4] = {0, 0, 0, 0}, at[4];
 #pragma unroll
-                for (uint32_t u = 0; u < kAhead; ++u) {
-                    if (!__builtin_amdgcn_ballot_w64(m[u] != 0u)) continue;
-                    const uint64_t gi = h_off + h0 + u * kStep + 4 * lane;
-                    uint32_t r[4], my[4] = {0, 0, 0, 0}, off[4];
+            for (uint32_t e = 0; e < 4; ++e) {
+                r[e] = (m[u] >> (8 * e)) & 0xFFu;
 #pragma unroll
-                    for (uint32_t e = 0; e < 4; ++e) {
-                        r[e] = (m[u] >> (8 * e)) & 0xFFu;
+                for (uint32_t k = 0; k < 4; ++k) my[k] += r[e] == k + 1u;
+            }
 #pragma unroll
-                        for (uint32_t k = 0; k < 4; ++k) my[k] += r[e] == k + 1u;
-                    }
+            for (uint32_t k = 0; k < 4; ++k) {
+                uint32_t n;
+                at[k] = next[k] + wave_exclusive_scan(my[k], n);
+                next[k] += n;
+            }
 #pragma unroll
-                    for (uint32_t k = 0; k < 4; ++k) {
-                        uint32_t n4;
-                        off[k] = next[k] + wave_exclusive_scan(my[k], n4);
-                        next[k] += n4;
-                    }
+            for (uint32_t e = 0; e < 4; ++e) {
 #pragma unroll
-                    for (uint32_t e = 0; e < 4; ++e) {
-#pragma unroll
-                        for (uint32_t k = 0; k < 4; ++k) {
-                            if (r[e] != k + 1u) continue;
-                            const uint32_t j = off[k]++;
-                            if (j + kAoiRecord >= tot[k])   // among the day's last kAoiRecord records of ring k
-                                ring[k * kAoiRecord + (base[k] + j) % kAoiRecord] =
-                                    (uint32_t)((int32_t)t - v.h_birth[gi + e]);
-                        }
-                    }
-                    if (m[u]) *reinterpret_cast<uint32_t*>(v.aoi_mark + gi) = 0u;
+                for (uint32_t k = 0; k < 4; ++k) {
+                    if (r[e] != k + 1u) continue;
+                    const uint32_t j = at[k]++;
+                    if (j + kAoiRecord >= tot[k])   // among the day's last kAoiRecord records of ring k
+                        ring[k * kAoiRecord + (base[k] + j) % kAoiRecord] = (uint32_t)((int32_t)t - v.h_birth[gi + e]);
                 }
             }
+            if (m[u]) *reinterpret_cast<uint32_t*>(v.aoi_mark + gi) = 0u;
         }
-        before += n;
     }
 }
 
@@ -1649,7 +1609,7 @@ hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st) 
         if (v.hist) hipLaunchKernelGGL((k_day_events<false, true, 1>), grid, block, 0, st, v);
         else hipLaunchKernelGGL((k_day_events<false, false, 1>), grid, block, 0, st, v);
     }
-    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, dim3(v.aoi_nblocks), dim3(256), 0, st, v);
+    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, grid, block, 0, st, v);
     return hipGetLastError();
 }
 
