@@ -12,6 +12,8 @@
 #pragma once
 #include <stdint.h>
 
+#include "arbo_rng.h"
+
 namespace arbo {
 
 constexpr uint32_t kWave = 64;            // threads per workgroup: one wavefront per community
@@ -60,6 +62,7 @@ struct SimDesc {
     float beta_hm, beta_mh, omega, recovery, eip, intro;
     uint32_t iip_min, iip_span;   // incubation uniform on [iip_min, iip_min + iip_span)
     uint32_t death_h_off;         // offsets into the shared table pools
+    uint32_t death_h_guide_off;   // [kHumanGuide + 1] smallest death age of each slice of draws
     uint32_t death_m_off;
     uint32_t init_h_off;
     uint32_t init_m_off;
@@ -188,7 +191,23 @@ __host__ __device__ inline uint32_t xcd_block(uint32_t b, uint32_t n) {
     return x * q + (x < r ? x : r) + i;
 }
 
-hipError_t launch_init(const EngineView& v, hipStream_t st);
+// Lifetime tables to build in the pool: a human table of kHumanAgeTable
+// thresholds and its guide, or the rows of one simulation's mosquitoes.
+struct HumanTable {
+    HumanLife life;
+    uint32_t off, guide;
+};
+struct MosquitoTable {
+    uint32_t off, guide;   // rows of dmax + 1 thresholds; [rows][256] guides
+    uint32_t dmax, rows;
+    float scale0, shape;   // row 0
+    uint32_t scales, days; // rows 1..: the daily scales at `scales`, `days` of them
+};
+
+hipError_t launch_life_tables(uint32_t* pool, const HumanTable* humans, uint32_t n_humans,
+                              const MosquitoTable* mosq, uint32_t n_mosq, uint32_t max_rows, const double* scales,
+                              hipStream_t st);
+hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st);
 hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_longdist(const EngineView& v, const Tuning& tu, hipStream_t st);

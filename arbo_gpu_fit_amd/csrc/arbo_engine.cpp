@@ -66,6 +66,9 @@ struct ArboEngine {
     DevBuf<unsigned long long> lam, scanned;
     DevBuf<uint32_t> part;   // per-community partials of the day
     DevBuf<float> dens;
+    DevBuf<double> scales;         // daily mosquito scales of the climates (lifetime tables)
+    DevBuf<HumanTable> life_h;
+    DevBuf<MosquitoTable> life_m;
     uint64_t series_total = 0;
     EngineView view{};
     // graph of kGraphDays days
@@ -130,6 +133,7 @@ void free_batch(ArboEngine* e) {
     dev_free(e->in_edge); dev_free(e->in_slot); dev_free(e->tables); dev_free(e->day_ctr);
     dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum);
     dev_free(e->lam); dev_free(e->scanned); dev_free(e->dens); dev_free(e->part);
+    dev_free(e->scales); dev_free(e->life_h); dev_free(e->life_m);
     e->ready = false;
 }
 
@@ -301,6 +305,13 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     std::vector<CommDesc> comm;
     std::vector<uint32_t> csr_thr, csr_inbox, in_edge, in_slot, table_pool;
     std::vector<float> dens_pool;
+    // lifetime tables, built on the device behind the uploaded ones: one per
+    // distinct set of parameters
+    std::vector<HumanTable> life_h;
+    std::vector<MosquitoTable> life_m;
+    std::vector<double> scales;
+    std::vector<uint32_t> sim_h(n_sims), sim_m(n_sims);
+    uint32_t max_rows = 1;
     std::map<std::vector<uint32_t>, uint32_t> seen_u32;
     std::map<std::vector<float>, uint32_t> seen_f32;
     uint64_t h_tot = 0, m_tot = 0, ser_tot = 0, spa_tot = 0;
@@ -339,8 +350,22 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         sd.intro = p.external_infection;
         sd.iip_min = p.iip_min;
         sd.iip_span = p.iip_max - p.iip_min + 1;
-        sd.death_h_off = pool_add(table_pool, seen_u32, t.death_h);
-        sd.death_m_off = pool_add(table_pool, seen_u32, t.death_m);
+        {
+            const HumanLife life{p.h_infant_shape, p.h_infant_scale, p.h_loc, p.h_scale, p.h_shape};
+            uint32_t k = 0;
+            while (k < life_h.size() && std::memcmp(&life_h[k].life, &life, sizeof life) != 0) ++k;
+            if (k == life_h.size()) life_h.push_back(HumanTable{life, 0u, 0u});
+            sim_h[i] = k;
+            MosquitoTable m{0u, 0u, t.death_m_max, t.m_rows, p.m_scale, p.m_shape, (uint32_t)scales.size(),
+                            t.climate ? max_days : 0u};
+            k = 0;   // rows that follow a climate are the simulation's own
+            while (k < life_m.size() && (t.climate || life_m[k].days || life_m[k].scale0 != m.scale0 ||
+                                         life_m[k].shape != m.shape)) ++k;
+            if (k == life_m.size()) life_m.push_back(m);
+            sim_m[i] = k;
+            scales.insert(scales.end(), t.scale.begin(), t.scale.end());
+            max_rows = std::max(max_rows, t.m_rows);
+        }
         sd.init_h_off = pool_add(table_pool, seen_u32, t.init_h);
         sd.init_m_off = pool_add(table_pool, seen_u32, t.init_m);
         sd.immune_off = pool_add(table_pool, seen_u32, t.immune);
@@ -350,7 +375,6 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         sd.seed_h = t.seed_h;
         sd.seed_m = t.seed_m;
         sd.death_m_max = t.death_m_max;
-        sd.death_m_guide_off = pool_add(table_pool, seen_u32, t.death_m_guide);
         sd.count_law = p.count_law;
         sd.no_distance = p.no_distance;
         death_m_lds = std::max(death_m_lds, t.death_m_max + 1);
@@ -414,6 +438,26 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     h_tot = align_up(h_tot, kHumanAlign) + kHumanAlign;
     m_tot = align_up(m_tot, kMosqAlign) + ARBO_MAX_COMMUNITY_SLOTS;  // room for whole-workgroup vector reads
     if (comm.size() >= (1ull << 31)) return fail(e, ARBO_E_INVALID, "too many communities in the batch");
+    uint64_t pool_words = table_pool.size();
+    for (HumanTable& h : life_h) {
+        pool_words = align_up(pool_words, 4);   // read as 16-byte vectors
+        h.off = (uint32_t)pool_words;
+        h.guide = h.off + kHumanAgeTable;
+        pool_words += kHumanAgeTable + kHumanGuide + 1;
+    }
+    for (MosquitoTable& m : life_m) {
+        m.off = (uint32_t)pool_words;
+        m.guide = m.off + m.rows * (m.dmax + 1);
+        pool_words += (uint64_t)m.rows * (m.dmax + 1 + kGuideBuckets);
+    }
+    if (pool_words >= (1ull << 32)) return fail(e, ARBO_E_ALLOC, "lifetime tables of the batch exceed 2^32 words");
+    for (uint32_t i = 0; i < n_sims; ++i) {
+        SimDesc& sd = e->sim_desc[i];
+        sd.death_h_off = life_h[sim_h[i]].off;
+        sd.death_h_guide_off = life_h[sim_h[i]].guide;
+        sd.death_m_off = life_m[sim_m[i]].off;
+        sd.death_m_guide_off = life_m[sim_m[i]].guide;
+    }
     e->n_comm = (uint32_t)comm.size();
     e->series_total = ser_tot;
 
@@ -431,7 +475,8 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         (rc = dev_alloc(e, e->hsum, comm.size() * 4)) || (rc = dev_alloc(e, e->active, comm.size())) ||
         (rc = dev_alloc(e, e->lam, (size_t)2 * n_sims * 8)) || (rc = dev_alloc(e, e->scanned, (size_t)2 * n_sims)) || (rc = dev_alloc(e, e->part, comm.size() * kPartWords)) || (rc = dev_alloc(e, e->series, ser_tot)) || (rc = dev_alloc(e, e->spatial, spa_tot)) ||
         (rc = dev_alloc(e, e->csr_thr, csr_thr.size())) || (rc = dev_alloc(e, e->csr_inbox, csr_inbox.size())) || (rc = dev_alloc(e, e->in_edge, in_edge.size())) ||
-        (rc = dev_alloc(e, e->in_slot, in_slot.size())) || (rc = dev_alloc(e, e->tables, table_pool.size())) ||
+        (rc = dev_alloc(e, e->in_slot, in_slot.size())) || (rc = dev_alloc(e, e->tables, pool_words)) || (rc = dev_alloc(e, e->scales, scales.size())) ||
+        (rc = dev_alloc(e, e->life_h, life_h.size())) || (rc = dev_alloc(e, e->life_m, life_m.size())) ||
         (rc = dev_alloc(e, e->dens, dens_pool.size())) || (rc = dev_alloc(e, e->day_ctr, 1))) {
         free_batch(e);
         return rc;
@@ -444,6 +489,11 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     HIP_TRY(e, hipMemcpy(e->in_slot.p, in_slot.data(), in_slot.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->tables.p, table_pool.data(), table_pool.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->dens.p, dens_pool.data(), dens_pool.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(e, hipMemcpy(e->life_h.p, life_h.data(), life_h.size() * sizeof(HumanTable), hipMemcpyHostToDevice));
+    HIP_TRY(e, hipMemcpy(e->life_m.p, life_m.data(), life_m.size() * sizeof(MosquitoTable), hipMemcpyHostToDevice));
+    if (!scales.empty()) HIP_TRY(e, hipMemcpy(e->scales.p, scales.data(), scales.size() * sizeof(double), hipMemcpyHostToDevice));
+    HIP_TRY(e, launch_life_tables(e->tables.p, e->life_h.p, (uint32_t)life_h.size(), e->life_m.p, (uint32_t)life_m.size(),
+                                  max_rows, e->scales.p, e->stream));
     HIP_TRY(e, launch_fill(e->series.p, ser_tot, 0u, e->stream));
     if (spa_tot) HIP_TRY(e, launch_fill(e->spatial.p, spa_tot, 0u, e->stream));
     HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->lam.p), (uint64_t)2 * n_sims * 8 * 2, 0u, e->stream));
@@ -512,7 +562,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         v.reduce_split = std::min<uint32_t>(cap, (max_c + 255) / 256);
     }
 
-    HIP_TRY(e, launch_init(v, e->stream));
+    HIP_TRY(e, launch_init(v, std::max(max_n, max_cap), e->stream));
     HIP_TRY(e, hipStreamSynchronize(e->stream));
     e->day = 0;
     e->ready = true;

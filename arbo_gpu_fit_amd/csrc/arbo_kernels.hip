@@ -42,6 +42,7 @@
 #include "arbo_c.h"
 #include "arbo_device.h"
 #include "arbo_rng.h"
+#include "arbo_tables.h"
 
 namespace arbo {
 
@@ -58,7 +59,6 @@ constexpr uint32_t kHash = 512;                                // claim-table en
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr uint32_t kKeyBits = 17;                              // member index < 2^17
 constexpr uint32_t kKeyMask = (1u << kKeyBits) - 1u;
-constexpr uint32_t kHumanTable = 65536;
 constexpr uint32_t kMaxRowLen = 9;                             // Moore-8 + self
 constexpr uint32_t kGuide = 256;                               // death-age guide entries (life_bucket, padded)
 static_assert(kMaxWaves == 8, "eight waves cover the largest community's bitmap");
@@ -117,20 +117,8 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t x, uint32_t& to
     return v - x;
 }
 
-// min{a in [1, hi] : K[a] >= k}; hi when K[hi] < k (hi = table end).
-template <class P>
-__device__ __forceinline__ uint32_t death_age(P K, uint32_t hi, uint32_t k) {
-    if (K[hi] < k) return hi;
-    uint32_t lo = 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (K[mid] >= k) hi = mid; else lo = mid + 1;
-    }
-    return lo;
-}
-
-// The same minimum, started from the smallest death age of k's bucket:
-// guide[b] = min{a >= 1 : K[a] >= life_bucket_kmin(b)} <= result.
+// A mosquito's death age min{a in [1, hi] : K[a] >= k} (hi when K[hi] < k),
+// from the smallest death age of k's bucket: guide[b] = min{a >= 1 : K[a] >= life_bucket_kmin(b)} <= result.
 __device__ __forceinline__ uint32_t death_age_guided(const uint32_t* K, const uint32_t* guide, uint32_t hi,
                                                      uint32_t k) {
     uint32_t a = guide[life_bucket(k)];
@@ -138,11 +126,26 @@ __device__ __forceinline__ uint32_t death_age_guided(const uint32_t* K, const ui
     return a;
 }
 
-// Death age given survival to age a0: PLE uniform on (F(a0-1), 1].
-__device__ __forceinline__ uint32_t death_age_given(const uint32_t* K, uint32_t hi, uint32_t a0, uint32_t r) {
+// A human's death age (kHumanAgeTable thresholds K): the same minimum between
+// the smallest death ages of the draw's slice of kHumanGuide and of the next
+// (guide[i] = min{a >= 1 : K[a] > i 2^12}, the table's last age where none is).
+// Three dependent loads or so where the search of the whole table has 16.
+__device__ __forceinline__ uint32_t human_death_age(const uint32_t* K, const uint32_t* guide, uint32_t k) {
+    const uint32_t i = (k - 1u) >> 12;
+    uint32_t lo = guide[i], hi = guide[i + 1];
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (K[mid] >= k) hi = mid; else lo = mid + 1;
+    }
+    return lo;
+}
+static_assert((kHumanGuide << 12) == (1u << 24), "slices of 2^12 draws");
+
+// The PLE draw of a death age given survival to age a0, uniform on (F(a0-1), 1];
+// 0 when F(a0 - 1) is 1: the death age is a0.
+__device__ __forceinline__ uint32_t surviving_draw(const uint32_t* K, uint32_t a0, uint32_t r) {
     const uint32_t prev = K[a0 >= 1 ? a0 - 1 : 0];
-    if (prev >= (1u << 24)) return a0;
-    return death_age(K, hi, prev + 1 + mulhi(r, (1u << 24) - prev));
+    return prev >= (1u << 24) ? 0u : prev + 1 + mulhi(r, (1u << 24) - prev);
 }
 
 // min{i : k <= T[i]} over a table ending at 2^24.
@@ -199,85 +202,228 @@ __device__ __forceinline__ void select_bit(uint32_t q, const uint32_t* word, con
 }
 
 // ---------------------------------------------------------------------------
-// t = 0 census: demographicintial.cu:86-297, epidemicinitial.cu:27-99.
-__global__ __launch_bounds__(kWave) void k_init(EngineView v) {
-    const uint32_t g = blockIdx.x, lane = threadIdx.x;
+// Lifetime tables (see arbo_tables.cpp): a threshold is two or three
+// exponentials and logarithms in double, 65,536 of them for the humans and up
+// to 2,047 for each day a mosquito may be born under a climate, every time a
+// batch is initialised (an MCMC iteration is one): 3 ms of the host for one
+// simulation, 13 for 364 climate rows, against 40-55 us here.
+
+// Inclusive running maximum over the workgroup's threads, 64 NW of them.
+template <uint32_t NW>
+__device__ __forceinline__ uint32_t block_max_scan(uint32_t x, uint32_t* s_w, uint32_t tid) {
+    const uint32_t lane = tid & (kWave - 1), wv = tid / kWave;
+#pragma unroll
+    for (uint32_t d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d, kWave);
+        if (lane >= d && y > x) x = y;
+    }
+    if (lane == kWave - 1) s_w[wv] = x;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w < NW; ++w)
+        if (w < wv && s_w[w] > x) x = s_w[w];
+    __syncthreads();
+    return x;
+}
+
+// Thresholds of 256 human ages of table blockIdx.y.
+__global__ __launch_bounds__(256) void k_life_human(uint32_t* pool, const HumanTable* tables) {
+    const HumanTable& h = tables[blockIdx.y];
+    const uint32_t a = blockIdx.x * 256 + threadIdx.x;
+    pool[h.off + a] = fixed24(human_cdf(h.life, (double)a));
+}
+
+// Their running maximum (thresholds never fall, whatever the last bit of a
+// double does) and the guide, one workgroup a table.
+__global__ __launch_bounds__(1024) void k_life_human_guide(uint32_t* pool, const HumanTable* tables) {
+    __shared__ uint32_t s_w[16];
+    const HumanTable& h = tables[blockIdx.x];
+    const uint32_t tid = threadIdx.x;
+    uint32_t* K = pool + h.off;
+    constexpr uint32_t kPer = kHumanAgeTable / 1024;
+    uint4* K4 = reinterpret_cast<uint4*>(K) + tid * (kPer / 4);   // tables start on multiples of four words
+    uint4 k[kPer / 4];
+    uint32_t m = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kPer / 4; ++q) {
+        k[q] = K4[q];
+        m = k[q].x > m ? k[q].x : m; k[q].x = m;
+        m = k[q].y > m ? k[q].y : m; k[q].y = m;
+        m = k[q].z > m ? k[q].z : m; k[q].z = m;
+        m = k[q].w > m ? k[q].w : m; k[q].w = m;
+    }
+    const uint32_t mine = m;
+    const uint32_t upto = block_max_scan<16>(mine, s_w, tid);   // of this thread and those before
+    // the maximum before this thread: its neighbour's
+    uint32_t prev = __shfl_up(upto, 1, kWave);
+    __shared__ uint32_t s_last[16];
+    if ((tid & 63u) == 63u) s_last[tid / kWave] = upto;
+    __syncthreads();
+    if ((tid & 63u) == 0u) prev = tid ? s_last[tid / kWave - 1] : 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kPer / 4; ++q) {
+        k[q].x = k[q].x > prev ? k[q].x : prev;
+        k[q].y = k[q].y > prev ? k[q].y : prev;
+        k[q].z = k[q].z > prev ? k[q].z : prev;
+        k[q].w = k[q].w > prev ? k[q].w : prev;
+        K4[q] = k[q];
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i <= kHumanGuide; i += 1024) {
+        uint32_t lo = 1, hi = kHumanAgeTable - 1;
+        if (i == kHumanGuide) lo = hi;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (K[mid] > (i << 12)) hi = mid; else lo = mid + 1;
+        }
+        pool[h.guide + i] = lo;
+    }
+}
+
+// One lifetime row of the mosquitoes of table blockIdx.y and its guide.
+__global__ __launch_bounds__(256) void k_life_mosquito(uint32_t* pool, const MosquitoTable* tables, const double* scales) {
+    __shared__ uint32_t s_k[kMosqAgeTable];
+    __shared__ uint32_t s_w[4];
+    const MosquitoTable& m = tables[blockIdx.y];
+    const uint32_t row = blockIdx.x, tid = threadIdx.x;
+    if (row >= m.rows) return;   // workgroup-uniform
+    uint32_t carry = 0;
+    for (uint32_t a0 = 0; a0 <= m.dmax; a0 += 256) {
+        const uint32_t a = a0 + tid;
+        uint32_t k = 0;
+        if (a <= m.dmax && (row == 0 || a > 0)) {
+            double scale = (double)m.scale0;
+            if (row > 0) {   // born on day row - 1, of age a on day row - 1 + a
+                const uint64_t day = (uint64_t)(row - 1) + a;
+                scale = scales[m.scales + (day < m.days ? (uint32_t)day : m.days - 1)];
+            }
+            k = fixed24(weibull_cdf((double)a, scale, (double)m.shape));
+        }
+        k = block_max_scan<4>(k > carry ? k : carry, s_w, tid);
+        if (a <= m.dmax) s_k[a] = a == m.dmax ? 1u << 24 : k;
+        __syncthreads();
+        carry = s_k[a0 + 255 < m.dmax ? a0 + 255 : m.dmax];
+    }
+    for (uint32_t a = tid; a <= m.dmax; a += 256) pool[m.off + row * (m.dmax + 1) + a] = s_k[a];
+    if (tid < kGuide) {   // the smallest death age of every life_bucket() of draws (padding: the largest)
+        uint32_t lo = 1, hi = m.dmax;
+        const uint32_t k = tid < kLifeBuckets ? life_bucket_kmin(tid) : 1u << 24;
+        if (tid >= kLifeBuckets) lo = hi;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (s_k[mid] >= k) hi = mid; else lo = mid + 1;
+        }
+        pool[m.guide + row * kGuide + tid] = lo;
+    }
+}
+static_assert(kGuide == kGuideBuckets && kGuide <= 256, "a thread per guide entry");
+
+// t = 0 census: demographicintial.cu:86-297, epidemicinitial.cu:27-99.  The
+// members of a community are dealt to gridDim.y workgroups of four waves
+// (kInitMembers at most a workgroup, so that one city does not hold the whole
+// launch), which stage the initial-age tables and the mosquito lifetimes in
+// LDS; counts are added with integer atomics.  One wave per community, its
+// searches in memory: 2.5 ms for 49 cities of up to 21,000 humans, 11.8 ms for
+// 257,000 communities; this 0.06 and 5.9, of which 1.3 are the 6.2 GB written.
+constexpr uint32_t kInitMembers = 4096;
+__global__ __launch_bounds__(256) void k_init(EngineView v) {
+    extern __shared__ uint32_t s_dtab[];   // mosquito lifetime thresholds
+    __shared__ uint32_t s_ih[kHumanYears], s_im[kMosqInitDays], s_guide[kLifeBuckets];
+    __shared__ uint32_t s_cnt[4];
+    const uint32_t g = blockIdx.x, part = blockIdx.y, parts = gridDim.y, tid = threadIdx.x;
     const CommDesc cd = v.comm[g];
-    const SimDesc sd = v.sims[cd.sim];
+    if (part * kInitMembers >= cd.n && part * kInitMembers >= cd.cap) return;   // workgroup-uniform
+    const SimDesc& sd = v.sims[cd.sim];
     const Key key{sd.k0, sd.k1};
-    const uint32_t S = sd.S;
+    const uint32_t S = sd.S, dmax = sd.death_m_max;
     const uint32_t* death_h = v.tables + sd.death_h_off;
-    const uint32_t* death_m = v.tables + sd.death_m_off;
-    const uint32_t* init_h = v.tables + sd.init_h_off;
-    const uint32_t* init_m = v.tables + sd.init_m_off;
-    const uint32_t* immune = v.tables + sd.immune_off + (size_t)cd.c * S;
+    const uint32_t* guide_h = v.tables + sd.death_h_guide_off;
+    for (uint32_t i = tid; i < kHumanYears; i += 256) s_ih[i] = v.tables[sd.init_h_off + i];
+    for (uint32_t i = tid; i < kMosqInitDays; i += 256) s_im[i] = v.tables[sd.init_m_off + i];
+    for (uint32_t i = tid; i < kLifeBuckets; i += 256) s_guide[i] = v.tables[sd.death_m_guide_off + i];
+    for (uint32_t i = tid; i <= dmax; i += 256) s_dtab[i] = v.tables[sd.death_m_off + i];
+    if (tid < 4) s_cnt[tid] = 0u;
+    uint32_t immune[4] = {0u, 0u, 0u, 0u}, some = 0u;
+    for (uint32_t s = 0; s < S; ++s) {
+        immune[s] = v.tables[sd.immune_off + (size_t)cd.c * S + s];
+        some |= immune[s];
+    }
     uint32_t alive0;
     {
         const U4 r = draw(key, cd.c, INIT_DAY, P_INIT_MT, 0);
         const uint32_t a = stoch_round(v.dens[sd.dens_off] * cd.base, r.x);
         alive0 = a < cd.cap ? a : cd.cap;
     }
-    uint32_t ih01 = 0, ih23 = 0;
-    for (uint32_t i = lane; i < cd.n; i += kWave) {
-        const uint32_t h = cd.h_base + i;
-        const U4 r0 = draw(key, h, INIT_DAY, P_INIT_H, 0);
-        const uint32_t y = pick_index(init_h, 151, (r0.x >> 8) + 1);
-        const uint32_t a0 = 365u * y + mulhi(r0.y, 365);
-        const uint32_t da = death_age_given(death_h, kHumanTable - 1, a0, r0.z);
-        const int32_t ddi = (int32_t)da - (int32_t)(a0 + 1);
-        const uint32_t dd = ddi < 0 ? 0u : (uint32_t)ddi;
-        const U4 r1 = draw(key, h, INIT_DAY, P_INIT_H, 1);
-        const uint32_t rr[4] = {r1.x, r1.y, r1.z, r1.w};
-        uint32_t imm = 0;
-        for (uint32_t s = 0; s < S; ++s)
-            if ((rr[s] >> 8) < immune[s]) imm |= 1u << s;
-        uint32_t st = 0, strain = 0, nxt = 0;
-        if ((r0.w >> 8) < sd.seed_h) {
-            const U4 r2 = draw(key, h, INIT_DAY, P_INIT_H, 2);
-            strain = mulhi(r2.x, S);
-            st = 2;
-            imm |= 1u << strain;
-            uint32_t R = stoch_round(sd.recovery, r2.z);
-            if (R < 1) R = 1;
-            nxt = mulhi(r2.y, R);
-            add_pair(ih01, ih23, strain);
+    __syncthreads();
+    for (uint32_t base = part * kInitMembers; base < cd.n; base += parts * kInitMembers) {
+        const uint32_t end = base + kInitMembers < cd.n ? base + kInitMembers : cd.n;
+        for (uint32_t i = base + tid; i < end; i += 256) {
+            const uint32_t h = cd.h_base + i;
+            const U4 r0 = draw(key, h, INIT_DAY, P_INIT_H, 0);
+            const uint32_t y = pick_index(s_ih, kHumanYears, (r0.x >> 8) + 1);
+            const uint32_t a0 = 365u * y + mulhi(r0.y, 365);
+            const uint32_t k = surviving_draw(death_h, a0, r0.z);
+            const uint32_t da = k ? human_death_age(death_h, guide_h, k) : a0;
+            const int32_t ddi = (int32_t)da - (int32_t)(a0 + 1);
+            const uint32_t dd = ddi < 0 ? 0u : (uint32_t)ddi;
+            uint32_t imm = 0;
+            if (some) {   // prior immunity in this community
+                const U4 r1 = draw(key, h, INIT_DAY, P_INIT_H, 1);
+                const uint32_t rr[4] = {r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+                for (uint32_t s = 0; s < 4; ++s)
+                    if ((rr[s] >> 8) < immune[s]) imm |= 1u << s;
+            }
+            uint32_t st = 0, strain = 0, nxt = 0;
+            if ((r0.w >> 8) < sd.seed_h) {
+                const U4 r2 = draw(key, h, INIT_DAY, P_INIT_H, 2);
+                strain = mulhi(r2.x, S);
+                st = 2;
+                imm |= 1u << strain;
+                uint32_t R = stoch_round(sd.recovery, r2.z);
+                if (R < 1) R = 1;
+                nxt = mulhi(r2.y, R);
+                atomicAdd(&s_cnt[strain], 1u);
+            }
+            const uint64_t gi = cd.h_off + i;
+            v.h_word[gi] = (dd << 8) | (imm << 4) | (strain << 2) | st;
+            v.h_next[gi] = (uint16_t)nxt;
+            v.h_birth[gi] = -(int32_t)(a0 + 1);
+            if (v.hist)   // immune at t = 0 (prior immunity or the seeded infection): -2, naive: -1
+                reinterpret_cast<int4*>(v.hist)[gi] = make_int4((imm & 1u) ? -2 : -1, (imm & 2u) ? -2 : -1,
+                                                                (imm & 4u) ? -2 : -1, (imm & 8u) ? -2 : -1);
         }
-        const uint64_t gi = cd.h_off + i;
-        v.h_word[gi] = (dd << 8) | (imm << 4) | (strain << 2) | st;
-        v.h_next[gi] = (uint16_t)nxt;
-        v.h_birth[gi] = -(int32_t)(a0 + 1);
-        if (v.hist)   // immune at t = 0 (prior immunity or the seeded infection): -2, naive: -1
-            reinterpret_cast<int4*>(v.hist)[gi] = make_int4((imm & 1u) ? -2 : -1, (imm & 2u) ? -2 : -1,
-                                                            (imm & 4u) ? -2 : -1, (imm & 8u) ? -2 : -1);
     }
-    for (uint32_t j = lane; j < cd.cap; j += kWave) {
-        const uint64_t gm = cd.m_off + j;
-        v.m_next[gm] = 0;
-        if (j >= alive0) { v.m_word[gm] = 3; continue; }
-        const uint32_t m = cd.m_base + j;
-        const U4 r0 = draw(key, m, INIT_DAY, P_INIT_M, 0);
-        const uint32_t a0 = pick_index(init_m, 301, (r0.x >> 8) + 1);
-        const uint32_t da = death_age_given(death_m, sd.death_m_max, a0, r0.z);
-        const uint32_t dd12 = (uint32_t)((int32_t)da - (int32_t)(a0 + 1)) & 0xFFFu;
-        uint32_t st = 0, strain = 0;
-        if ((r0.w >> 8) < sd.seed_m) {
-            st = 2;
-            strain = mulhi(r0.y, S);
+    for (uint32_t base = part * kInitMembers; base < cd.cap; base += parts * kInitMembers) {
+        const uint32_t end = base + kInitMembers < cd.cap ? base + kInitMembers : cd.cap;
+        for (uint32_t j = base + tid; j < end; j += 256) {
+            const uint64_t gm = cd.m_off + j;
+            v.m_next[gm] = 0;
+            if (j >= alive0) { v.m_word[gm] = 3; continue; }
+            const uint32_t m = cd.m_base + j;
+            const U4 r0 = draw(key, m, INIT_DAY, P_INIT_M, 0);
+            const uint32_t a0 = pick_index(s_im, kMosqInitDays, (r0.x >> 8) + 1);
+            const uint32_t k = a0 > dmax ? 0u : surviving_draw(s_dtab, a0, r0.z);
+            const uint32_t da = k ? death_age_guided(s_dtab, s_guide, dmax, k) : a0;
+            const uint32_t dd12 = (uint32_t)((int32_t)da - (int32_t)(a0 + 1)) & 0xFFFu;
+            uint32_t st = 0, strain = 0;
+            if ((r0.w >> 8) < sd.seed_m) {
+                st = 2;
+                strain = mulhi(r0.y, S);
+            }
+            v.m_word[gm] = (uint16_t)((dd12 << 4) | (strain << 2) | st);
         }
-        v.m_word[gm] = (uint16_t)((dd12 << 4) | (strain << 2) | st);
     }
-    ih01 = wave_sum(ih01);
-    ih23 = wave_sum(ih23);
+    __syncthreads();
     const SeriesIdx si = series_index(sd.series_off, v.max_days, S);
-    if (lane == 0) {
+    if (tid == 0 && part == 0) {
         atomicAdd(&v.series[si.n_count], cd.n);
         atomicAdd(&v.series[si.m_count], alive0);
     }
-    if (lane < S) {
-        const uint32_t ih = unpack_pair(ih01, ih23, lane);
-        atomicAdd(&v.series[si.n_inf + lane], ih);
-        if (cd.c == 0) v.series[si.n_one + lane] = ih;
-        if (v.spatial) v.spatial[sd.spatial_off + (uint64_t)lane * sd.C + cd.c] = ih;   // row 0
+    if (tid < S && s_cnt[tid]) {   // row 0, zero until here
+        atomicAdd(&v.series[si.n_inf + tid], s_cnt[tid]);
+        if (cd.c == 0) atomicAdd(&v.series[si.n_one + tid], s_cnt[tid]);
+        if (v.spatial) atomicAdd(&v.spatial[sd.spatial_off + (uint64_t)tid * sd.C + cd.c], s_cnt[tid]);
     }
 }
 
@@ -360,7 +506,7 @@ __device__ __forceinline__ void human_deferred(const EngineView& v, const CommDe
         const uint64_t gi = cd.h_off + i;
         if (w < ((t + 1u) << 8)) {   // death and instant rebirth
             const U4 r = draw(key, cd.h_base + i, t, P_H_BIRTH, 0);
-            const uint32_t da = death_age(v.tables + sd.death_h_off, kHumanTable - 1, (r.x >> 8) + 1);
+            const uint32_t da = human_death_age(v.tables + sd.death_h_off, v.tables + sd.death_h_guide_off, (r.x >> 8) + 1);
             v.h_word[gi] = (t + da) << 8;
             v.h_birth[gi] = (int32_t)t;
             if (HIST && v.hist) reinterpret_cast<int4*>(v.hist)[gi] = make_int4(-1, -1, -1, -1);   // naive newborn
@@ -1523,8 +1669,29 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t value) {
 
 // ---------------------------------------------------------------------------
 // Launchers (host).
-hipError_t launch_init(const EngineView& v, hipStream_t st) {
-    hipLaunchKernelGGL(k_init, dim3(v.n_comm), dim3(kWave), 0, st, v);
+hipError_t launch_life_tables(uint32_t* pool, const HumanTable* humans, uint32_t n_humans,
+                              const MosquitoTable* mosq, uint32_t n_mosq, uint32_t max_rows, const double* scales,
+                              hipStream_t st) {
+    constexpr uint32_t kMostY = 65535;   // tables of one launch
+    for (uint32_t i = 0; i < n_humans; i += kMostY) {
+        const uint32_t n = n_humans - i < kMostY ? n_humans - i : kMostY;
+        hipLaunchKernelGGL(k_life_human, dim3(kHumanAgeTable / 256, n), dim3(256), 0, st, pool, humans + i);
+    }
+    hipLaunchKernelGGL(k_life_human_guide, dim3(n_humans), dim3(1024), 0, st, pool, humans);
+    for (uint32_t i = 0; i < n_mosq; i += kMostY) {
+        const uint32_t n = n_mosq - i < kMostY ? n_mosq - i : kMostY;
+        hipLaunchKernelGGL(k_life_mosquito, dim3(max_rows, n), dim3(256), 0, st, pool, mosq + i, scales);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
+    // workgroups per community: those its largest one has work for, while the launch stays small
+    uint32_t parts = (largest + kInitMembers - 1) / kInitMembers, most = 16384u / v.n_comm;
+    if (most < 1) most = 1;
+    if (parts > most) parts = most;
+    if (parts < 1) parts = 1;
+    hipLaunchKernelGGL(k_init, dim3(v.n_comm, parts), dim3(256), (size_t)v.death_m_lds * 4, st, v);
     return hipGetLastError();
 }
 

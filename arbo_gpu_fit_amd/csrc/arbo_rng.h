@@ -259,6 +259,28 @@ ARBO_HD double dlogfact(double k) {
     return (x - 0.5) * dlog(x) - x + half_log_2pi + series * ix;
 }
 
+// x^y for x >= 0 (0 at 0), y real.
+ARBO_HD double powd(double x, double y) { return x > 0.0 ? dexp(y * dlog(x)) : 0.0; }
+
+// floor(f 2^24), clamped to [0, 2^24].
+ARBO_HD uint32_t fixed24(double f) {
+    const double v = floor(f * 16777216.0);
+    if (!(v > 0.0)) return 0u;
+    if (v >= 16777216.0) return 1u << 24;
+    return (uint32_t)v;
+}
+
+// Lifetime distributions.  Humans (ndemographic.cu:13-29): F(a) = 1 -
+// exp(-[(a b)^alpha + 1{a >= L} ((a-L)/d)^c]); mosquitoes
+// (mdemographic.cu:13-17): F(a) = 1 - exp(-(a/scale)^shape).
+struct HumanLife { float infant_shape, infant_scale, loc, scale, shape; };
+ARBO_HD double human_cdf(const HumanLife& p, double a) {
+    double haz = powd(a * (double)p.infant_scale, (double)p.infant_shape);
+    if (a >= (double)p.loc) haz = haz + powd((a - (double)p.loc) / (double)p.scale, (double)p.shape);
+    return 1.0 - dexp(-haz);
+}
+ARBO_HD double weibull_cdf(double a, double scale, double shape) { return 1.0 - dexp(-powd(a / scale, shape)); }
+
 // Counter base of one Poisson variate: x3 is the draw index.
 struct Stream { Key key; uint32_t x0, x1, x2; };
 

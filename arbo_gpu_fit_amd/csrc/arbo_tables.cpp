@@ -3,8 +3,8 @@
 // Lifetimes: the reference draws PLE ~ U(0,1] at birth and kills on the first
 // day with F(age) >= PLE (ndemographic.cu:62, mdemographic.cu:72).  Here F is
 // tabulated once per parameter set as 24-bit thresholds K[a] = floor(F(a) 2^24)
-// and the kernels search K for a 24-bit PLE: an exact integer version of the
-// same law.  Initial ages follow the cumulative survival sums of
+// (on the device, from the same double arithmetic) and the kernels search K
+// for a 24-bit PLE: an exact integer version of the same law.  Initial ages follow the cumulative survival sums of
 // demographicintial.cu:48-83.  The network is the reference's non-wrapping
 // lattice (network.cpp:31-41) with rows in ascending column order
 // (network.cpp:95-113), generalised to Moore neighbourhoods, a self entry and
@@ -19,25 +19,10 @@
 
 namespace arbo {
 
-uint32_t fixed24(double f) {
-    const double v = floor(f * 16777216.0);
-    if (!(v > 0.0)) return 0u;
-    if (v >= 16777216.0) return kOne24;
-    return (uint32_t)v;
+static HumanLife human_life(const ArboParams& p) {
+    return HumanLife{p.h_infant_shape, p.h_infant_scale, p.h_loc, p.h_scale, p.h_shape};
 }
-
-static double powd(double x, double y) { return x > 0.0 ? dexp(y * dlog(x)) : 0.0; }
-
-// ndemographic.cu:13-29: F(a) = 1 - exp(-[(a b)^alpha + 1{a >= L} ((a-L)/d)^c]).
-static double human_cdf(const ArboParams& p, double a) {
-    double haz = powd(a * (double)p.h_infant_scale, (double)p.h_infant_shape);
-    if (a >= (double)p.h_loc) haz = haz + powd((a - (double)p.h_loc) / (double)p.h_scale, (double)p.h_shape);
-    return 1.0 - dexp(-haz);
-}
-
-// mdemographic.cu:13-17: F(a) = 1 - exp(-(a/scale)^shape).
-static double weibull_cdf(double a, double scale, double shape) { return 1.0 - dexp(-powd(a / scale, shape)); }
-
+static double human_cdf(const ArboParams& p, double a) { return human_cdf(human_life(p), a); }
 static double mosq_cdf(const ArboParams& p, double a) { return weibull_cdf(a, (double)p.m_scale, (double)p.m_shape); }
 
 // ---- climate (SimulationParam.cpp:92-137, simulation.cpp:87,129-131) ----
@@ -96,16 +81,12 @@ static std::string validate_climate(const ArboClimate& c, uint32_t max_days) {
     return std::string();
 }
 
+// The first age from 1 whose threshold is 2^24, at most the table's last.
 template <class Cdf>
-static void threshold_table(uint32_t n, Cdf cdf, std::vector<uint32_t>& K) {
-    K.resize(n);
-    uint32_t prev = 0;
-    for (uint32_t a = 0; a < n; ++a) {
-        uint32_t k = fixed24(cdf((double)a));
-        if (k < prev) k = prev;
-        K[a] = k;
-        prev = k;
-    }
+static uint32_t first_certain(Cdf cdf) {
+    uint32_t a = 1;
+    while (a < kMosqAgeTable - 1 && fixed24(cdf((double)a)) < kOne24) ++a;
+    return a;
 }
 
 template <class Cdf>
@@ -280,59 +261,29 @@ static void build_network(const ArboParams& p, SimTables& t) {
     }
 }
 
-// Mosquito lifetime rows and their guides.  Row 0 is the tabulated F of
-// m_scale.  With a climate, a mosquito born on day b dies on the first day
-// b + a whose F(a; scale(b + a)) reaches its PLE (mdemographic.cu:72 with the
-// day's mScaleLifeExpectancy); the running maximum over a of those
-// thresholds turns that first passage into a search of a monotone row.
-// Days past the run use the last day's scale.  Every row ends at its first
-// 2^24 entry, and all rows share the largest such length.
-static void build_mosquito_rows(const ArboShape& sh, const ArboParams& p, uint32_t max_days, SimTables& t) {
-    std::vector<std::vector<uint32_t>> rows;
-    rows.emplace_back();
-    threshold_table(kMosqAgeTable, [&](double a) { return mosq_cdf(p, a); }, rows[0]);
-    if (t.climate) {
-        std::vector<double> scale(max_days);
-        for (uint32_t d = 0; d < max_days; ++d) {
-            double x[4];
-            climate_day(*sh.climate, d + 1, x);
-            scale[d] = x[3];
-        }
-        for (uint32_t b = 0; b < max_days; ++b) {
-            std::vector<uint32_t> K(1, 0u);
-            uint32_t run = 0;
-            for (uint32_t a = 1; a < kMosqAgeTable && run < kOne24; ++a) {
-                const uint64_t day = std::min<uint64_t>((uint64_t)b + a, max_days - 1);
-                run = std::max(run, fixed24(weibull_cdf((double)a, scale[day], (double)p.m_shape)));
-                K.push_back(run);
-            }
-            rows.push_back(std::move(K));
-        }
+// What sizes the mosquito lifetime rows.  Row 0 is the tabulated F of m_scale.
+// With a climate, a mosquito born on day b dies on the first day b + a whose
+// F(a; scale(b + a)) reaches its PLE (mdemographic.cu:72 with the day's
+// mScaleLifeExpectancy); the running maximum over a of those thresholds turns
+// that first passage into a search of a monotone row.  Days past the run use
+// the last day's scale.  Every such row reaches 2^24 no later than F of the
+// run's largest scale does; one more day covers the rounding of F.
+static void size_mosquito_rows(const ArboShape& sh, const ArboParams& p, uint32_t max_days, SimTables& t) {
+    t.m_rows = 1;
+    t.death_m_max = first_certain([&](double a) { return mosq_cdf(p, a); });
+    t.scale.clear();
+    if (!t.climate) return;
+    t.m_rows = max_days + 1;
+    t.scale.resize(max_days);
+    double smax = 0.0;
+    for (uint32_t d = 0; d < max_days; ++d) {
+        double x[4];
+        climate_day(*sh.climate, d + 1, x);
+        t.scale[d] = x[3];
+        smax = std::max(smax, x[3]);
     }
-    // the largest death age any row returns: its first 2^24 entry, else the table end
-    uint32_t dmax = 1;
-    for (const auto& K : rows) {
-        uint32_t first = kMosqAgeTable - 1;
-        for (uint32_t a = 1; a < K.size(); ++a)
-            if (K[a] >= kOne24) { first = a; break; }
-        dmax = std::max(dmax, first);
-    }
-    t.death_m_max = dmax;
-    t.m_rows = (uint32_t)rows.size();
-    t.death_m.assign((size_t)t.m_rows * (dmax + 1), kOne24);
-    t.death_m_guide.assign((size_t)t.m_rows * kGuideBuckets, dmax);
-    for (uint32_t r = 0; r < t.m_rows; ++r) {
-        uint32_t* K = t.death_m.data() + (size_t)r * (dmax + 1);
-        for (uint32_t a = 0; a <= dmax && a < rows[r].size(); ++a) K[a] = rows[r][a];
-        K[dmax] = kOne24;
-        // the smallest death age of every life_bucket() of 24-bit draws (padding: the largest)
-        for (uint32_t b = 0; b < kLifeBuckets; ++b) {
-            const uint32_t k = life_bucket_kmin(b);
-            uint32_t a = 1;
-            while (a < dmax && K[a] < k) ++a;
-            t.death_m_guide[(size_t)r * kGuideBuckets + b] = a;
-        }
-    }
+    const uint32_t last = first_certain([&](double a) { return weibull_cdf(a, smax, (double)p.m_shape); });
+    t.death_m_max = std::max(t.death_m_max, std::min(last + 1, kMosqAgeTable - 1));
 }
 
 void build_tables(const ArboShape& sh, const ArboParams& p, uint64_t seed, uint32_t max_days,
@@ -376,8 +327,7 @@ void build_tables(const ArboShape& sh, const ArboParams& p, uint64_t seed, uint3
         else t.base[c] = t.climate ? (float)hs : (float)((double)p.m_ratio * hs);
         t.n_slots += t.slots[c];
     }
-    threshold_table(kHumanAgeTable, [&](double a) { return human_cdf(p, a); }, t.death_h);
-    build_mosquito_rows(sh, p, max_days, t);
+    size_mosquito_rows(sh, p, max_days, t);
     initial_age_table(kHumanYears, 365, [&](double a) { return human_cdf(p, a); }, t.init_h);
     initial_age_table(kMosqInitDays, 1, [&](double a) { return mosq_cdf(p, a); }, t.init_m);
     if (!t.climate) {

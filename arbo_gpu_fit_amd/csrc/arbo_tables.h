@@ -19,20 +19,21 @@ constexpr uint32_t kMosqInitDays = 301;     // C_MMAXINITIALAGE + 1 (constant.h:
 constexpr uint32_t kOne24 = 1u << 24;
 constexpr uint32_t kMaxRow = 9;             // Moore-8 + self
 constexpr uint32_t kGuideBuckets = 256;     // life_bucket() range (176), padded
+constexpr uint32_t kHumanGuide = 4096;      // equal slices of the 24-bit draws in the human table's guide
 
 struct SimTables {
     uint32_t W = 0, H = 0, C = 0, S = 0;
     std::vector<uint32_t> humans, slots;   // per community
     std::vector<float> base;               // m_ratio * humans, f32
-    std::vector<uint32_t> death_h;         // [kHumanAgeTable]  floor(F_h(a) 2^24)
-    // mosquito lifetimes, m_rows rows of death_m_max + 1 thresholds: row 0
-    // floor(F_m(a) 2^24) of m_scale (the t = 0 census; every birth without a
-    // climate); with a climate, row 1 + b the running maximum over a' <= a of
-    // floor(F_m(a'; scale(b + a')) 2^24) for births on day b
-    std::vector<uint32_t> death_m;
-    uint32_t death_m_max = 0;              // largest death age any row returns (its first 2^24 entry)
+    // Lifetime thresholds are tabulated on the device (k_life_human,
+    // k_life_mosquito); here only what sizes them.  Mosquitoes: m_rows rows of
+    // death_m_max + 1 thresholds, row 0 floor(F_m(a) 2^24) of m_scale (the t =
+    // 0 census; every birth without a climate); with a climate, row 1 + b the
+    // running maximum over a' <= a of floor(F_m(a'; scale(b + a')) 2^24) for
+    // births on day b.
+    uint32_t death_m_max = 0;              // a death age no row's draws exceed
     uint32_t m_rows = 1;
-    std::vector<uint32_t> death_m_guide;   // [m_rows][kGuideBuckets] death age of life_bucket_kmin(b)
+    std::vector<double> scale;             // with a climate: [max_days] Weibull scale of day t
     bool climate = false;
     std::vector<float> clim;               // with a climate: [max_days][3] beta_hm, beta_mh, eip of day t
     std::vector<uint32_t> init_h;          // [kHumanYears]     initial-age year thresholds
@@ -60,8 +61,5 @@ void climate_day(const ArboClimate& c, uint32_t row, double out[4]);
 // Builds every table of one simulation.  validate() must have passed.
 void build_tables(const ArboShape& shape, const ArboParams& p, uint64_t seed,
                   uint32_t max_days, SimTables& out);
-
-// 24-bit fixed point of a probability: floor(f 2^24) clamped to [0, 2^24].
-uint32_t fixed24(double f);
 
 }  // namespace arbo

@@ -69,3 +69,43 @@ def test_age_of_infection_records_across_blocks(hip_lib, oracle_lib, grid, human
         assert np.array_equal(gpu.aoi(i), orc.aoi(i)) and np.array_equal(gpu.history(i), orc.history(i))
     gpu.close()
     orc.close()
+
+
+def test_lifetime_tables_shared_and_distinct(hip_lib, oracle_lib):
+    """A batch whose simulations share lifespans, differ in one parameter of
+    them, reach the last ages of the tables or follow climates: every table
+    the device builds is read by births, rebirths and the t = 0 census."""
+    T = 30
+    base = dict(seed_frac_h=0.02, seed_frac_m=0.02)
+    short = dict(h_scale=60.0, h_shape=1.0)       # rebirths every day
+    specs = []
+
+    def add(n, **over):
+        climate = over.pop("climate", None)
+        specs.append(SimSpec(3, 3, np.full(9, n, np.uint32), configs.base_params(**{**base, **over}), 50 + len(specs),
+                             climate=climate))
+    add(300)
+    add(300, m_scale=10.5)
+    add(200, **short)
+    add(200, **short, h_infant_scale=1e-4)
+    add(200, **short, h_loc=20.0)
+    add(150, h_scale=3500.0, h_shape=1.0)          # exponential: draws up to the last tabulated age
+    add(150, m_scale=100.0, m_shape=1.0)
+    add(120, m_scale=1.0, m_shape=0.8)             # most die within a day or two
+    add(100, climate=configs.seasonal_climate(T + 1))
+    add(100, climate=configs.seasonal_climate(T + 1, t_amp=7.0, phase=2.0, scale_mle=2.0), m_shape=4.0)
+    add(100, m_shape=4.0)
+    add(300)
+    print("[edges] lifetime tables", flush=True)
+    _both(hip_lib, oracle_lib, specs, T, checks=(0, 1, 7))
+
+
+@pytest.mark.parametrize("humans,slots", [([1, 4095, 4096], [0, 4097, 4096]), ([4097, 8193, 30], [1, 12289, 8192]),
+                                          ([65535, 1, 7], [100, 65535, 0])])
+def test_first_census_across_workgroups(hip_lib, oracle_lib, humans, slots):
+    """Communities below, at and above the members one workgroup of the t = 0
+    census takes."""
+    print(f"[edges] census {humans} {slots}", flush=True)
+    p = configs.base_params(n_serotypes=3, immunity_mode=1, seed_frac_h=0.05, seed_frac_m=0.05)
+    specs = [SimSpec(3, 1, np.array(humans, np.uint32), p, 77, mosq_slots=np.array(slots, np.uint32))]
+    _both(hip_lib, oracle_lib, specs, 3, flags=abi.F_AOI | abi.F_SPATIAL, checks=(0,))
