@@ -21,19 +21,24 @@ namespace arbo {
 
 struct U4 { uint32_t x, y, z, w; };
 
-// a ^ b ^ c, one instruction on gfx950.  The compiler keeps two v_xor_b32, 40
-// of them in each Philox block next to its 20 multiplies.
-ARBO_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+// a ^ b ^ k, k the same in every lane: one instruction on gfx950 (v_bitop3_b32,
+// truth table 0x96) with k from a scalar register.  The compiler writes two
+// v_xor_b32, 40 of them in a Philox block next to its 20 multiplies; given the
+// builtin it copies the 20 round keys to vector registers and keeps them there
+// (84 for the event kernel's 57).
+ARBO_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t k) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+    uint32_t r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x96" : "=v"(r) : "v"(a), "v"(b), "s"(k));
+    return r;
 #else
-    return a ^ b ^ c;
+    return a ^ b ^ k;
 #endif
 }
 
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers: as easy
 // as 1, 2, 3", SC'11).  Multipliers and Weyl key increments are the published
-// constants of the generator.
+// constants of the generator.  The key is the same in every lane of a wave.
 ARBO_HD U4 philox(U4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
     for (int i = 0; i < 10; ++i) {
