@@ -163,8 +163,23 @@ struct EngineView {
     uint32_t max_days;
     uint32_t death_m_lds;          // entries of the largest mosquito death table (LDS staging)
     uint32_t reduce_split;         // workgroups per simulation of k_day_reduce
+    uint32_t small;                // 1: the event kernel also sums the day's series and draws the long-distance
+                                   // events (small_batch), no k_day_reduce and k_day_longdist
     uint32_t max_words;            // alive-bitmap words of the batch's largest community
 };
+
+// Batches whose event kernel sums the series and draws the long-distance
+// events itself (EngineView.small).  Every community's wave then reads its
+// simulation's C partials and draws all its long-distance events, so C is
+// bounded, and so is what a simulation may send a day: about a tenth of
+// omega x humans at an epidemic's peak.  All waves have to run side by side
+// for the repeated work to cost only its latency: 4,096 communities are half
+// of the device's 8,192 one-wave slots.  A day of 100 communities takes 34.5
+// us with it for 40.2, of 289 (rings kept) 32 for 36.3, of 16 x 144 37.5 for
+// 42.6.
+constexpr uint32_t kSmallCommunities = 4096;
+constexpr uint32_t kSmallSimulation = 512;
+constexpr float kSmallSent = 32768.0f;
 
 // Launch knobs of the day kernels.  None of them changes a result: every
 // random draw is keyed by model entities, never by workgroup or lane.

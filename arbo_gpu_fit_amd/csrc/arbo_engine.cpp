@@ -560,6 +560,10 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         for (const SimHost& sh : e->sims) max_c = std::max(max_c, sh.C);
         const uint32_t cap = std::max<uint32_t>(1, std::min<uint32_t>(kMaxReduceSplit, 2048 / n_sims));
         v.reduce_split = std::min<uint32_t>(cap, (max_c + 255) / 256);
+        float sent = 0.0f;   // omega x humans of the simulation that may send most
+        for (uint32_t i = 0; i < n_sims; ++i)
+            sent = std::max(sent, e->sim_desc[i].omega * (float)e->sims[i].n_humans);
+        v.small = e->n_comm <= kSmallCommunities && max_c <= kSmallSimulation && sent <= kSmallSent ? 1u : 0u;
     }
 
     HIP_TRY(e, launch_init(v, std::max(max_n, max_cap), e->stream));

@@ -1160,16 +1160,69 @@ constexpr uint32_t kHumanKey = ARBO_MAX_COMMUNITY_SLOTS;   // claim keys of huma
 static_assert(ARBO_MAX_COMMUNITY_SLOTS + ARBO_MAX_COMMUNITY_HUMANS <= (1u << kKeyBits),
               "mosquito and human claim keys fit the key field");
 
+// Number of long-distance events of direction k / 4 and serotype k % 4 from
+// their summed rate (2^-24 units) or count.
+__device__ __forceinline__ uint32_t longdist_count(const SimDesc& sd, Key key, uint32_t t, uint32_t k,
+                                                   unsigned long long fx) {
+    if ((k & 3u) >= sd.S) return 0u;
+    if (sd.count_law == ARBO_COUNT_STOCH_ROUND) return (uint32_t)fx;   // the sources' own long-distance counts
+    const Stream st{key, INIT_DAY, t, ctr_tag(P_NLD, k >> 2, k & 3u, 0)};
+    return poisson((double)fx * 0x1p-24, st);
+}
+
+// Community event l of direction k / 4 and serotype k % 4 lands on.
+__device__ __forceinline__ uint32_t longdist_dest(const SimDesc& sd, Key key, uint32_t t, uint32_t k, uint32_t l) {
+    return mulhi(draw(key, l, t, ctr_tag(P_LD_DEST, k >> 2, k & 3u, 0), 0).x, sd.C);
+}
+
+// One wave sums the day's partials of a simulation into series row t + 1
+// (k_day_reduce's job, for batches that launch no k_day_reduce).
+__device__ __forceinline__ void reduce_simulation(const EngineView& v, uint32_t sim, uint32_t t, uint32_t lane) {
+    const SimDesc& sd = v.sims[sim];
+    uint32_t n[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // humans, mosquitoes, infectious[4], onsets[4], vectors
+    for (uint32_t c = lane; c < sd.C; c += kWave) {
+        const uint32_t* pw = v.part + (size_t)(sd.comm_off + c) * kPartWords;
+        const uint4 a = reinterpret_cast<const uint4*>(pw)[0];
+        const uint4 b = reinterpret_cast<const uint4*>(pw + 4)[0];
+        n[0] += a.y; n[1] += a.x;
+        n[2] += a.z & 0xFFFFu; n[3] += a.z >> 16; n[4] += a.w & 0xFFFFu; n[5] += a.w >> 16;
+        n[6] += b.x & 0xFFFFu; n[7] += b.x >> 16; n[8] += b.y & 0xFFFFu; n[9] += b.y >> 16;
+        n[10] += b.z; n[11] += b.w;
+    }
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 12; ++k) {
+        const uint32_t w = wave_sum(n[k]);
+        mine = lane == k ? w : mine;
+    }
+    const uint32_t S = sd.S, row = t + 1;
+    const SeriesIdx si = series_index(sd.series_off, v.max_days, S);
+    if (lane == 0) v.series[si.n_count + row] = mine;
+    else if (lane == 1) v.series[si.m_count + row] = mine;
+    else if (lane < 6) { if (lane - 2 < S) v.series[si.n_inf + (size_t)row * S + (lane - 2)] = mine; }
+    else if (lane < 10) { if (lane - 6 < S) v.series[si.n_inc + (size_t)row * S + (lane - 6)] = mine; }
+    else if (lane < 12) v.scanned[2 * (size_t)sim + (lane - 10)] += mine;
+}
+
 // MW: bitmap words of a community in units of kWaveWords (1, or kMaxWaves
 // for batches with communities above 8,192 slots): the alive-rank index is
 // built in MW passes of four words per lane.
-template <bool XCD, bool HIST, uint32_t MW>
+// SMALL: the day has no k_day_reduce and no k_day_longdist, 5 us of a launch
+// each where a day of 100 communities takes 30: every community's wave sums
+// its simulation's long-distance rates and draws all of its events' landing
+// places itself, keeping those that land here, and one more workgroup per
+// simulation sums the series row beside them (kSmallCommunities).
+template <bool XCD, bool HIST, uint32_t MW, bool SMALL>
 __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
     const uint32_t g = XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x, lane = threadIdx.x;
     const uint32_t t = *v.day + v.day_offset;
+    if (SMALL && g >= v.n_comm) {
+        reduce_simulation(v, g - v.n_comm, t, lane);
+        return;
+    }
     const CommDesc cd = v.comm[g];
     const uint32_t act = v.active[g];
-    if (!act && !(cd.flags & kCommIntro)) return;   // no events arrive and no introductions
+    if (!SMALL && !act && !(cd.flags & kCommIntro)) return;   // no events arrive and no introductions
     if (act && lane == 0) v.active[g] = 0u;         // consumed
     const SimDesc sd = v.sims[cd.sim];
     const Key key{sd.k0, sd.k1};
@@ -1194,7 +1247,37 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
         s_slot[lane] = v.in_slot[cd.in_off + lane];
     }
     uint32_t tot_dir[2] = {0, 0};
-    if (lane < 8) {  // long-distance arrivals of the day, consumed
+    if (SMALL) {
+        // lane 8 q + k sums rate k over every eighth community from q
+        const unsigned long long* rate =
+            reinterpret_cast<const unsigned long long*>(v.part + (size_t)sd.comm_off * kPartWords + 8) + (lane & 7u);
+        unsigned long long fx = 0;
+#pragma unroll 4
+        for (uint32_t c = lane >> 3; c < sd.C; c += 8) fx += rate[(size_t)c * (kPartWords / 2)];
+#pragma unroll
+        for (uint32_t d = 8; d < kWave; d <<= 1) fx += __shfl_xor(fx, d, kWave);
+        uint32_t L = 0;
+        if (lane < 8) {
+            s_nld[lane] = 0u;
+            L = longdist_count(sd, key, t, lane, fx);
+        }
+        uint32_t pre[9];
+        pre[0] = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) pre[k + 1] = pre[k] + (uint32_t)__builtin_amdgcn_readlane((int)L, (int)k);
+        __syncthreads();
+        for (uint32_t l = lane; l < pre[8]; l += kWave) {
+            uint32_t k = 0, first = 0;
+#pragma unroll
+            for (uint32_t q = 1; q < 8; ++q) {
+                k += (l >= pre[q]) ? 1u : 0u;
+                first = l >= pre[q] ? pre[q] : first;
+            }
+            if (longdist_dest(sd, key, t, k, l - first) == cd.c) atomicAdd(&s_nld[k], 1u);
+        }
+        __syncthreads();
+        if (lane < 8) tot_dir[lane >> 2] += s_nld[lane];
+    } else if (lane < 8) {  // long-distance arrivals of the day, consumed
         const uint32_t n = v.nld[(size_t)g * 8 + lane];
         s_nld[lane] = n;
         if (n) v.nld[(size_t)g * 8 + lane] = 0;
@@ -1448,17 +1531,8 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
     const Key key{sd.k0, sd.k1};
     __shared__ uint32_t s_L[8];
     if (tid < 8) {
-        const uint32_t dir = tid >> 2, s = tid & 3u;
-        uint32_t L = 0;
-        if (s < sd.S) {
-            const unsigned long long fx = v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + tid];   // summed by k_day_reduce
-            if (sd.count_law == ARBO_COUNT_STOCH_ROUND) {
-                L = (uint32_t)fx;   // the sources' own long-distance counts
-            } else {
-                const Stream st{key, INIT_DAY, t, ctr_tag(P_NLD, dir, s, 0)};
-                L = poisson((double)fx * 0x1p-24, st);
-            }
-        }
+        const unsigned long long fx = v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + tid];   // summed by k_day_reduce
+        const uint32_t L = longdist_count(sd, key, t, tid, fx);
         s_L[tid] = L;
     }
     __syncthreads();
@@ -1470,8 +1544,7 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
         uint32_t k = 0;
 #pragma unroll
         for (uint32_t q = 1; q < 8; ++q) k += (l >= pre[q]) ? 1u : 0u;
-        const uint32_t idx = l - pre[k];
-        const uint32_t d = mulhi(draw(key, idx, t, ctr_tag(P_LD_DEST, k >> 2, k & 3u, 0), 0).x, sd.C);
+        const uint32_t d = longdist_dest(sd, key, t, k, l - pre[k]);
         atomicAdd(&v.nld[(size_t)(sd.comm_off + d) * 8 + k], 1u);
         v.active[sd.comm_off + d] = 1u;
     }
@@ -1764,23 +1837,30 @@ hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t 
     return (tu.xcd & 1u) ? launch_demography_x<true>(v, tu, st) : launch_demography_x<false>(v, tu, st);
 }
 
-hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st) {
-    const dim3 grid(v.n_comm), block(kWave);
+template <bool HIST>
+static void launch_events_h(const EngineView& v, const Tuning& tu, hipStream_t st) {
+    const dim3 grid(v.n_comm + (v.small ? v.n_sims : 0u)), block(kWave);
     if (v.max_words > kWaveWords) {   // communities above 8,192 slots
-        if (v.hist) hipLaunchKernelGGL((k_day_events<false, true, kMaxWaves>), grid, block, 0, st, v);
-        else hipLaunchKernelGGL((k_day_events<false, false, kMaxWaves>), grid, block, 0, st, v);
+        if (v.small) hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, true>), grid, block, 0, st, v);
+        else hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, false>), grid, block, 0, st, v);
+    } else if (v.small) {
+        hipLaunchKernelGGL((k_day_events<false, HIST, 1, true>), grid, block, 0, st, v);
     } else if (tu.xcd & 2u) {
-        if (v.hist) hipLaunchKernelGGL((k_day_events<true, true, 1>), grid, block, 0, st, v);
-        else hipLaunchKernelGGL((k_day_events<true, false, 1>), grid, block, 0, st, v);
+        hipLaunchKernelGGL((k_day_events<true, HIST, 1, false>), grid, block, 0, st, v);
     } else {
-        if (v.hist) hipLaunchKernelGGL((k_day_events<false, true, 1>), grid, block, 0, st, v);
-        else hipLaunchKernelGGL((k_day_events<false, false, 1>), grid, block, 0, st, v);
+        hipLaunchKernelGGL((k_day_events<false, HIST, 1, false>), grid, block, 0, st, v);
     }
-    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, grid, block, 0, st, v);
+}
+
+hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st) {
+    if (v.hist) launch_events_h<true>(v, tu, st);
+    else launch_events_h<false>(v, tu, st);
+    if (v.aoi_mark) hipLaunchKernelGGL(k_day_aoi, dim3(v.n_comm), dim3(kWave), 0, st, v);
     return hipGetLastError();
 }
 
 hipError_t launch_longdist(const EngineView& v, const Tuning& tu, hipStream_t st) {
+    if (v.small) return hipSuccess;   // the event kernel does both
     hipLaunchKernelGGL(k_day_reduce, dim3(v.n_sims * v.reduce_split), dim3(256), 0, st, v, v.reduce_split);
     hipLaunchKernelGGL(k_day_longdist, dim3(v.n_sims * tu.ld_split), dim3(256), 0, st, v, tu.ld_split);
     return hipGetLastError();
