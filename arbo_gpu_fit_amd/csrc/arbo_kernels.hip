@@ -1376,30 +1376,38 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
                                            s_rot[dir], S, dir, s_src, s_slot, cd.c);
                 const U4 r = draw(key, q.x0, t, q.x2, q.j);
                 const uint32_t w4[4] = {r.x, r.y, r.z, r.w};
+                // The four targets' words are requested together, before any
+                // claim: one after another, each load waited for the claim
+                // of the event before it.  Events past the quad's last read
+                // its first one's target and claim nothing.
+                uint32_t tgt[4], tw[4];
+                if (hum) {
 #pragma unroll
-                for (uint32_t e = 0; e < 4; ++e) {
-                    if (e >= q.count) break;
-                    const uint32_t rank = 4 * (u * kWave + lane) + e;
-                    if (hum) {
-                        const uint32_t h = mulhi(w4[e], N);
-                        const uint32_t w = v.h_word[cd.h_off + h];
-                        if ((w & 3u) == 0 && !((w >> (4 + q.s)) & 1u)) {
-                            claim(s_tab, kHumanKey + h, rank);
-                            cache[4 * u + e] = kEligible | (q.s << kKeyBits) | (kHumanKey + h);
-                            word[4 * u + e] = w;
-                        }
-                    } else {
-                        const uint32_t rk = mulhi(w4[e], Md);   // alive rank of the target
+                    for (uint32_t e = 0; e < 4; ++e) tgt[e] = mulhi(w4[e], N);
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) tw[e] = v.h_word[cd.h_off + (e < q.count ? tgt[e] : tgt[0])];
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) tgt[e] += kHumanKey;
+                } else {
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) {
+                        const uint32_t rk = mulhi(w4[e < q.count ? e : 0u], Md);   // alive rank of the target
                         uint32_t w = s_sel[rk >> 5];
                         while (w + 1 < nwords && s_wpre[w + 1] <= rk) ++w;
-                        const uint32_t slot = 32u * w + select_in_word(s_word[w], rk - s_wpre[w]);
-                        const uint32_t mw = v.m_word[cd.m_off + slot];
-                        if ((mw & 3u) == 0) {
-                            claim(s_tab, slot, rank);
-                            cache[4 * u + e] = kEligible | (q.s << kKeyBits) | slot;
-                            word[4 * u + e] = mw;
-                        }
+                        tgt[e] = 32u * w + select_in_word(s_word[w], rk - s_wpre[w]);
                     }
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; ++e) tw[e] = v.m_word[cd.m_off + tgt[e]];
+                }
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e) {
+                    // a human: susceptible and never infected by s; a mosquito: susceptible (no immunity bits)
+                    const bool ok = e < q.count && (tw[e] & 3u) == 0 && !(hum && ((tw[e] >> (4 + q.s)) & 1u));
+                    if (ok) {
+                        claim(s_tab, tgt[e], 4 * (u * kWave + lane) + e);
+                        cache[4 * u + e] = kEligible | (q.s << kKeyBits) | tgt[e];
+                    }
+                    word[4 * u + e] = tw[e];
                 }
             }
             __syncthreads();
