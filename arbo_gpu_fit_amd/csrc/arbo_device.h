@@ -23,16 +23,21 @@ constexpr uint32_t kHumanAlign = 4;       // humans per 16-byte vector
 constexpr uint32_t kMosqAlign = 128;      // mosquito slots per 16-byte group of alive-bitmap words
 constexpr uint32_t kAoiRecord = 5000;     // ages per age-of-infection ring
 // Per-community partials of a day, written by the demography kernel and
-// summed per simulation by k_day_reduce: word 0 mosquitoes alive after the
+// summed per simulation by k_day_counts: word 0 mosquitoes alive after the
 // births, 1 humans, 2-3 infectious humans (two 16-bit serotype pairs), 4-5
 // E->I onsets (pairs), 6-7 the 16-byte census vectors of humans and of
-// mosquitoes the day's scan read, 8-23 the eight long-distance rates or
-// counts (u64).
+// mosquitoes the day's scan read, 8-9 infectious mosquitoes (pairs); in small
+// batches 8-23 the eight long-distance rates or counts (u64) instead.
 constexpr uint32_t kPartWords = 24;
-constexpr uint32_t kMaxReduceSplit = 64;  // workgroups per simulation of k_day_reduce: about one
-                                          // community per thread, 1..64, about 2,048 in all
+constexpr uint32_t kCountComms = 32;      // communities of a workgroup of k_day_counts
 constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this
+
+// A workgroup of k_day_counts: n communities of one simulation from community
+// c0, global index `first`, whose CSR rows are entries [row, row + rows).
+struct CountBlock {
+    uint32_t sim, c0, first, n, row, rows;
+};
 
 struct CommDesc {
     uint64_t h_off;       // global offset of the first human
@@ -137,7 +142,7 @@ struct EngineView {
     uint32_t* series;
     uint32_t* part;                // [G][kPartWords] per-community partials of the day (see kPartWords)
     unsigned long long* scanned;   // [n_sims][2] census vectors read by the demography kernel (humans,
-                                   // mosquitoes), summed over days by k_day_reduce
+                                   // mosquitoes), summed over days by k_day_counts
     uint32_t* spatial;             // per-community infectious humans [(T+1)][S][C] per simulation, or null
     int32_t* hist;                 // per human 4 infection-history words (one per serotype), or null
     uint8_t* aoi_mark;             // per human: 1 + ring when a mosquito event infected it today
@@ -162,9 +167,11 @@ struct EngineView {
     uint32_t n_comm;
     uint32_t max_days;
     uint32_t death_m_lds;          // entries of the largest mosquito death table (LDS staging)
-    uint32_t reduce_split;         // workgroups per simulation of k_day_reduce
+    const CountBlock* count_map;   // [count_blocks]
+    uint32_t count_blocks;
     uint32_t small;                // 1: the event kernel also sums the day's series and draws the long-distance
-                                   // events (small_batch), no k_day_reduce and k_day_longdist
+                                   // events (kSmallCommunities), the demography kernel the local ones: no
+                                   // k_day_counts and k_day_longdist
     uint32_t max_words;            // alive-bitmap words of the batch's largest community
 };
 

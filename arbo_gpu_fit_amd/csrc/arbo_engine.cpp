@@ -63,6 +63,7 @@ struct ArboEngine {
     DevBuf<int32_t> h_birth, hist;
     DevBuf<uint8_t> aoi_mark;
     DevBuf<uint32_t> aoi, aoi_pos, aoi_cnt, aoi_sum;
+    DevBuf<CountBlock> count_map;
     DevBuf<unsigned long long> lam, scanned;
     DevBuf<uint32_t> part;   // per-community partials of the day
     DevBuf<float> dens;
@@ -131,7 +132,7 @@ void free_batch(ArboEngine* e) {
     dev_free(e->comm); dev_free(e->simd);
     dev_free(e->h_word); dev_free(e->alive); dev_free(e->cnt); dev_free(e->nld); dev_free(e->active); dev_free(e->hsum); dev_free(e->series); dev_free(e->spatial); dev_free(e->csr_thr); dev_free(e->csr_inbox);
     dev_free(e->in_edge); dev_free(e->in_slot); dev_free(e->tables); dev_free(e->day_ctr);
-    dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum);
+    dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum); dev_free(e->count_map);
     dev_free(e->lam); dev_free(e->scanned); dev_free(e->dens); dev_free(e->part);
     dev_free(e->scales); dev_free(e->life_h); dev_free(e->life_m);
     e->ready = false;
@@ -304,6 +305,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     e->sim_desc.assign(n_sims, SimDesc());
     std::vector<CommDesc> comm;
     std::vector<uint32_t> csr_thr, csr_inbox, in_edge, in_slot, table_pool;
+    std::vector<CountBlock> count_map;
     std::vector<float> dens_pool;
     // lifetime tables, built on the device behind the uploaded ones: one per
     // distinct set of parameters
@@ -431,6 +433,10 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
             max_n = std::max(max_n, cd.n);
             max_cap = std::max(max_cap, cd.cap);
         }
+        for (uint32_t c = 0; c < t.C; c += kCountComms) {
+            const uint32_t n = std::min(kCountComms, t.C - c), row = row_base + t.row_ptr[c];
+            count_map.push_back(CountBlock{i, c, sh.comm_off + c, n, row, t.row_ptr[c + n] - t.row_ptr[c]});
+        }
         sd.aoi_block = aoi_blocks;
         sd.aoi_blocks = (t.C + kAoiBlock - 1) / kAoiBlock;
         aoi_blocks += sd.aoi_blocks;
@@ -475,7 +481,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         (rc = dev_alloc(e, e->hsum, comm.size() * 4)) || (rc = dev_alloc(e, e->active, comm.size())) ||
         (rc = dev_alloc(e, e->lam, (size_t)2 * n_sims * 8)) || (rc = dev_alloc(e, e->scanned, (size_t)2 * n_sims)) || (rc = dev_alloc(e, e->part, comm.size() * kPartWords)) || (rc = dev_alloc(e, e->series, ser_tot)) || (rc = dev_alloc(e, e->spatial, spa_tot)) ||
         (rc = dev_alloc(e, e->csr_thr, csr_thr.size())) || (rc = dev_alloc(e, e->csr_inbox, csr_inbox.size())) || (rc = dev_alloc(e, e->in_edge, in_edge.size())) ||
-        (rc = dev_alloc(e, e->in_slot, in_slot.size())) || (rc = dev_alloc(e, e->tables, pool_words)) || (rc = dev_alloc(e, e->scales, scales.size())) ||
+        (rc = dev_alloc(e, e->in_slot, in_slot.size())) || (rc = dev_alloc(e, e->tables, pool_words)) || (rc = dev_alloc(e, e->count_map, count_map.size())) || (rc = dev_alloc(e, e->scales, scales.size())) ||
         (rc = dev_alloc(e, e->life_h, life_h.size())) || (rc = dev_alloc(e, e->life_m, life_m.size())) ||
         (rc = dev_alloc(e, e->dens, dens_pool.size())) || (rc = dev_alloc(e, e->day_ctr, 1))) {
         free_batch(e);
@@ -489,6 +495,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     HIP_TRY(e, hipMemcpy(e->in_slot.p, in_slot.data(), in_slot.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->tables.p, table_pool.data(), table_pool.size() * 4, hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->dens.p, dens_pool.data(), dens_pool.size() * 4, hipMemcpyHostToDevice));
+    HIP_TRY(e, hipMemcpy(e->count_map.p, count_map.data(), count_map.size() * sizeof(CountBlock), hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->life_h.p, life_h.data(), life_h.size() * sizeof(HumanTable), hipMemcpyHostToDevice));
     HIP_TRY(e, hipMemcpy(e->life_m.p, life_m.data(), life_m.size() * sizeof(MosquitoTable), hipMemcpyHostToDevice));
     if (!scales.empty()) HIP_TRY(e, hipMemcpy(e->scales.p, scales.data(), scales.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -541,6 +548,8 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     v.aoi_cnt = e->aoi_cnt.p;
     v.aoi_sum = e->aoi_sum.p;
     v.aoi_nblocks = aoi_blocks;
+    v.count_map = e->count_map.p;
+    v.count_blocks = (uint32_t)count_map.size();
     v.aoi_from = max_days > kAoiWindow ? max_days - kAoiWindow : 0u;
     v.csr_inbox = e->csr_inbox.p;
     v.csr_thr = e->csr_thr.p;
@@ -554,12 +563,9 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     v.max_days = max_days;
     v.death_m_lds = death_m_lds;
     v.max_words = (max_cap + 31) >> 5;   // above 256 the day kernels take their eight-wave forms
-    {   // about one community per thread of k_day_reduce, at most kMaxReduceSplit workgroups per
-        // simulation and about 2,048 in all (8 per CU)
+    {
         uint32_t max_c = 1;
         for (const SimHost& sh : e->sims) max_c = std::max(max_c, sh.C);
-        const uint32_t cap = std::max<uint32_t>(1, std::min<uint32_t>(kMaxReduceSplit, 2048 / n_sims));
-        v.reduce_split = std::min<uint32_t>(cap, (max_c + 255) / 256);
         float sent = 0.0f;   // omega x humans of the simulation that may send most
         for (uint32_t i = 0; i < n_sims; ++i)
             sent = std::max(sent, e->sim_desc[i].omega * (float)e->sims[i].n_humans);

@@ -15,10 +15,14 @@
 //     per serotype with wave reductions, fills the lowest-index dead mosquito
 //     slots up to the seasonal target with a wave prefix scan over the
 //     dead-slot bitmap (newborn lifetimes from an LDS copy of the mosquito
-//     lifetime table), publishes the alive-slot bitmap, draws the Poisson
-//     event counts of the community as a source, spreads the local events
-//     over its CSR row with the alias table into an LDS histogram, and adds
-//     its counters into the series row of the next day.
+//     lifetime table), publishes the alive-slot bitmap and leaves its counters
+//     as the community's partials of the day.
+//
+//  k_day_counts      (nepidemic.cu:49-136)
+//     draws the Poisson event counts of the communities as sources, spreads
+//     the local events over their CSR rows with the alias tables into LDS
+//     histograms and adds the partials into the series row of the next day
+//     (small batches: in the demography and event kernels).
 //
 //  k_day_events      mepidemic.cu:143-246 (nmTransmission) +
 //                    nepidemic.cu:146-319 (mnTransmission)
@@ -486,6 +490,63 @@ __device__ __forceinline__ uint32_t human_states(const EngineView& v, const Comm
     return ons;
 }
 
+// Events of a community as a source in direction k / 4 and of serotype k % 4
+// (nepidemic.cu:49-136): n dispersed locally, `stay` that stay, and the
+// long-distance rate (2^-24 units) or count.
+struct SourceCount {
+    uint32_t n, stay;
+    unsigned long long fx;
+};
+__device__ __forceinline__ SourceCount source_count(const SimDesc& sd, const float* dens, Key key, uint32_t c,
+                                                    uint32_t flags, uint32_t t, uint32_t k, uint32_t I, uint32_t Mc,
+                                                    uint32_t humans) {
+    SourceCount o{0u, 0u, 0ull};
+    const uint32_t dir = k >> 2, s = k & 3u;
+    if (s >= sd.S || I == 0) return o;
+    const DayParams dp = day_params(sd, dens, t);
+    const float lam = dir == DIR_HM ? (float)Mc / (float)humans * dp.beta_hm * (float)I : dp.beta_mh * (float)I;
+    const bool staying = (flags & kCommStay) != 0;
+    if (sd.count_law == ARBO_COUNT_STOCH_ROUND) {   // nepidemic.cu:67-104
+        const U4 r = draw(key, c, t, ctr_tag(P_NSR, dir, s, 0), 0);
+        uint32_t all = stoch_round(lam, r.x);
+        if (staying) o.stay = stoch_round((float)all * sd.no_distance, r.y);
+        all -= o.stay;
+        const uint32_t ld = stoch_round((float)all * sd.omega, r.z);
+        o.n = all - ld;
+        o.fx = ld;   // an event count: the long-distance kernel sends exactly these
+    } else {
+        const float go = staying ? lam * (1.0f - sd.no_distance) : lam;
+        const float mu_loc = go * (1.0f - sd.omega);
+        const float mu_ld = go * sd.omega;
+        o.fx = (unsigned long long)floor((double)mu_ld * 16777216.0);
+        const Stream st{key, c, t, ctr_tag(P_NLOC, dir, s, 0)};
+        o.n = poisson((double)mu_loc, st);
+        if (staying) {
+            const Stream ss{key, c, t, ctr_tag(P_NSTAY, dir, s, 0)};
+            o.stay = poisson((double)(lam * sd.no_distance), ss);
+        }
+    }
+    return o;
+}
+
+// Destination columns of events 4 j .. 4 j + 3 of segment k's n, counted in
+// hist: the product word * row length gives the column (high half) and the
+// alias test's uniform (low half).
+__device__ __forceinline__ void spread_quad(Key key, uint32_t c, uint32_t t, uint32_t k, uint32_t j, uint32_t n,
+                                            const uint32_t* row, uint32_t rl, uint32_t* hist) {
+    const U4 r = draw(key, c, t, ctr_tag(P_DEST, k >> 2, k & 3u, 0), j);
+    const uint32_t w4[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+        if (4 * j + e >= n) break;
+        const uint64_t prod = (uint64_t)w4[e] * rl;
+        uint32_t col = (uint32_t)(prod >> 32);
+        const uint32_t en = row[col];
+        if ((((uint32_t)prod) >> 8) >= (en & 0x1FFFFFFu)) col = en >> 27;
+        atomicAdd(&hist[col], 1u);
+    }
+}
+
 // Queue of the wave's deferred human changes (in LDS): entry k holds the
 // member index (bits 0-15) and, for an onset, its E -> I day (bits 16-31) in
 // qi[k], the member's word in qw[k].  A death is told from an onset by the
@@ -531,7 +592,8 @@ __device__ __forceinline__ void human_deferred(const EngineView& v, const CommDe
 // and the counts, the dead-slot prefix and the high-water mark are combined
 // across the waves through LDS; a community may hold up to NW times
 // kWaveWords bitmap words of slots (four per thread).
-template <uint32_t UNROLL, uint32_t EARLY_M, bool XCD, bool HIST, uint32_t WPS, uint32_t NW>
+// SMALL: a small batch (EngineView.small), whose event counts are drawn here.
+template <uint32_t UNROLL, uint32_t EARLY_M, bool XCD, bool HIST, uint32_t WPS, uint32_t NW, bool SMALL = false>
 __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(WPS ? WPS : 1)))
 void k_day_demography(EngineView v) {
     static_assert(EARLY_M >= 1 && EARLY_M <= UNROLL, "early mosquito batch within the first unrolled batch");
@@ -624,9 +686,14 @@ void k_day_demography(EngineView v) {
             if (b < kLifeBuckets) s_mguide[b] = gv[k];
         }
     }
-    if (tid < cd.row_len) s_row[tid] = v.csr_thr[cd.row_off + tid];
-    const uint32_t inboxent = tid < cd.row_len ? v.csr_inbox[cd.row_off + tid] : 0u;
-    for (uint32_t i = tid; i < kCntPerComm; i += NT) s_hist[i] = 0;
+    uint32_t inboxent = 0u;
+    if (SMALL) {
+        if (tid < cd.row_len) {
+            s_row[tid] = v.csr_thr[cd.row_off + tid];
+            inboxent = v.csr_inbox[cd.row_off + tid];
+        }
+        for (uint32_t i = tid; i < kCntPerComm; i += NT) s_hist[i] = 0;
+    }
     // emergence target of the day: the next day's expected population E[t+1]
     // (simulation.cpp:129-132), drawn once the census is counted
     const float dens_next = v.dens[sd.dens_off + t + 1];
@@ -983,87 +1050,47 @@ void k_day_demography(EngineView v) {
         reinterpret_cast<uint4*>(v.hsum)[g] = make_uint4(minev, ih01, ih23, ((top + 7) >> 3) + 1u);
     const uint32_t Mc = alive_c + births;
 
-    // ---- event counts of this community as a source (nepidemic.cu:49-136) ----
-    if (tid < 8) {
-        const uint32_t dir = tid >> 2, s = tid & 3u;
-        uint32_t n = 0;
-        unsigned long long fx = 0;
-        if (s < S) {
+    // ---- event counts of this community as a source ----
+    // Small batches draw and spread them here, others in k_day_counts.
+    if (SMALL) {
+        if (tid < 8) {
+            const uint32_t dir = tid >> 2, s = tid & 3u;
             const uint32_t I = dir == DIR_HM ? unpack_pair(ih01, ih23, s) : unpack_pair(im01, im23, s);
-            if (I > 0) {
-                const DayParams dp = day_params(sd, v.dens, t);
-                const float lam = dir == DIR_HM ? (float)Mc / (float)cd.n * dp.beta_hm * (float)I
-                                                : dp.beta_mh * (float)I;
-                const bool staying = (cd.flags & kCommStay) != 0;
-                uint32_t stay = 0;
-                if (sd.count_law == ARBO_COUNT_STOCH_ROUND) {   // nepidemic.cu:67-104
-                    const U4 r = draw(key, cd.c, t, ctr_tag(P_NSR, dir, s, 0), 0);
-                    uint32_t all = stoch_round(lam, r.x);
-                    if (staying) stay = stoch_round((float)all * sd.no_distance, r.y);
-                    all -= stay;
-                    const uint32_t ld = stoch_round((float)all * sd.omega, r.z);
-                    n = all - ld;
-                    fx = ld;   // an event count: the long-distance kernel sends exactly these
-                } else {
-                    const float go = staying ? lam * (1.0f - sd.no_distance) : lam;
-                    const float mu_loc = go * (1.0f - sd.omega);
-                    const float mu_ld = go * sd.omega;
-                    fx = (unsigned long long)floor((double)mu_ld * 16777216.0);
-                    const Stream st{key, cd.c, t, ctr_tag(P_NLOC, dir, s, 0)};
-                    n = poisson((double)mu_loc, st);
-                    if (staying) {
-                        const Stream ss{key, cd.c, t, ctr_tag(P_NSTAY, dir, s, 0)};
-                        stay = poisson((double)(lam * sd.no_distance), ss);
-                    }
-                }
-                // staying events join the count of the source's own column
-                if (stay) atomicAdd(&s_hist[tid * 9 + ((cd.flags >> kCommSelfShift) & 15u)], stay);
+            const SourceCount sc = source_count(sd, v.dens, key, cd.c, cd.flags, t, tid, I, Mc, cd.n);
+            // staying events join the count of the source's own column
+            if (sc.stay) atomicAdd(&s_hist[tid * 9 + ((cd.flags >> kCommSelfShift) & 15u)], sc.stay);
+            s_n[tid] = sc.n;
+            // read by every community of the simulation (no same-address atomics)
+            reinterpret_cast<unsigned long long*>(v.part + (size_t)g * kPartWords + 8)[tid] = sc.fx;
+        }
+        __syncthreads();
+        // Destinations: event i of source segment k takes word i%4 of Philox
+        // block i/4 (one block per lane and quad of events).
+        const uint32_t rl = cd.row_len;
+        uint32_t qtot = 0;   // quads of the 8 segments (the segment of a quad is found by walking s_n)
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) qtot += (s_n[k] + 3) >> 2;
+        for (uint32_t gq = tid; gq < qtot; gq += NT) {
+            uint32_t k = 0, base = 0, nq = (s_n[0] + 3) >> 2;
+            while (gq >= base + nq) {   // ends: gq < qtot
+                base += nq;
+                nq = (s_n[++k] + 3) >> 2;
+            }
+            spread_quad(key, cd.c, t, k, gq - base, s_n[k], s_row, rl, s_hist + k * 9);
+        }
+        __syncthreads();
+        // push the counts into each destination's inbox: 8 contiguous words per (destination, in-edge)
+        for (uint32_t i0 = 0; wv == 0 && i0 < 8 * rl; i0 += kWave) {   // wave 0, every lane shuffles
+            const uint32_t i = i0 + lane, col = i >> 3, k = i & 7u;
+            const uint32_t dst = __shfl(inboxent, col < rl ? col : 0u, kWave);
+            if (i < 8 * rl) {
+                const uint32_t n = s_hist[k * 9 + col];
+                v.cnt[(size_t)dst * 8 + k] = n;
+                if (n) v.active[dst / kInboxEdges] = 1u;   // the destination has events today
             }
         }
-        s_n[tid] = n;
-        // summed over the simulation by k_day_reduce (no same-address atomics
-        // across the simulation's communities)
-        reinterpret_cast<unsigned long long*>(v.part + (size_t)g * kPartWords + 8)[tid] = fx;
-    }
-    __syncthreads();
-    // Destinations: event i of source segment k takes word i%4 of Philox
-    // block i/4 (one block per lane and quad of events); the product
-    // word * row length gives the column (high half) and the alias test
-    // uniform (low half).
-    const uint32_t rl = cd.row_len;
-    uint32_t qtot = 0;   // quads of the 8 segments (the segment of a quad is found by walking s_n)
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) qtot += (s_n[k] + 3) >> 2;
-    for (uint32_t gq = tid; gq < qtot; gq += NT) {
-        uint32_t k = 0, base = 0, nq = (s_n[0] + 3) >> 2;
-        while (gq >= base + nq) {   // ends: gq < qtot
-            base += nq;
-            nq = (s_n[++k] + 3) >> 2;
-        }
-        const uint32_t j = gq - base;
-        const uint32_t n = s_n[k];
-        const U4 r = draw(key, cd.c, t, ctr_tag(P_DEST, k >> 2, k & 3u, 0), j);
-        const uint32_t w4[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-        for (uint32_t e = 0; e < 4; ++e) {
-            if (4 * j + e >= n) break;
-            const uint64_t prod = (uint64_t)w4[e] * rl;
-            uint32_t col = (uint32_t)(prod >> 32);
-            const uint32_t en = s_row[col];
-            if ((((uint32_t)prod) >> 8) >= (en & 0x1FFFFFFu)) col = en >> 27;
-            atomicAdd(&s_hist[k * 9 + col], 1u);
-        }
-    }
-    __syncthreads();
-    // push the counts into each destination's inbox: 8 contiguous words per (destination, in-edge)
-    for (uint32_t i0 = 0; wv == 0 && i0 < 8 * rl; i0 += kWave) {   // wave 0, every lane shuffles
-        const uint32_t i = i0 + lane, col = i >> 3, k = i & 7u;
-        const uint32_t dst = __shfl(inboxent, col < rl ? col : 0u, kWave);
-        if (i < 8 * rl) {
-            const uint32_t n = s_hist[k * 9 + col];
-            v.cnt[(size_t)dst * 8 + k] = n;
-            if (n) v.active[dst / kInboxEdges] = 1u;   // the destination has events today
-        }
+    } else if (tid == 2) {
+        reinterpret_cast<uint2*>(v.part + (size_t)g * kPartWords + 8)[0] = make_uint2(im01, im23);
     }
 
     // ---- series row t+1 (datacollect.cu:79-189): this community's part ----
@@ -1176,7 +1203,7 @@ __device__ __forceinline__ uint32_t longdist_dest(const SimDesc& sd, Key key, ui
 }
 
 // One wave sums the day's partials of a simulation into series row t + 1
-// (k_day_reduce's job, for batches that launch no k_day_reduce).
+// (for batches without k_day_counts).
 __device__ __forceinline__ void reduce_simulation(const EngineView& v, uint32_t sim, uint32_t t, uint32_t lane) {
     const SimDesc& sd = v.sims[sim];
     uint32_t n[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // humans, mosquitoes, infectious[4], onsets[4], vectors
@@ -1207,7 +1234,7 @@ __device__ __forceinline__ void reduce_simulation(const EngineView& v, uint32_t 
 // MW: bitmap words of a community in units of kWaveWords (1, or kMaxWaves
 // for batches with communities above 8,192 slots): the alive-rank index is
 // built in MW passes of four words per lane.
-// SMALL: the day has no k_day_reduce and no k_day_longdist, 5 us of a launch
+// SMALL: the day has no k_day_counts and no k_day_longdist, 5 us of a launch
 // each where a day of 100 communities takes 30: every community's wave sums
 // its simulation's long-distance rates and draws all of its events' landing
 // places itself, keeping those that land here, and one more workgroup per
@@ -1539,7 +1566,7 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
     const Key key{sd.k0, sd.k1};
     __shared__ uint32_t s_L[8];
     if (tid < 8) {
-        const unsigned long long fx = v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + tid];   // summed by k_day_reduce
+        const unsigned long long fx = v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + tid];   // summed by k_day_counts
         const uint32_t L = longdist_count(sd, key, t, tid, fx);
         s_L[tid] = L;
     }
@@ -1566,78 +1593,153 @@ __global__ __launch_bounds__(256) void k_day_longdist(EngineView v, uint32_t spl
     longdist_part(v, sim, *v.day + v.day_offset, part, split, threadIdx.x);
 }
 
-// Sums the day's per-community partials of a simulation: `split`
-// workgroups of 256 threads (about one community per thread, at most 64
-// per simulation and about 2,048 in all) each take a share of its
-// communities and add
-// their sums to the series row t + 1 (datacollect.cu:79-189, zero until
-// then) and to the long-distance totals the long-distance kernel reads
-// (zeroed by the previous day's long-distance kernel), `split` integer
-// atomics per word, so the order does not matter.
-__global__ __launch_bounds__(256) void k_day_reduce(EngineView v, uint32_t split) {
-    const uint32_t sim = blockIdx.x / split, part = blockIdx.x % split;
+// The communities of a day as sources, kCountComms of one simulation a
+// workgroup, and the sums of their partials.  Eight lanes a community draw its
+// event counts (direction and serotype each), the workgroup spreads all its
+// events' quads over its threads and pushes the counts into the destinations'
+// inboxes; integer atomics add the workgroup's sums to the series row t + 1
+// (datacollect.cu:79-189, zero until then) and to the long-distance totals
+// (zeroed by the previous day's long-distance kernel).
+// Why here: the demography kernel issues a vector instruction on 9 of 10
+// cycles during an epidemic, and the counts took it 500 of 2,400 a wave with
+// 8 of 64 lanes (the Poisson draws in double) or a few quads' lanes at work.
+// Here 8 communities share those instructions.
+__global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
+    constexpr uint32_t kSeg = 8 * kCountComms;   // a segment (community, direction, serotype) a thread
+    constexpr uint32_t kRows = kMaxRowLen * kCountComms;
+    static_assert(kSeg == 256 && kRows <= 2 * 256, "one segment, at most two CSR entries per thread");
+    const CountBlock cb = v.count_map[blockIdx.x];
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    const uint32_t j = tid >> 3, k = tid & 7u;
+    __shared__ uint32_t s_hist[kCountComms][kCntPerComm];
+    __shared__ uint32_t s_row[kRows], s_box[kRows];   // the communities' CSR rows, one behind the other
+    __shared__ uint8_t s_own[kRows];                  // community of each entry
+    __shared__ uint32_t s_off[kCountComms], s_rl[kCountComms];
+    __shared__ uint32_t s_n[kSeg], s_q[kSeg];         // events and first quad of each segment
+    __shared__ uint32_t s_wt[4];
+    __shared__ uint32_t s_cnt[4][12];                 // per wave: humans, mosquitoes, infectious[4], onsets[4], vectors
+    __shared__ unsigned long long s_fx[4][8];
+    // everything the block's descriptor leads to is requested at once
+    const bool in = j < cb.n;
+    const uint32_t g = cb.first + (in ? j : 0u);
+    const uint32_t* pw = v.part + (size_t)g * kPartWords;
+    const uint4 pa = reinterpret_cast<const uint4*>(pw)[0];        // mosquitoes, humans, infectious humans
+    const uint4 pb = reinterpret_cast<const uint4*>(pw + 4)[0];    // onsets, census vectors read
+    const uint2 pm = reinterpret_cast<const uint2*>(pw + 8)[0];    // infectious mosquitoes
+    const CommDesc& cd = v.comm[g];
+    const uint32_t row_off = cd.row_off, rl = cd.row_len, c = cd.c, flags = cd.flags;
+    uint32_t thr[2], box[2];
+#pragma unroll
+    for (uint32_t u = 0; u < 2; ++u) {
+        const uint32_t e = u * 256 + tid;
+        thr[u] = e < cb.rows ? v.csr_thr[cb.row + e] : 0u;
+        box[u] = e < cb.rows ? v.csr_inbox[cb.row + e] : 0u;
+    }
     const uint32_t t = *v.day + v.day_offset;
-    const SimDesc& sd = v.sims[sim];
-    __shared__ unsigned long long s_fx[8];
-    __shared__ uint32_t s_cnt[4][10];   // per wave: humans, mosquitoes, infectious[4], onsets[4]
-    __shared__ unsigned long long s_scan[2];
-    if (tid < 8) s_fx[tid] = 0ull;
-    if (tid < 2) s_scan[tid] = 0ull;
-    __syncthreads();
-    uint32_t nh = 0, nm = 0, inf[4] = {0, 0, 0, 0}, inc[4] = {0, 0, 0, 0};
-    uint32_t sv_h = 0, sv_m = 0;   // census vectors scanned (fits 32 bits: at most 64 communities per thread)
-    unsigned long long fx[8] = {0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull};
-    for (uint32_t c = part * 256 + tid; c < sd.C; c += split * 256) {
-        const uint32_t* pw = v.part + (size_t)(sd.comm_off + c) * kPartWords;
-        const uint4 a = reinterpret_cast<const uint4*>(pw)[0];
-        const uint4 b = reinterpret_cast<const uint4*>(pw + 4)[0];
-        sv_h += b.z;
-        sv_m += b.w;
-        nm += a.x;
-        nh += a.y;
-        inf[0] += a.z & 0xFFFFu; inf[1] += a.z >> 16; inf[2] += a.w & 0xFFFFu; inf[3] += a.w >> 16;
-        inc[0] += b.x & 0xFFFFu; inc[1] += b.x >> 16; inc[2] += b.y & 0xFFFFu; inc[3] += b.y >> 16;
-        const unsigned long long* f = reinterpret_cast<const unsigned long long*>(pw + 8);
+    const SimDesc& sd = v.sims[cb.sim];
+    const Key key{sd.k0, sd.k1};
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) fx[k] += f[k];
-    }
-    const uint32_t cnt[10] = {nh, nm, inf[0], inf[1], inf[2], inf[3], inc[0], inc[1], inc[2], inc[3]};
-#pragma unroll
-    for (uint32_t k = 0; k < 10; ++k) {
-        const uint32_t w = wave_sum(cnt[k]);
-        if (lane == 0) s_cnt[wv][k] = w;
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {   // butterfly over the wave, then one LDS add per wave
-        unsigned long long x = fx[k];
-#pragma unroll
-        for (uint32_t d = kWave / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, kWave);
-        if (lane == 0 && x) atomicAdd(&s_fx[k], x);
-    }
-    {
-        const unsigned long long h = wave_sum(sv_h), m = wave_sum(sv_m);
-        if (lane == 0) {
-            atomicAdd(&s_scan[0], h);
-            atomicAdd(&s_scan[1], m);
+    for (uint32_t u = 0; u < 2; ++u) {
+        const uint32_t e = u * 256 + tid;
+        if (e < cb.rows) {
+            s_row[e] = thr[u];
+            s_box[e] = box[u];
         }
+    }
+    if (in) {
+        for (uint32_t e = k; e < rl; e += 8) s_own[row_off - cb.row + e] = (uint8_t)j;
+        if (k == 0) {
+            s_off[j] = row_off - cb.row;
+            s_rl[j] = rl;
+        }
+    }
+    SourceCount sc{0u, 0u, 0ull};
+    if (in) {
+        const uint32_t I = k < 4 ? unpack_pair(pa.z, pa.w, k) : unpack_pair(pm.x, pm.y, k & 3u);
+        sc = source_count(sd, v.dens, key, c, flags, t, k, I, pa.x, pa.y);
+    }
+    const bool some = __syncthreads_or((int)(sc.n | sc.stay)) != 0;
+    if (some) {
+        for (uint32_t i = tid; i < kCountComms * kCntPerComm; i += 256) (&s_hist[0][0])[i] = 0u;
+        // quads of the workgroup's segments
+        uint32_t wtot;
+        uint32_t q0 = wave_exclusive_scan((sc.n + 3) >> 2, wtot);
+        if (lane == 0) s_wt[wv] = wtot;
+        s_n[tid] = sc.n;
+        __syncthreads();
+        // staying events join the count of the source's own column
+        if (sc.stay) atomicAdd(&s_hist[j][k * 9 + ((flags >> kCommSelfShift) & 15u)], sc.stay);
+        uint32_t qtot = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            if (w < wv) q0 += s_wt[w];
+            qtot += s_wt[w];
+        }
+        s_q[tid] = q0;
+        __syncthreads();
+        for (uint32_t q = tid; q < qtot; q += 256) {
+            uint32_t lo = 0, hi = kSeg - 1;   // the last segment that starts at or before q
+#pragma unroll
+            for (uint32_t b = 0; b < 8; ++b) {
+                const uint32_t mid = (lo + hi + 1) >> 1;
+                if (s_q[mid] <= q) lo = mid; else hi = mid - 1;
+            }
+            const uint32_t jj = lo >> 3, kk = lo & 7u;
+            spread_quad(key, cb.c0 + jj, t, kk, q - s_q[lo], s_n[lo], s_row + s_off[jj], s_rl[jj], &s_hist[jj][kk * 9]);
+        }
+        __syncthreads();
+    }
+    // each entry's eight counts to its destination's inbox
+    for (uint32_t e = tid; e < cb.rows; e += 256) {
+        uint4 lo = make_uint4(0u, 0u, 0u, 0u), hi = lo;
+        const uint32_t dst = s_box[e];
+        if (some) {
+            const uint32_t jj = s_own[e];
+            const uint32_t* h = &s_hist[jj][e - s_off[jj]];
+            lo = make_uint4(h[0], h[9], h[18], h[27]);
+            hi = make_uint4(h[36], h[45], h[54], h[63]);
+            if (lo.x | lo.y | lo.z | lo.w | hi.x | hi.y | hi.z | hi.w)
+                v.active[dst / kInboxEdges] = 1u;   // the destination has events today
+        }
+        uint4* box4 = reinterpret_cast<uint4*>(v.cnt + (size_t)dst * 8);
+        box4[0] = lo;
+        box4[1] = hi;
+    }
+    // the workgroup's sums: lane k of a community has two of its twelve
+    // partials, added over the wave's communities, then over the waves
+    uint32_t x = k == 0 ? pa.y : k == 1 ? pa.x : k == 2 ? pa.z & 0xFFFFu : k == 3 ? pa.z >> 16 : k == 4 ? pa.w & 0xFFFFu
+               : k == 5 ? pa.w >> 16 : k == 6 ? pb.x & 0xFFFFu : pb.x >> 16;
+    uint32_t y = k == 0 ? pb.y & 0xFFFFu : k == 1 ? pb.y >> 16 : k == 2 ? pb.z : k == 3 ? pb.w : 0u;
+    if (!in) x = y = 0u;
+    unsigned long long fx = sc.fx;
+#pragma unroll
+    for (uint32_t d = 8; d < kWave; d <<= 1) {
+        x += __shfl_xor(x, d, kWave);
+        y += __shfl_xor(y, d, kWave);
+        fx += __shfl_xor(fx, d, kWave);
+    }
+    if (lane < 8) {
+        s_cnt[wv][k] = x;
+        if (k < 4) s_cnt[wv][8 + k] = y;
+        s_fx[wv][k] = fx;
     }
     __syncthreads();
     const uint32_t S = sd.S, row = t + 1;
     const SeriesIdx si = series_index(sd.series_off, v.max_days, S);
-    if (tid < 10) {
-        const uint32_t k = tid;
-        const uint32_t x = s_cnt[0][k] + s_cnt[1][k] + s_cnt[2][k] + s_cnt[3][k];
+    if (tid < 12) {
+        const uint32_t n = s_cnt[0][tid] + s_cnt[1][tid] + s_cnt[2][tid] + s_cnt[3][tid];
         uint32_t* dst = nullptr;
-        if (k == 0) dst = &v.series[si.n_count + row];
-        else if (k == 1) dst = &v.series[si.m_count + row];
-        else if (k < 6) { if (k - 2 < S) dst = &v.series[si.n_inf + (size_t)row * S + (k - 2)]; }
-        else if (k - 6 < S) dst = &v.series[si.n_inc + (size_t)row * S + (k - 6)];
-        if (dst && x) atomicAdd(dst, x);
+        if (tid == 0) dst = &v.series[si.n_count + row];
+        else if (tid == 1) dst = &v.series[si.m_count + row];
+        else if (tid < 6) { if (tid - 2 < S) dst = &v.series[si.n_inf + (size_t)row * S + (tid - 2)]; }
+        else if (tid < 10) { if (tid - 6 < S) dst = &v.series[si.n_inc + (size_t)row * S + (tid - 6)]; }
+        else if (n) atomicAdd(&v.scanned[2 * (size_t)cb.sim + (tid - 10)], (unsigned long long)n);
+        if (dst && n) atomicAdd(dst, n);
     }
-    if (tid >= 32 && tid < 40 && s_fx[tid - 32])
-        atomicAdd(&v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + (tid - 32)], s_fx[tid - 32]);
-    if (tid >= 64 && tid < 66 && s_scan[tid - 64]) atomicAdd(&v.scanned[2 * (size_t)sim + (tid - 64)], s_scan[tid - 64]);
+    if (tid >= 64 && tid < 72) {
+        const unsigned long long n = s_fx[0][tid - 64] + s_fx[1][tid - 64] + s_fx[2][tid - 64] + s_fx[3][tid - 64];
+        if (n) atomicAdd(&v.lam[((size_t)(t & 1u) * v.n_sims + cb.sim) * 8 + (tid - 64)], n);
+    }
 }
 
 // Age-of-infection rings (nepidemic.cu:229-243), a wave per community after
@@ -1776,6 +1878,21 @@ hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Small batches: one shape for each number of waves per community (the order
+// of so few communities and their registers make no difference).
+template <bool HIST>
+static hipError_t launch_demography_small(const EngineView& v, uint32_t nw, hipStream_t st) {
+    const size_t lds = (size_t)v.death_m_lds * 4;
+    if (v.max_words > kWaveWords * nw) nw = kMaxWaves;   // a community's bitmap needs more waves than the tuning's
+    const dim3 grid(v.n_comm), block(kWave * nw);
+    if (nw == 1) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 1, true>), grid, block, lds, st, v);
+    else if (nw == 2) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 2, true>), grid, block, lds, st, v);
+    else if (nw == 4) hipLaunchKernelGGL((k_day_demography<2, 2, false, HIST, 0, 4, true>), grid, block, lds, st, v);
+    else if (nw == 8) hipLaunchKernelGGL((k_day_demography<2, 2, false, HIST, 0, 8, true>), grid, block, lds, st, v);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 // Demography variants: (UNROLL, EARLY_M) pairs of kDemographyShapes with one
 // wave per community, the kOccShapes pairs under an 8-waves-per-SIMD register
 // budget, and the kWideShapes with several waves per community.
@@ -1842,6 +1959,11 @@ bool tuning_supported(const Tuning& tu) {
 }
 
 hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t st) {
+    if (v.small) {
+        if (!tuning_supported(tu)) return hipErrorInvalidValue;
+        return (v.hist || v.spatial) ? launch_demography_small<true>(v, tu.nw, st)
+                                     : launch_demography_small<false>(v, tu.nw, st);
+    }
     return (tu.xcd & 1u) ? launch_demography_x<true>(v, tu, st) : launch_demography_x<false>(v, tu, st);
 }
 
@@ -1869,7 +1991,7 @@ hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st) 
 
 hipError_t launch_longdist(const EngineView& v, const Tuning& tu, hipStream_t st) {
     if (v.small) return hipSuccess;   // the event kernel does both
-    hipLaunchKernelGGL(k_day_reduce, dim3(v.n_sims * v.reduce_split), dim3(256), 0, st, v, v.reduce_split);
+    hipLaunchKernelGGL(k_day_counts, dim3(v.count_blocks), dim3(256), 0, st, v);
     hipLaunchKernelGGL(k_day_longdist, dim3(v.n_sims * tu.ld_split), dim3(256), 0, st, v, tu.ld_split);
     return hipGetLastError();
 }

@@ -40,6 +40,12 @@ ARBO_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t k) {
 // as 1, 2, 3", SC'11).  Multipliers and Weyl key increments are the published
 // constants of the generator.  The key is the same in every lane of a wave.
 ARBO_HD U4 philox(U4 c, uint32_t k0, uint32_t k1) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // each block steps its own copy of the key with scalar adds: shared
+    // between a kernel's blocks, the 20 round keys stay in scalar registers
+    // all through it and push others out to vector lanes
+    asm("" : "+s"(k0), "+s"(k1));
+#endif
 #pragma unroll
     for (int i = 0; i < 10; ++i) {
         const uint64_t p0 = (uint64_t)0xD2511F53u * c.x;

@@ -109,3 +109,21 @@ def test_first_census_across_workgroups(hip_lib, oracle_lib, humans, slots):
     p = configs.base_params(n_serotypes=3, immunity_mode=1, seed_frac_h=0.05, seed_frac_m=0.05)
     specs = [SimSpec(3, 1, np.array(humans, np.uint32), p, 77, mosq_slots=np.array(slots, np.uint32))]
     _both(hip_lib, oracle_lib, specs, 3, flags=abi.F_AOI | abi.F_SPATIAL, checks=(0,))
+
+
+@pytest.mark.parametrize("grids,humans,omega", [([(32, 16)], 30, 0.3), ([(27, 19)], 30, 0.3), ([(8, 8)], 512, 1.0),
+                                                ([(8, 8)], 513, 1.0), ([(32, 16)] * 8, 5, 0.1),
+                                                ([(32, 16)] * 8 + [(1, 1)], 5, 0.1), ([(33, 1), (521, 1), (31, 1)], 25, 0.2)])
+def test_small_batches_and_their_limits(hip_lib, oracle_lib, grids, humans, omega):
+    """On both sides of the sizes up to which a batch's event kernel draws the
+    long-distance events and sums the series itself, under both count laws,
+    with staying events, and communities around the workgroups of 32."""
+    print(f"[edges] small {grids[:2]} {humans} {omega}", flush=True)
+    specs = []
+    for i, (w, h) in enumerate(grids):
+        over = dict(count_law=abi.COUNT_STOCH_ROUND) if i % 2 else {}
+        if i % 3 == 1:
+            over.update(no_distance=0.3, include_self=0)
+        p = configs.base_params(beta_hm=0.7, beta_mh=0.7, seed_frac_h=0.05, seed_frac_m=0.05, long_distance=omega, **over)
+        specs.append(SimSpec(w, h, np.full(w * h, humans, np.uint32), p, 90 + i))
+    _both(hip_lib, oracle_lib, specs, 25, flags=abi.F_GRAPH, checks=(3, 9))
