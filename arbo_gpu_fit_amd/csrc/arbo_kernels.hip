@@ -104,6 +104,11 @@ __device__ __forceinline__ uint32_t sub_u16x2(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) - __builtin_bit_cast(u16x2, b));
 }
 
+// The smaller of each pair of 16-bit halves (v_pk_min_u16).
+__device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
 // Exclusive prefix sum over the wavefront, every lane active; `total` gets
 // the wave sum.  An inclusive scan by DPP: row_shr 1, 2, 4, 8 within each
 // row of 16 lanes (lanes shifted in from outside the row add 0), then lane
@@ -437,7 +442,9 @@ __global__ __launch_bounds__(256) void k_init(EngineView v) {
 // Per-lane tallies of the exposed and infectious humans: infectious (ih)
 // and E -> I onsets today (inc) as pairs of 16-bit serotype counts, and the
 // earliest next state-change day of those members (minev).
-struct HumanCount { uint32_t ih01, ih23, inc01, inc23, minev; };
+// soon: the days from t to the earliest next state change of the members
+// human_states_packed kept, least of each 16-bit half (0xFFFF: none).
+struct HumanCount { uint32_t ih01, ih23, inc01, inc23, minev, soon; };
 
 __device__ __forceinline__ uint32_t day_of(uint32_t t, uint32_t nx) {   // absolute day of a 16-bit day near t
     return (uint32_t)((int32_t)t + (int32_t)(int16_t)(uint16_t)(nx - t));
@@ -486,6 +493,55 @@ __device__ __forceinline__ uint32_t human_states(const EngineView& v, const Comm
             ev = day_of(t, nx) + 1;
         }
         hc.minev = ev < hc.minev ? ev : hc.minev;
+    }
+    return ons;
+}
+
+// human_states for a vector none of whose members dies today (nor in any
+// other lane of the wave): the four members' statuses, strains and due tests
+// packed in bytes, member e at bit 8 e, and the days to the next change as
+// 16-bit halves.  About 55 instructions where member by member takes 140, on
+// most vectors of a community with an epidemic.
+__device__ __forceinline__ uint32_t human_states_packed(const EngineView& v, const CommDesc& cd, uint32_t t,
+                                                        uint32_t q, const uint32_t (&ws)[4], HumanCount& hc,
+                                                        uint16_t* onx) {
+    constexpr uint32_t kB = 0x01010101u;
+    asm volatile("" : "+v"(hc.ih01), "+v"(hc.ih23), "+v"(hc.inc01), "+v"(hc.inc23), "+v"(hc.soon));   // as in human_states
+    const uint2 nx = *reinterpret_cast<const uint2*>(v.h_next + cd.h_off + 4 * q);
+    const uint32_t T16 = (t & 0xFFFFu) * 0x00010001u;
+    // the members' low bytes: status, strain << 2
+    const uint32_t r = __builtin_amdgcn_perm(ws[1], ws[0], 0x0C0C0400u) |
+                       (__builtin_amdgcn_perm(ws[3], ws[2], 0x0C0C0400u) << 16);
+    const uint32_t ex = r & kB, inf = (r >> 1) & kB, sa = (r >> 2) & kB, sb = (r >> 3) & kB;   // status 1, status 2
+    // due: (int16)(t - next) > 0, i.e. bit 15 clear in both d = t - next and d - 1
+    const uint32_t d0 = sub_u16x2(T16, nx.x), d1 = sub_u16x2(T16, nx.y);
+    const uint32_t n0 = d0 | sub_u16x2(d0, 0x00010001u), n1 = d1 | sub_u16x2(d1, 0x00010001u);
+    const uint32_t due = (~__builtin_amdgcn_perm(n1, n0, 0x07050301u) >> 7) & kB;
+    const uint32_t on = ex & due, stay = (ex | inf) & ~due;
+    const uint32_t ill = (inf & ~due) | on;
+    hc.ih01 += (uint32_t)__popc(ill & ~sa & ~sb) + ((uint32_t)__popc(ill & sa & ~sb) << 16);
+    hc.ih23 += (uint32_t)__popc(ill & ~sa & sb) + ((uint32_t)__popc(ill & sa & sb) << 16);
+    // days to the next change of those whose state stays, the others' halves full
+    const uint32_t g0 = (__builtin_amdgcn_perm(0u, stay, 0x0C010C00u) ^ 0x00010001u) * 0xFFFFu;
+    const uint32_t g1 = (__builtin_amdgcn_perm(0u, stay, 0x0C030C02u) ^ 0x00010001u) * 0xFFFFu;
+    hc.soon = min_u16x2(hc.soon, min_u16x2(sub_u16x2(nx.x, T16) | g0, sub_u16x2(nx.y, T16) | g1));
+    uint32_t rec = inf & due;
+    while (rec) {   // recovered
+        const uint32_t b = (uint32_t)__ffs((int)rec) - 1u, e = b >> 3;
+        rec &= rec - 1u;
+        const uint32_t w = e == 0 ? ws[0] : e == 1 ? ws[1] : e == 2 ? ws[2] : ws[3];
+        v.h_word[cd.h_off + 4 * q + e] = w & ~0xFu;
+    }
+    uint32_t ons = 0;
+    if (on) {   // E -> I: counted now, the infectious period drawn later
+        const uint32_t nxs[4] = {nx.x & 0xFFFFu, nx.x >> 16, nx.y & 0xFFFFu, nx.y >> 16};
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e) {
+            if (!((on >> (8 * e)) & 1u)) continue;
+            add_pair(hc.inc01, hc.inc23, (ws[e] >> 2) & 3u);
+            ons |= 1u << e;
+            onx[e] = (uint16_t)nxs[e];
+        }
     }
     return ons;
 }
@@ -699,7 +755,7 @@ void k_day_demography(EngineView v) {
     const float dens_next = v.dens[sd.dens_off + t + 1];
 
     // ---- humans ----
-    HumanCount hc{0, 0, 0, 0, 0xFFFFFFFFu};
+    HumanCount hc{0, 0, 0, 0, 0xFFFFFFFFu, 0xFFFFFFFFu};
     // Changes that need a random draw queue up in LDS (the dead-slot bitmap
     // arrays, not used before the mosquito scan; one queue per wave) and are
     // processed a lane each when the queue could overflow and after the scan.
@@ -752,8 +808,12 @@ void k_day_demography(EngineView v) {
         minw = in ? umin(minw, umin(m01, m23)) : minw;
         // exposed and infectious members (rare): their onsets join the deaths
         uint32_t ons = 0;
-        if (in && ((ws[0] | ws[1] | ws[2] | ws[3]) & 3u) != 0u)
+        const bool any = in && ((ws[0] | ws[1] | ws[2] | ws[3]) & 3u) != 0u;
+        if ((bal[0] | bal[1] | bal[2] | bal[3]) == 0ull) {
+            if (any) ons = human_states_packed(v, cd, t, q, ws, hc, s_onx + 4 * tid);
+        } else if (any) {
             ons = human_states(v, cd, t, tt, q, ws, hc, s_onx + 4 * tid);
+        }
         if (__builtin_amdgcn_ballot_w64(ons != 0u)) {
 #pragma unroll
             for (uint32_t e = 0; e < 4; ++e) bal[e] |= __builtin_amdgcn_ballot_w64((ons >> e) & 1u);
@@ -907,7 +967,8 @@ void k_day_demography(EngineView v) {
     if (scan_h) {
         ih01 = wave_sum(hc.ih01); ih23 = wave_sum(hc.ih23);
         inc01 = wave_sum(hc.inc01); inc23 = wave_sum(hc.inc23);
-        minev = wave_min(umin(hc.minev, minw >> 8));
+        const uint32_t soon = umin(hc.soon & 0xFFFFu, hc.soon >> 16);
+        minev = wave_min(umin(umin(hc.minev, minw >> 8), soon == 0xFFFFu ? 0xFFFFFFFFu : t + soon + 1u));
     } else {
         ih01 = wv == 0 ? hs.y : 0u;
         ih23 = wv == 0 ? hs.z : 0u;
