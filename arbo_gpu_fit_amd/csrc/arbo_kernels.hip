@@ -57,9 +57,7 @@ constexpr uint32_t kMaxWaves = (kMaxWords + kWaveWords - 1) / kWaveWords;   // w
 // The demography kernel's census loads in flight per lane (UNROLL) and, of
 // the first batch, the mosquito vectors issued before the human scan
 // (EARLY_M) are template parameters chosen per engine (Tuning).
-constexpr uint32_t kChunk = 256;                               // events per claim pass
-constexpr uint32_t kPerLane = kChunk / kWave;                  // 4
-constexpr uint32_t kHash = 512;                                // claim-table entries (2 x chunk)
+constexpr uint32_t kChunk = 256;                               // events per claim pass and wave
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;
 constexpr uint32_t kKeyBits = 17;                              // member index < 2^17
 constexpr uint32_t kKeyMask = (1u << kKeyBits) - 1u;
@@ -1177,10 +1175,9 @@ void k_day_demography(EngineView v) {
 // source) and then the long-distance arrivals.  Event k of a segment draws its
 // target from word k%4 of the segment's Philox block k/4, so a lane handles a
 // quad of consecutive events with one block.  Quads are applied in chunks of
-// kChunkQuads with an LDS claim-min table.
+// one per lane with an LDS claim-min table: up to 256 events a wave, and
+// every wave of the community's workgroup takes part in a chunk.
 
-constexpr uint32_t kChunkQuads = kChunk / 4;   // 64 quads = up to 256 events
-constexpr uint32_t kQuadsPerLane = kChunkQuads / kWave;  // 1
 
 struct Quad {
     uint32_t s;       // serotype
@@ -1215,13 +1212,17 @@ __device__ __forceinline__ Quad decode_quad(uint32_t gq, const uint32_t* seg, co
     return q;
 }
 
-__device__ __forceinline__ uint32_t claim_slot(uint32_t key) { return (key * 2654435761u) >> 23; }
+template <uint32_t HASH>
+__device__ __forceinline__ uint32_t claim_slot(uint32_t key) {
+    return (key * 2654435761u) >> (32 - __builtin_ctz(HASH));
+}
 
 // Record event `rank` of the chunk on member `key`; the table keeps the
-// smallest rank per member (open addressing, at most kChunk keys in kHash).
+// smallest rank per member (open addressing, at most HASH / 2 keys).
+template <uint32_t HASH>
 __device__ __forceinline__ void claim(uint32_t* tab, uint32_t key, uint32_t rank) {
     const uint32_t packed = (rank << kKeyBits) | key;
-    uint32_t h = claim_slot(key);
+    uint32_t h = claim_slot<HASH>(key);
     while (true) {
         uint32_t cur = tab[h];
         if (cur == kEmpty) {
@@ -1232,13 +1233,14 @@ __device__ __forceinline__ void claim(uint32_t* tab, uint32_t key, uint32_t rank
             atomicMin(&tab[h], packed);
             return;
         }
-        h = (h + 1) & (kHash - 1);
+        h = (h + 1) & (HASH - 1);
     }
 }
 
+template <uint32_t HASH>
 __device__ __forceinline__ uint32_t claimed_rank(const uint32_t* tab, uint32_t key) {
-    uint32_t h = claim_slot(key);
-    while (tab[h] == kEmpty || (tab[h] & kKeyMask) != key) h = (h + 1) & (kHash - 1);
+    uint32_t h = claim_slot<HASH>(key);
+    while (tab[h] == kEmpty || (tab[h] & kKeyMask) != key) h = (h + 1) & (HASH - 1);
     return tab[h] >> kKeyBits;
 }
 
@@ -1294,24 +1296,31 @@ __device__ __forceinline__ void reduce_simulation(const EngineView& v, uint32_t 
 
 // MW: bitmap words of a community in units of kWaveWords (1, or kMaxWaves
 // for batches with communities above 8,192 slots): the alive-rank index is
-// built in MW passes of four words per lane.
+// built in MW spans of four words per lane.
 // SMALL: the day has no k_day_counts and no k_day_longdist, 5 us of a launch
 // each where a day of 100 communities takes 30: every community's wave sums
 // its simulation's long-distance rates and draws all of its events' landing
 // places itself, keeping those that land here, and one more workgroup per
 // simulation sums the series row beside them (kSmallCommunities).
-template <bool XCD, bool HIST, uint32_t MW, bool SMALL>
-__global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
-    const uint32_t g = XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x, lane = threadIdx.x;
+// NW: waves of a community's workgroup.  Each finds the same segments for
+// itself; the alive index, the long-distance draws and the chunks are split
+// over them.
+template <bool XCD, bool HIST, uint32_t MW, bool SMALL, uint32_t NW = 1>
+__global__ __launch_bounds__(kWave * NW) void k_day_events(EngineView v) {
+    static_assert(NW == 1 || SMALL, "arrivals counted by k_day_longdist are read and cleared by one wave");
+    constexpr uint32_t kHash = 2 * NW * kChunk;   // claim-table entries
+    const uint32_t g = XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x, tid = threadIdx.x;
+    const uint32_t lane = tid % kWave, wave = NW > 1 ? tid / kWave : 0u;
     const uint32_t t = *v.day + v.day_offset;
     if (SMALL && g >= v.n_comm) {
-        reduce_simulation(v, g - v.n_comm, t, lane);
+        if (wave == 0) reduce_simulation(v, g - v.n_comm, t, lane);
         return;
     }
     const CommDesc cd = v.comm[g];
     const uint32_t act = v.active[g];
     if (!SMALL && !act && !(cd.flags & kCommIntro)) return;   // no events arrive and no introductions
-    if (act && lane == 0) v.active[g] = 0u;         // consumed
+    if (NW > 1) __syncthreads();                    // every wave has read it
+    if (act && tid == 0) v.active[g] = 0u;          // consumed
     const SimDesc sd = v.sims[cd.sim];
     const Key key{sd.k0, sd.k1};
     const uint32_t S = sd.S;
@@ -1331,7 +1340,7 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
     __shared__ uint32_t s_tab[kHash];
 
     if (lane < in_len) {
-        s_src[lane] = v.in_edge[cd.in_off + lane];
+        s_src[lane] = v.in_edge[cd.in_off + lane] - sd.comm_off;   // simulation-local source ids
         s_slot[lane] = v.in_slot[cd.in_off + lane];
     }
     uint32_t tot_dir[2] = {0, 0};
@@ -1354,7 +1363,7 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) pre[k + 1] = pre[k] + (uint32_t)__builtin_amdgcn_readlane((int)L, (int)k);
         __syncthreads();
-        for (uint32_t l = lane; l < pre[8]; l += kWave) {
+        for (uint32_t l = tid; l < pre[8]; l += kWave * NW) {
             uint32_t k = 0, first = 0;
 #pragma unroll
             for (uint32_t q = 1; q < 8; ++q) {
@@ -1403,37 +1412,72 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
         if (lane < nseg) { s_seg[dir][lane] = start; s_qseg[dir][lane] = qstart; }
         if (lane == 0) { s_seg[dir][nseg] = total; s_qseg[dir][nseg] = qtotal; }
     }
-    if (lane < in_len) s_src[lane] -= sd.comm_off;   // simulation-local source ids
     __syncthreads();
 
     // ---- onto mosquitoes: uniform over alive slots, success iff susceptible ----
     const uint32_t tq_m = s_qseg[DIR_HM][nseg], tq_h = s_qseg[DIR_MH][nseg];
     const uint32_t nwords = (cd.cap + 31) >> 5;
     uint32_t Md = 0;
-    for (uint32_t c0 = 0; tq_m > 0 && c0 < MW && kWaveWords * c0 < nwords; ++c0) {   // wave-uniform
+    constexpr uint32_t kPasses = (MW + NW - 1) / NW;   // spans of kWaveWords words per wave
+    __shared__ uint32_t s_span[NW > 1 ? MW : 1];       // alive slots of each span
+    uint32_t wv[NW > 1 ? kPasses : 1][kWordsPerLane], pre_in[NW > 1 ? kPasses : 1];
+    // the span's words and the alive slots before each lane's
+    auto read_span = [&](uint32_t c0, uint32_t* w4, uint32_t& total) {
         const uint32_t i4 = kWave * c0 + lane;   // the lane's 16-byte group of words
-        uint32_t wv[kWordsPerLane] = {0u, 0u, 0u, 0u}, c = 0;
+        w4[0] = w4[1] = w4[2] = w4[3] = 0u;
         if (kWordsPerLane * i4 < nwords) {   // one 16-byte load (words past the capacity are zero)
             const uint4 a4 = reinterpret_cast<const uint4*>(v.alive + (cd.m_off >> 5))[i4];
-            wv[0] = a4.x; wv[1] = a4.y; wv[2] = a4.z; wv[3] = a4.w;
+            w4[0] = a4.x; w4[1] = a4.y; w4[2] = a4.z; w4[3] = a4.w;
         }
+        uint32_t c = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < kWordsPerLane; ++k) c += __popc(wv[k]);
-        uint32_t chunk;
-        uint32_t pre = Md + wave_exclusive_scan(c, chunk);
+        for (uint32_t k = 0; k < kWordsPerLane; ++k) c += __popc(w4[k]);
+        return wave_exclusive_scan(c, total);
+    };
+    auto index_span = [&](uint32_t c0, const uint32_t* w4, uint32_t pre) {
+        const uint32_t i4 = kWave * c0 + lane;
 #pragma unroll
         for (uint32_t k = 0; k < kWordsPerLane; ++k) {
             const uint32_t w = kWordsPerLane * i4 + k;
-            const uint32_t cw = __popc(wv[k]);
+            const uint32_t cw = __popc(w4[k]);
             if (w < nwords) {
-                s_word[w] = wv[k];
+                s_word[w] = w4[k];
                 s_wpre[w] = (uint16_t)pre;
                 const uint32_t m = (pre + 31u) & ~31u;   // the multiple of 32 among this word's ranks, if any
                 if (m < pre + cw) s_sel[m >> 5] = (uint16_t)w;
             }
             pre += cw;
         }
-        Md += chunk;
+    };
+    if (NW == 1) {
+        for (uint32_t c0 = 0; tq_m > 0 && c0 < MW && kWaveWords * c0 < nwords; ++c0) {   // wave-uniform
+            uint32_t span;
+            const uint32_t pre = read_span(c0, wv[0], span);
+            index_span(c0, wv[0], Md + pre);
+            Md += span;
+        }
+    } else if (tq_m > 0) {   // uniform over the workgroup
+#pragma unroll
+        for (uint32_t p = 0; p < kPasses; ++p) {
+            const uint32_t c0 = p * NW + wave;
+            uint32_t span;
+            pre_in[p] = read_span(c0, wv[p], span);
+            if (c0 < MW && lane == 0) s_span[c0] = span;
+        }
+        __syncthreads();
+        uint32_t before[MW];
+#pragma unroll
+        for (uint32_t c = 0; c < MW; ++c) {
+            before[c] = Md;
+            Md += s_span[c];
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < kPasses; ++p) {
+            uint32_t b = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < NW && p * NW + w < MW; ++w) b = wave == w ? before[p * NW + w] : b;
+            index_span(p * NW + wave, wv[p], b + pre_in[p]);
+        }
     }
     const uint32_t mq = Md > 0 ? tq_m : 0u;   // with no alive mosquito every event onto one fails
     // ---- onto humans: uniform target, success iff S and never infected by s ----
@@ -1448,16 +1492,12 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
     // chunk rank 4 p + e keeps the list order.
     auto apply_run = [&](uint32_t m_lo, uint32_t m_hi, uint32_t h_lo, uint32_t h_hi) {
         const uint32_t lm = m_hi - m_lo, len = lm + (h_hi - h_lo);
-        for (uint32_t c0 = 0; c0 < len; c0 += kChunkQuads) {
-            for (uint32_t i = lane; i < kHash; i += kWave) s_tab[i] = kEmpty;
+        for (uint32_t c0 = 0; c0 < len; c0 += kWave * NW) {
+            for (uint32_t i = tid; i < kHash; i += kWave * NW) s_tab[i] = kEmpty;
             __syncthreads();
-            uint32_t cache[kPerLane], word[kPerLane];
-#pragma unroll
-            for (uint32_t u = 0; u < kQuadsPerLane; ++u) {
-#pragma unroll
-                for (uint32_t e = 0; e < 4; ++e) cache[4 * u + e] = 0;
-                const uint32_t p = c0 + u * kWave + lane;
-                if (p >= len) continue;
+            uint32_t cache[4] = {0, 0, 0, 0}, word[4];
+            const uint32_t p = c0 + tid;
+            if (p < len) {
                 const bool hum = p >= lm;
                 const uint32_t dir = hum ? DIR_MH : DIR_HM;
                 const Quad q = decode_quad(hum ? h_lo + (p - lm) : m_lo + p, s_seg[dir], s_qseg[dir], nseg, in_len,
@@ -1492,18 +1532,18 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
                     // a human: susceptible and never infected by s; a mosquito: susceptible (no immunity bits)
                     const bool ok = e < q.count && (tw[e] & 3u) == 0 && !(hum && ((tw[e] >> (4 + q.s)) & 1u));
                     if (ok) {
-                        claim(s_tab, tgt[e], 4 * (u * kWave + lane) + e);
-                        cache[4 * u + e] = kEligible | (q.s << kKeyBits) | tgt[e];
+                        claim<kHash>(s_tab, tgt[e], 4 * tid + e);
+                        cache[e] = kEligible | (q.s << kKeyBits) | tgt[e];
                     }
-                    word[4 * u + e] = tw[e];
+                    word[e] = tw[e];
                 }
             }
             __syncthreads();
 #pragma unroll
-            for (uint32_t i = 0; i < kPerLane; ++i) {
+            for (uint32_t i = 0; i < 4; ++i) {
                 if (!(cache[i] & kEligible)) continue;
                 const uint32_t k = cache[i] & kKeyMask;
-                if (claimed_rank(s_tab, k) != 4 * ((i >> 2) * kWave + lane) + (i & 3u)) continue;
+                if (claimed_rank<kHash>(s_tab, k) != 4 * tid + i) continue;
                 const uint32_t s = (cache[i] >> kKeyBits) & 3u;
                 const uint32_t w = word[i];   // as read by the claim pass: only the winner writes it
                 if (k >= kHumanKey) {
@@ -1587,6 +1627,7 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
                     }
                 }
             };
+            if (NW > 1 && wave != 0) x = 0;   // one wave walks the tries
             if (x > 0) introduce(0, std::integral_constant<uint32_t, 1>{});
             for (uint32_t att = kWave; x > 0 && att < kIntroTries; att += 4 * kWave)
                 introduce(att, std::integral_constant<uint32_t, 4>{});
@@ -1596,7 +1637,15 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
     if (HIST && v.aoi_mark) {   // the community's records of the day, for k_day_aoi
         aoi01 = wave_sum(aoi01);
         aoi23 = wave_sum(aoi23);
-        if (aoi01 | aoi23) {
+        if (NW > 1) {
+            __shared__ uint32_t s_aoi[2][NW];
+            if (lane == 0) { s_aoi[0][wave] = aoi01; s_aoi[1][wave] = aoi23; }
+            __syncthreads();
+            aoi01 = aoi23 = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < NW; ++w) { aoi01 += s_aoi[0][w]; aoi23 += s_aoi[1][w]; }
+        }
+        if ((aoi01 | aoi23) && wave == 0) {
             if (lane == 0) reinterpret_cast<uint4*>(v.aoi_cnt)[g] = make_uint4(t + 1u, aoi01, aoi23, 0u);
             if (lane < 4) {
                 const uint32_t n = unpack_pair(aoi01, aoi23, lane);
@@ -1606,6 +1655,7 @@ __global__ __launch_bounds__(kWave) void k_day_events(EngineView v) {
         }
     }
     // a human exposed today turns infectious on day t + iip + 1 at the earliest
+    // (waves that store here store the same day)
     if (__any(infected) && lane == 0) {
         const uint32_t ev = t + sd.iip_min + 1;
         if (ev < v.hsum[4 * (size_t)g]) v.hsum[4 * (size_t)g] = ev;
@@ -2028,11 +2078,22 @@ hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t 
     return (tu.xcd & 1u) ? launch_demography_x<true>(v, tu, st) : launch_demography_x<false>(v, tu, st);
 }
 
+// Waves of the event kernel's workgroups in small batches with communities
+// above 8,192 slots.  Smaller communities keep one: their day's events are
+// one or two chunks, and four waves made 100 communities of 1,000 humans
+// 33.9 us a day instead of 32.0 and 4,000 of them 89.7 instead of 62.2.
+constexpr uint32_t kEventWaves = 8;
+
 template <bool HIST>
 static void launch_events_h(const EngineView& v, const Tuning& tu, hipStream_t st) {
     const dim3 grid(v.n_comm + (v.small ? v.n_sims : 0u)), block(kWave);
     if (v.max_words > kWaveWords) {   // communities above 8,192 slots
-        if (v.small) hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, true>), grid, block, 0, st, v);
+        // A small batch's large communities: eight waves each.  With one, 49
+        // cities of 3,000 to 21,000 humans took 44 us a day (a chain of
+        // 256-event chunks); with four 29.8, with eight 26.9.
+        if (v.small)
+            hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, true, kEventWaves>), grid,
+                               dim3(kEventWaves * kWave), 0, st, v);
         else hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, false>), grid, block, 0, st, v);
     } else if (v.small) {
         hipLaunchKernelGGL((k_day_events<false, HIST, 1, true>), grid, block, 0, st, v);

@@ -127,3 +127,18 @@ def test_small_batches_and_their_limits(hip_lib, oracle_lib, grids, humans, omeg
         p = configs.base_params(beta_hm=0.7, beta_mh=0.7, seed_frac_h=0.05, seed_frac_m=0.05, long_distance=omega, **over)
         specs.append(SimSpec(w, h, np.full(w * h, humans, np.uint32), p, 90 + i))
     _both(hip_lib, oracle_lib, specs, 25, flags=abi.F_GRAPH, checks=(3, 9))
+
+
+@pytest.mark.parametrize("humans,slots", [([30, 9000, 400, 5], [8193, 30000, 300, 1]),
+                                          ([20000, 1, 65535, 700], [8192, 16385, 65535, 40000])])
+@pytest.mark.parametrize("flags", [0, abi.F_AOI])
+def test_large_communities_of_small_batches(hip_lib, oracle_lib, humans, slots, flags):
+    """Several waves apply a community's events: bitmaps that end in the
+    first, a middle and the last wave's words, days of one and of many
+    chunks, introductions between the serotypes, long-distance arrivals."""
+    print(f"[edges] large {humans} {slots} {flags}", flush=True)
+    p = configs.base_params(beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.05, seed_frac_m=0.05, external_infection=60.0,
+                            long_distance=0.1)
+    q = configs.base_params(n_serotypes=2, beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.02, long_distance=0.05)
+    specs = [SimSpec(2, 2, np.array(humans, np.uint32), c, 31, mosq_slots=np.array(slots, np.uint32)) for c in (p, q)]
+    _both(hip_lib, oracle_lib, specs, 16, flags=flags, checks=(1, 6))
