@@ -198,6 +198,7 @@ struct Tuning {
     uint32_t ld_split;   // long-distance kernel: workgroups per simulation
     uint32_t wps;        // demography: 0 the compiler's register budget, 8 eight waves per SIMD
     uint32_t nw;         // demography: waves per community (1, 2, 4)
+    bool chosen;         // set or autotuned; the default leaves a small batch's waves per community to the launch
 };
 constexpr uint32_t kDemographyShapes[][2] = {{4, 4}, {4, 2}, {8, 4}, {2, 2}};   // (unroll, early_m)
 constexpr uint32_t kOccShapes[][2] = {{4, 2}, {2, 2}};   // shapes also built for 8 waves per SIMD

@@ -78,7 +78,7 @@ struct ArboEngine {
     // timing
     std::vector<hipEvent_t> ev_pool, ev_used;
     double kernel_ms[2] = {0.0, 0.0};
-    Tuning tuning{4, 2, 0, 8, 0, 1};   // the autotuner's usual pick on large batches
+    Tuning tuning{4, 2, 0, 8, 0, 1, false};   // the autotuner's usual pick on large batches
     uint64_t kernel_launches[2] = {0, 0};
 };
 
@@ -606,7 +606,7 @@ int arbo_batch_step(ArboEngine* e, uint32_t n_days) {
 namespace {
 
 Tuning from_abi(const ArboTuning& t) {
-    return Tuning{t.census_unroll, t.early_mosq, t.xcd_order, t.ld_split, t.waves_per_simd, t.waves_per_comm};
+    return Tuning{t.census_unroll, t.early_mosq, t.xcd_order, t.ld_split, t.waves_per_simd, t.waves_per_comm, true};
 }
 ArboTuning to_abi(const Tuning& t) { return ArboTuning{t.unroll, t.early_m, t.xcd, t.ld_split, t.wps, t.nw}; }
 

@@ -1990,11 +1990,21 @@ hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
 }
 
 // Small batches: one shape for each number of waves per community (the order
-// of so few communities and their registers make no difference).
+// of so few communities and their registers make no difference).  A tuning
+// that nobody set leaves the number to the batch: up to 1,024 communities get
+// four waves, a SIMD's four then being one community's.  One wave and four, us
+// a day: 100 communities of 1,000 humans 35.5 and 32.0, 484 43.7 and 40.3,
+// 1,000 42.4 and 39.7; 2,304 of 400 humans 36.7 and 44.0, 4,000 of 1,000
+// humans 62.2 and 78.1; 100 of 200 humans 23.2 and 22.9.  Eight waves are no
+// better than four up to 400 communities and slower from 484 on.
+constexpr uint32_t kWideCommunities = 1024;
+
 template <bool HIST>
-static hipError_t launch_demography_small(const EngineView& v, uint32_t nw, hipStream_t st) {
+static hipError_t launch_demography_small(const EngineView& v, const Tuning& tu, hipStream_t st) {
     const size_t lds = (size_t)v.death_m_lds * 4;
+    uint32_t nw = tu.nw;
     if (v.max_words > kWaveWords * nw) nw = kMaxWaves;   // a community's bitmap needs more waves than the tuning's
+    else if (!tu.chosen && v.n_comm <= kWideCommunities) nw = 4;
     const dim3 grid(v.n_comm), block(kWave * nw);
     if (nw == 1) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 1, true>), grid, block, lds, st, v);
     else if (nw == 2) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 2, true>), grid, block, lds, st, v);
@@ -2072,8 +2082,8 @@ bool tuning_supported(const Tuning& tu) {
 hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t st) {
     if (v.small) {
         if (!tuning_supported(tu)) return hipErrorInvalidValue;
-        return (v.hist || v.spatial) ? launch_demography_small<true>(v, tu.nw, st)
-                                     : launch_demography_small<false>(v, tu.nw, st);
+        return (v.hist || v.spatial) ? launch_demography_small<true>(v, tu, st)
+                                     : launch_demography_small<false>(v, tu, st);
     }
     return (tu.xcd & 1u) ? launch_demography_x<true>(v, tu, st) : launch_demography_x<false>(v, tu, st);
 }

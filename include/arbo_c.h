@@ -279,8 +279,12 @@ ARBO_API int arbo_scan_counts(ArboEngine* e, uint64_t* human_vectors, uint64_t* 
 /* Launch knobs of the day kernels.  No knob changes a result: every random
  * draw is keyed by model entities (simulation, community, individual, day,
  * event), never by workgroup or lane, so runs under any tuning are
- * bit-identical.  No counterpart in the reference, whose launch shapes come
- * from the device properties (cudaidentities.h:14-37). */
+ * bit-identical.  Small batches (up to 4,096 communities, 512 in a simulation)
+ * have one kernel shape per waves_per_comm, no long-distance kernel and no
+ * order: only waves_per_comm acts there, and until a tuning is set the engine
+ * gives communities of such a batch four waves where that is the faster.  No
+ * counterpart in the reference, whose launch shapes come from the device
+ * properties (cudaidentities.h:14-37). */
 typedef struct ArboTuning {
     uint32_t census_unroll;   /* demography kernel: 16-byte census loads in flight per lane (2, 4, 8) */
     uint32_t early_mosq;      /* of the first batch, mosquito loads issued before the human scan */

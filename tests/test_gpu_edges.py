@@ -129,6 +129,34 @@ def test_small_batches_and_their_limits(hip_lib, oracle_lib, grids, humans, omeg
     _both(hip_lib, oracle_lib, specs, 25, flags=abi.F_GRAPH, checks=(3, 9))
 
 
+@pytest.mark.parametrize("grids", [[(32, 16), (16, 32)], [(32, 16), (16, 32), (1, 1)]])
+def test_waves_per_community_of_an_unset_tuning(hip_lib, oracle_lib, grids):
+    """1,024 communities, which the engine gives four waves each, and 1,025,
+    which keep one; a tuning that was set holds for both, and reading one sets
+    none."""
+    print(f"[edges] waves {grids}", flush=True)
+    p = configs.base_params(beta_hm=0.7, beta_mh=0.7, seed_frac_h=0.05, seed_frac_m=0.05)
+    specs = [SimSpec(w, h, np.where(np.arange(w * h) % 7 == i, 600, 9).astype(np.uint32), p, 40 + i)
+             for i, (w, h) in enumerate(grids)]
+    orc = Engine(oracle_lib, threads=8)
+    gpu = Engine(hip_lib, flags=abi.F_GRAPH)
+    orc.init(specs, 12)
+    orc.step(12)
+    default = gpu.tuning()
+    assert default["waves_per_comm"] == 1
+    for knobs in ({}, default):
+        gpu.init(specs, 12)
+        if knobs:
+            gpu.set_tuning(**knobs)
+        gpu.step(12)
+        assert gpu.tuning() == default
+        for i in range(len(grids)):
+            _compare_state(gpu.state(i), orc.state(i), f"sim {i}")
+            _compare_series(gpu.series(i), orc.series(i), f"sim {i}")
+    gpu.close()
+    orc.close()
+
+
 @pytest.mark.parametrize("humans,slots", [([30, 9000, 400, 5], [8193, 30000, 300, 1]),
                                           ([20000, 1, 65535, 700], [8192, 16385, 65535, 40000])])
 @pytest.mark.parametrize("flags", [0, abi.F_AOI])
