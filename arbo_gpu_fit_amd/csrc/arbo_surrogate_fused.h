@@ -21,7 +21,7 @@
 //    (sixteen waves of one tile: 28 us for the pass's 20);
 //  * the next 64 k of fragments (the next layer's first ones at a layer's
 //    end) are in flight while the current ones multiply.
-// A 64-row forward pass: 83 -> 19.5 us, 4,096 rows 95 -> 20.5, a training step
+// A 64-row forward pass: 83 -> 18.5 us, 4,096 rows 95 -> 20.5, a training step
 // of 512 rows (this pass there and back, then k_wgrad) 235 -> 56 us.
 // The arithmetic is the bf16x3 split of k_gemm: hi*hi + hi*lo + lo*hi with
 // float32 accumulation, biases, GELU and losses in float32.
@@ -243,12 +243,27 @@ __global__ __launch_bounds__(kFuseThreads) void k_mlp(PassArgs g) {
         // wait for them leaves the requests in flight.
         float side[NT][4] = {};
         if (MODE != PASS_FORWARD && S.kind == STAGE_OUTPUT) {
+            if (MODE == PASS_INPUT && S.N % 4 == 0) {   // dout may be host memory: in segments, as `out` below
+                const __amdgpu_buffer_rsrc_t y = buffer_of(g.y + (uint64_t)row0 * S.N, left * S.N * 4);
+                f32x4 q[NT];
 #pragma unroll
-            for (uint32_t i = 0; i < NT; ++i) {
-                const uint32_t col = (S.tile0 + wave + kFuseWaves * i) * 16 + c4;
+                for (uint32_t i = 0; i < NT; ++i) {
+                    const uint32_t col = (S.tile0 + wave + kFuseWaves * i) * 16 + 4 * (lane & 3u);
+                    q[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         y, col < S.N ? ((lane >> 2) * S.N + col) * 4 : kNoFrag, 0, 0));
+                }
 #pragma unroll
-                for (uint32_t r = 0; r < 4; ++r)   // columns past the last read the first's
-                    side[i][r] = g.y[src * S.N + (col + r < S.N ? col + r : 0u)];
+                for (uint32_t i = 0; i < NT; ++i)
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; ++r) side[i][r] = __shfl(q[i][r], 4 * (lane & 15u) + (lane >> 4), 64);
+            } else {
+#pragma unroll
+                for (uint32_t i = 0; i < NT; ++i) {
+                    const uint32_t col = (S.tile0 + wave + kFuseWaves * i) * 16 + c4;
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; ++r)   // columns past the last read the first's
+                        side[i][r] = g.y[src * S.N + (col + r < S.N ? col + r : 0u)];
+                }
             }
         }
         multiply(S.groups - 1, noff, nsteps, ntiles, 0, no);
@@ -277,18 +292,32 @@ __global__ __launch_bounds__(kFuseThreads) void k_mlp(PassArgs g) {
                 if (MODE != PASS_FORWARD) *reinterpret_cast<f32x4*>(s_f + S.gg_at + row * gg_row(S.N) + col) = gr;
             } else if (S.kind == STAGE_OUTPUT) {
                 const f32x4 bias = *reinterpret_cast<const f32x4*>(s_f + S.bias_at + col);
+                float z[4];
 #pragma unroll
                 for (uint32_t r = 0; r < 4; ++r) {
-                    const float z = acc[i][r] + bias[r];
+                    z[r] = acc[i][r] + bias[r];
                     v[r] = side[i][r];
                     if (MODE == PASS_LOSS) {
-                        const float e = expf(z);
-                        if (col + r < S.N && row < left) loss += (double)e - (double)v[r] * (double)z;
+                        const float e = expf(z[r]);
+                        if (col + r < S.N && row < left) loss += (double)e - (double)v[r] * (double)z[r];
                         v[r] = (e - v[r]) * g.scale;
-                    } else {
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, z), res,
-                                                              col + r < S.N ? (row * S.N + col + r) * 4 : kNoFrag, 0, 0);
                     }
+                }
+                // Four neighbouring lanes take a row's 64 bytes of the tile:
+                // one write each, which matters where `out` is host memory.
+                if (MODE != PASS_LOSS && S.N % 4 == 0) {
+                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                    u32x4 q;
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; ++r)
+                        q[r] = (uint32_t)__shfl((int)__builtin_bit_cast(uint32_t, z[r]), 16 * (lane & 3u) + (lane >> 2), 64);
+                    const uint32_t qc = tile * 16 + 4 * (lane & 3u);
+                    __builtin_amdgcn_raw_buffer_store_b128(q, res, qc < S.N ? ((lane >> 2) * S.N + qc) * 4 : kNoFrag, 0, 0);
+                } else if (MODE != PASS_LOSS) {
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; ++r)
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, z[r]), res,
+                                                              col + r < S.N ? (row * S.N + col + r) * 4 : kNoFrag, 0, 0);
                 }
             } else if (S.kind == STAGE_BACK) {
                 const f32x4 gr = *reinterpret_cast<const f32x4*>(s_f + S.gg_at + row * gg_row(S.N) + col);

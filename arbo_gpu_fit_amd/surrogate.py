@@ -92,15 +92,15 @@ class Surrogate:
     def forward(self, x) -> np.ndarray:
         x = _f32(x)
         n = x.shape[0]
-        out = np.zeros((n, self.widths[-1]), np.float32)
+        out = np.empty((n, self.widths[-1]), np.float32)
         self._check(self.lib.arbo_sur_forward(self._h, n, x.ctypes.data_as(_f32p), out.ctypes.data_as(_f32p)))
         return out
 
     def input_grad(self, x, dout):
         x, dout = _f32(x), _f32(dout)
         n = x.shape[0]
-        out = np.zeros((n, self.widths[-1]), np.float32)
-        dx = np.zeros_like(x)
+        out = np.empty((n, self.widths[-1]), np.float32)
+        dx = np.empty_like(x)
         self._check(self.lib.arbo_sur_input_grad(self._h, n, x.ctypes.data_as(_f32p), dout.ctypes.data_as(_f32p),
                                                  out.ctypes.data_as(_f32p), dx.ctypes.data_as(_f32p)))
         return out, dx

@@ -108,3 +108,75 @@ def test_training_steps_and_packed_weights(hip_lib, widths):
     dout = rng.normal(size=(n, widths[-1])).astype(np.float32)
     assert rel(s.input_grad(x, dout)[1], backward64(after, x, dout)[1]) < 1e-3
     s.close()
+
+
+@pytest.mark.parametrize("widths,max_batch,rows", [([6, 64, 20], 2100, (1023, 1024, 1025, 2049, 2100)),
+                                                   ([512, 16, 511], 4200, (2047, 2051, 4200)),
+                                                   ([3, 300, 7], 1030, (1030,))],
+                         ids=lambda w: "-".join(map(str, w)) if isinstance(w, list) else None)
+def test_host_rows_in_chunks(hip_lib, widths, max_batch, rows):
+    """Host calls around the 1,024 rows of a chunk, and of more rows than the
+    pinned ones hold: every row as in a call of 64 rows."""
+    s = Surrogate(widths, max_batch=max_batch, seed=6, lib=hip_lib)
+    rng = np.random.default_rng(7)
+    x = rng.normal(size=(max_batch, widths[0])).astype(np.float32)
+    dout = rng.normal(size=(max_batch, widths[-1])).astype(np.float32)
+    parts = [s.input_grad(x[i:i + 64], dout[i:i + 64]) for i in range(0, max_batch, 64)]
+    out, dx = (np.concatenate([p[k] for p in parts]) for k in (0, 1))
+    for n in rows:
+        print(f"[tiles] host rows widths={widths} rows={n}", flush=True)
+        assert np.array_equal(s.forward(x[:n]), out[:n])
+        got_out, got_dx = s.input_grad(x[:n], dout[:n])
+        assert np.array_equal(got_out, out[:n]) and np.array_equal(got_dx, dx[:n])
+    s.close()
+
+
+@pytest.mark.parametrize("outputs", [16, 19, 20])
+def test_device_rows_at_any_float_address(hip_lib, outputs):
+    """x and out one to three floats past a 16-byte boundary."""
+    hip = Hip()
+    s = Surrogate([6, 32, outputs], max_batch=64, seed=8, lib=hip_lib)
+    x = np.random.default_rng(9).normal(size=(33, 6)).astype(np.float32)
+    ref = s.forward(x)
+    for k in (1, 2, 3):
+        dev_x = hip.upload(np.concatenate([np.zeros(k, np.float32), x.ravel()]))
+        dev_out = hip.upload(np.full(k + ref.size + 1, 7.0, np.float32))
+        at = [p.value + 4 * k for p in (dev_x, dev_out)]
+        print(f"[tiles] offset {k} outputs={outputs}", flush=True)
+        assert s.lib.arbo_sur_forward_noalloc(s._h, 33, at[0], at[1], None) == 0
+        hip.check(hip.lib.hipDeviceSynchronize(), "hipDeviceSynchronize")
+        got = hip.download(dev_out, (k + ref.size + 1,))
+        assert np.array_equal(got[k:-1].reshape(ref.shape), ref)
+        assert np.all(got[:k] == 7.0) and got[-1] == 7.0
+        hip.check(hip.lib.hipFree(dev_x), "hipFree")
+        hip.check(hip.lib.hipFree(dev_out), "hipFree")
+    s.close()
+
+
+@pytest.mark.parametrize("widths", [[6, 33, 12], [6, 520, 9]], ids=lambda w: "-".join(map(str, w)))
+def test_epochs_take_their_own_row_orders(hip_lib, widths):
+    """Two epochs in one call give the weights of two calls of one, the second
+    on rows laid out so that the first epoch's order reads the second's."""
+    from arbo_gpu_fit_amd.configs import philox4x32
+    n, seed = 50, 11
+    rng = np.random.default_rng(12)
+    x = rng.normal(size=(n, 6)).astype(np.float32)
+    y = rng.poisson(2.0, size=(n, widths[-1])).astype(np.float32)
+    order = []
+    for e in (0, 1):
+        r = philox4x32(np.arange(n), e, 7, 0, seed, 0)[0].astype(np.uint64)
+        perm = list(range(n))
+        for i in range(n - 1, 0, -1):
+            j = int((int(r[i]) * (i + 1)) >> 32)
+            perm[i], perm[j] = perm[j], perm[i]
+        order.append(perm)
+    x2, y2 = np.empty_like(x), np.empty_like(y)
+    x2[order[0]], y2[order[0]] = x[order[1]], y[order[1]]
+    got = []
+    for calls in ([(x, y, 2)], [(x, y, 1), (x2, y2, 1)]):
+        s = Surrogate(widths, max_batch=64, seed=13, lib=hip_lib)
+        for cx, cy, epochs in calls:
+            s.train(cx, cy, epochs=epochs, batch=16, lr=1e-3, seed=seed)
+        got.append(s.get_params())
+        s.close()
+    assert np.array_equal(got[0], got[1])
