@@ -311,6 +311,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     // distinct set of parameters
     std::vector<HumanTable> life_h;
     std::vector<MosquitoTable> life_m;
+    std::map<std::string, uint32_t> seen_life_h, seen_life_m;   // by the bytes of the parameters
     std::vector<double> scales;
     std::vector<uint32_t> sim_h(n_sims), sim_m(n_sims);
     uint32_t max_rows = 1;
@@ -354,18 +355,21 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         sd.iip_span = p.iip_max - p.iip_min + 1;
         {
             const HumanLife life{p.h_infant_shape, p.h_infant_scale, p.h_loc, p.h_scale, p.h_shape};
-            uint32_t k = 0;
-            while (k < life_h.size() && std::memcmp(&life_h[k].life, &life, sizeof life) != 0) ++k;
-            if (k == life_h.size()) life_h.push_back(HumanTable{life, 0u, 0u});
-            sim_h[i] = k;
-            MosquitoTable m{0u, 0u, t.death_m_max, t.m_rows, p.m_scale, p.m_shape, (uint32_t)scales.size(),
-                            t.climate ? max_days : 0u};
-            k = 0;   // rows that follow a climate are the simulation's own
-            while (k < life_m.size() && (t.climate || life_m[k].days || life_m[k].scale0 != m.scale0 ||
-                                         life_m[k].shape != m.shape)) ++k;
-            if (k == life_m.size()) life_m.push_back(m);
-            sim_m[i] = k;
-            scales.insert(scales.end(), t.scale.begin(), t.scale.end());
+            const auto h = seen_life_h.emplace(std::string(reinterpret_cast<const char*>(&life), sizeof life),
+                                               (uint32_t)life_h.size());
+            if (h.second) life_h.push_back(HumanTable{life, 0u, 0u});
+            sim_h[i] = h.first->second;
+            // with a climate the rows follow its daily scales
+            std::string row0(reinterpret_cast<const char*>(&p.m_scale), sizeof p.m_scale);
+            row0.append(reinterpret_cast<const char*>(&p.m_shape), sizeof p.m_shape);
+            row0.append(reinterpret_cast<const char*>(t.scale.data()), t.scale.size() * sizeof(double));
+            const auto m = seen_life_m.emplace(std::move(row0), (uint32_t)life_m.size());
+            if (m.second) {
+                life_m.push_back(MosquitoTable{0u, 0u, t.death_m_max, t.m_rows, p.m_scale, p.m_shape,
+                                               (uint32_t)scales.size(), t.climate ? max_days : 0u});
+                scales.insert(scales.end(), t.scale.begin(), t.scale.end());
+            }
+            sim_m[i] = m.first->second;
             max_rows = std::max(max_rows, t.m_rows);
         }
         sd.init_h_off = pool_add(table_pool, seen_u32, t.init_h);

@@ -1,5 +1,7 @@
 """Day kernels where their waves' shares of work end (GPU), bit for bit
 against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -98,6 +100,34 @@ def test_lifetime_tables_shared_and_distinct(hip_lib, oracle_lib):
     add(300)
     print("[edges] lifetime tables", flush=True)
     _both(hip_lib, oracle_lib, specs, T, checks=(0, 1, 7))
+
+
+def test_equal_climates_share_their_lifetime_rows(hip_lib, oracle_lib):
+    """Simulations under one climate and lifespan share the rows of its
+    lifetime table (a row a day): a batch of them takes the memory of a few,
+    and one of them that differs still gets its own."""
+    hip = ctypes.CDLL("libamdhip64.so.7")   # the runtime the engine is linked with
+
+    def free():
+        n, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(n), ctypes.byref(total)) == 0
+        return n.value
+
+    T, n = 3000, 48
+    cl = configs.seasonal_climate(T + 1)
+    other = configs.seasonal_climate(T + 1, scale_mle=2.0)
+    spec = [SimSpec(1, 1, np.full(1, 50, np.uint32), configs.base_params(), 7 + i, climate=other if i == 3 else cl)
+            for i in range(n)]
+    print("[edges] shared climates", flush=True)
+    gpu, used = Engine(hip_lib), []
+    for k in (4, n):
+        before = free()
+        gpu.init(spec[:k], T)
+        used.append(before - free())
+    gpu.close()
+    # a row has a guide of 256 words; a batch that replaces another returns its memory, so used[1] is the growth
+    assert used[1] < (n - 4) * T * 256 * 4 // 4, used
+    _both(hip_lib, oracle_lib, spec[:6], 20)
 
 
 @pytest.mark.parametrize("humans,slots", [([1, 4095, 4096], [0, 4097, 4096]), ([4097, 8193, 30], [1, 12289, 8192]),
