@@ -10,7 +10,7 @@ Headline workload: the 256-simulation batch (communities log-uniform
 400..10,000 squared to a lattice, 200..2,000 humans per community,
 per-simulation transmission, long-distance and seasonal parameters, 1,825 days
 configured).  One step = one simulated day of every simulation of the batch:
-the demography, reduce, long-distance and event-application kernels over
+the demography, event-count, long-distance and event-application kernels over
 every community.  W warm-up days, then K timed days (W + K <= 1,825; by
 default 25 and 1,800).  With --autotune-days D and at least 10 D warm-up days
 the warm-up first times every launch tuning for D days each and keeps the
@@ -32,10 +32,9 @@ day, against HBM bandwidth.
     death or state change) + 32 B per mosquito vector (8 packed slots, read
     and written back; slots above the highest alive one are skipped) + 4 B
     per 32 mosquito slots of alive bitmap written + per community 64 B of
-    descriptor, 32 B of summary read and written, 96 B of partials and 40 B
-    per CSR entry (its row read, its inbox counts written).  `achieved`
-    divides them by the kernel's mean launch time, measured with HIP events
-    on the engine's stream.
+    descriptor, 32 B of summary read and written and 40 B of partials.
+    `achieved` divides them by the kernel's mean launch time, measured with
+    HIP events on the engine's stream.
   * `traffic` is the kernel's HBM bytes per launch from rocprofv3's
     FETCH_SIZE and WRITE_SIZE passes over this same command (calibrated
     against a plain copy), read from the committed profile; `traffic_frac`
@@ -86,22 +85,6 @@ def profiled_traffic(workload: str, warmup: int, steps: int) -> float | None:
     except (OSError, KeyError, ValueError):
         pass
     return None
-
-
-def row_lengths(spec) -> list[int]:
-    """CSR entries of every community of a simulation: its lattice
-    neighbours (Moore or von Neumann) plus itself when it is a dispersal
-    target or keeps a staying fraction."""
-    p = spec.params
-    own = 1 if (p.include_self or p.no_distance > 0.0) else 0
-    out = []
-    for y in range(spec.grid_h):
-        ny = 1 + (y > 0) + (y < spec.grid_h - 1)
-        for x in range(spec.grid_w):
-            nx = 1 + (x > 0) + (x < spec.grid_w - 1)
-            n = nx * ny - 1 if p.neighbourhood == 8 else (nx - 1) + (ny - 1)
-            out.append(max(1, n + own))
-    return out
 
 
 def host_cpu() -> str:
@@ -233,7 +216,7 @@ def sim_bench(workload: str, args, lib) -> dict:
 
     mean_a = ms_a / max(n_a, 1)
     bitmap = 4 * ((slots + 31) // 32)
-    per_comm = sum(64 + 32 + 96 + 40 * rl for s in specs for rl in row_lengths(s))
+    per_comm = (64 + 32 + 40) * comms
     alg = (16 * hv + 32 * mv) / max(n_a, 1) + bitmap + per_comm
     achieved = alg / (mean_a * 1e-3) / 1e9
     traffic = profiled_traffic(workload, warmup, steps)
