@@ -29,6 +29,9 @@ constexpr uint32_t kAoiRecord = 5000;     // ages per age-of-infection ring
 // mosquitoes the day's scan read, 8-9 infectious mosquitoes (pairs); in small
 // batches 8-23 the eight long-distance rates or counts (u64) instead.
 constexpr uint32_t kPartWords = 24;
+// Communities of a batch: a launch holds fewer than 2^32 threads, and the day
+// kernels take at least 64 a community.
+constexpr uint64_t kMaxCommunities = (1ull << 26) - 1;
 constexpr uint32_t kCountComms = 32;      // communities of a workgroup of k_day_counts
 constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this

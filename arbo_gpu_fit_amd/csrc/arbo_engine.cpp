@@ -277,10 +277,13 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     if (!e) return ARBO_E_INVALID;
     if (n_sims == 0 || !shapes || !params || !seeds) return fail(e, ARBO_E_INVALID, "empty batch");
     if (max_days == 0 || max_days > (1u << 23)) return fail(e, ARBO_E_INVALID, "max_days must be 1..2^23");
+    uint64_t communities = 0;
     for (uint32_t i = 0; i < n_sims; ++i) {
         std::string why = validate(shapes[i], params[i], max_days);
         if (!why.empty()) return fail(e, ARBO_E_INVALID, "simulation " + std::to_string(i) + ": " + why);
+        communities += (uint64_t)shapes[i].grid_w * shapes[i].grid_h;
     }
+    if (communities > kMaxCommunities) return fail(e, ARBO_E_INVALID, "more than 2^26 - 1 communities in the batch");
     HIP_TRY(e, hipSetDevice(e->device));
     HIP_TRY(e, hipStreamSynchronize(e->stream));
     release_graph(e);   // the graph captured the old buffers' addresses
@@ -447,7 +450,6 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     }
     h_tot = align_up(h_tot, kHumanAlign) + kHumanAlign;
     m_tot = align_up(m_tot, kMosqAlign) + ARBO_MAX_COMMUNITY_SLOTS;  // room for whole-workgroup vector reads
-    if (comm.size() >= (1ull << 31)) return fail(e, ARBO_E_INVALID, "too many communities in the batch");
     uint64_t pool_words = table_pool.size();
     for (HumanTable& h : life_h) {
         pool_words = align_up(pool_words, 4);   // read as 16-byte vectors

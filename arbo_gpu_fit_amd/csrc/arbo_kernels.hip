@@ -332,12 +332,15 @@ static_assert(kGuide == kGuideBuckets && kGuide <= 256, "a thread per guide entr
 // LDS; counts are added with integer atomics.  One wave per community, its
 // searches in memory: 2.5 ms for 49 cities of up to 21,000 humans, 11.8 ms for
 // 257,000 communities; this 0.06 and 5.9, of which 1.3 are the 6.2 GB written.
+// Communities beyond kInitSlice take a launch of their own: at 256 threads
+// each, 2^24 of them would be more than a launch holds.
 constexpr uint32_t kInitMembers = 4096;
-__global__ __launch_bounds__(256) void k_init(EngineView v) {
+constexpr uint32_t kInitSlice = 1u << 20;
+__global__ __launch_bounds__(256) void k_init(EngineView v, uint32_t first) {
     extern __shared__ uint32_t s_dtab[];   // mosquito lifetime thresholds
     __shared__ uint32_t s_ih[kHumanYears], s_im[kMosqInitDays], s_guide[kLifeBuckets];
     __shared__ uint32_t s_cnt[4];
-    const uint32_t g = blockIdx.x, part = blockIdx.y, parts = gridDim.y, tid = threadIdx.x;
+    const uint32_t g = first + blockIdx.x, part = blockIdx.y, parts = gridDim.y, tid = threadIdx.x;
     const CommDesc cd = v.comm[g];
     if (part * kInitMembers >= cd.n && part * kInitMembers >= cd.cap) return;   // workgroup-uniform
     const SimDesc& sd = v.sims[cd.sim];
@@ -1985,7 +1988,10 @@ hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
     if (most < 1) most = 1;
     if (parts > most) parts = most;
     if (parts < 1) parts = 1;
-    hipLaunchKernelGGL(k_init, dim3(v.n_comm, parts), dim3(256), (size_t)v.death_m_lds * 4, st, v);
+    for (uint32_t g = 0; g < v.n_comm; g += kInitSlice) {
+        const uint32_t n = v.n_comm - g < kInitSlice ? v.n_comm - g : kInitSlice;
+        hipLaunchKernelGGL(k_init, dim3(n, parts), dim3(256), (size_t)v.death_m_lds * 4, st, v, g);
+    }
     return hipGetLastError();
 }
 

@@ -200,3 +200,26 @@ def test_large_communities_of_small_batches(hip_lib, oracle_lib, humans, slots, 
     q = configs.base_params(n_serotypes=2, beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.02, long_distance=0.05)
     specs = [SimSpec(2, 2, np.array(humans, np.uint32), c, 31, mosq_slots=np.array(slots, np.uint32)) for c in (p, q)]
     _both(hip_lib, oracle_lib, specs, 16, flags=flags, checks=(1, 6))
+
+
+@pytest.mark.parametrize("grid", [(1024, 1024), (1025, 1024), (4096, 4096)])
+def test_first_census_of_many_communities(hip_lib, oracle_lib, grid):
+    """As many communities as one launch of the t = 0 census takes, one row
+    more, and the most that a simulation may have; beyond 2^26 - 1 a batch is
+    refused."""
+    print(f"[edges] communities {grid}", flush=True)
+    p = configs.base_params(n_serotypes=2, seed_frac_h=0.1, seed_frac_m=0.1, neighbourhood=4)
+    spec = SimSpec(*grid, np.ones(grid[0] * grid[1], np.uint32), p, 5)
+    gpu, orc = Engine(hip_lib), Engine(oracle_lib, threads=8)
+    for e in (orc, gpu):
+        e.init([spec], 1)
+        e.step(1)
+        print("[edges] stepped", flush=True)
+    _compare_series(gpu.series(0), orc.series(0), "series")
+    if grid != (4096, 4096):
+        _compare_state(gpu.state(0), orc.state(0), "state")
+    else:
+        with pytest.raises(RuntimeError, match="communities"):
+            gpu.init([spec] * 4, 1)
+    gpu.close()
+    orc.close()
