@@ -344,6 +344,11 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
     p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + 1e-8f);
 }
 
+__global__ void k_copy_f32(const float* __restrict__ from, float* __restrict__ to, uint64_t n) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) to[i] = from[i];
+}
+
 __global__ void k_zero_f32(float* __restrict__ p, uint64_t n) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0.0f;
@@ -737,6 +742,14 @@ void alloc_staging(ArboSurrogate* s) {
     }
 }
 
+// Whether a pass may write rows of `out` while it has yet to read later rows
+// of `in`: n rows of each that lie apart, or in the same place and of one
+// width (a row is read before it is written).
+bool rows_apart(const float* in, size_t in_width, const float* out, size_t out_width, size_t n) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(in), b = reinterpret_cast<uintptr_t>(out);
+    return a + n * in_width * 4 <= b || b + n * out_width * 4 <= a || (a == b && in_width == out_width);
+}
+
 // Outputs, and with dout the input gradients, of n host rows.  The kernel
 // reads and writes pinned copies of the rows in place: a 64-row forward call
 // took 47.9 us through two hipMemcpyAsync of pageable rows (11 and 13 us) and
@@ -960,7 +973,8 @@ ARBO_API int arbo_sur_forward(ArboSurrogate* s, uint32_t n, const float* x, floa
     if (!s || !x || !out || n == 0) return ARBO_E_INVALID;
     if (n > s->max_batch) return fail(s, ARBO_E_CAPACITY, "more rows than max_batch");
     SUR_TRY(s, hipSetDevice(s->device));
-    if (s->pin) return pass_host_rows<PASS_FORWARD>(s, n, x, nullptr, out, nullptr);
+    if (s->pin && rows_apart(x, s->w[0], out, s->w[s->L], n))
+        return pass_host_rows<PASS_FORWARD>(s, n, x, nullptr, out, nullptr);
     if (int rc = upload_x(s, n, x)) return rc;
     if (s->fused) {
         PassArgs a = pass_args(s, PASS_FORWARD, n);
@@ -983,7 +997,21 @@ ARBO_API int arbo_sur_forward_noalloc(ArboSurrogate* s, uint32_t n, const float*
     if (!s->scratch) return fail(s, ARBO_E_STATE, "no scratch address on this device");
     SUR_TRY(s, hipSetDevice(s->device));
     const hipStream_t st = stream ? static_cast<hipStream_t>(stream) : s->stream;
-    if (s->fused) {   // the activations stay on chip
+    bool fused = s->fused;
+    if (fused && !rows_apart(x, s->w[0], out, s->w[s->L], n)) {
+        // a tile's results would land on rows that others have yet to read:
+        // the inputs go to the scratch first, or the products below, the
+        // first of which reads all rows, take them
+        const uint64_t nx = (uint64_t)n * s->w[0];
+        if (nx <= 2 * kScratchElems) {
+            hipLaunchKernelGGL(k_copy_f32, dim3(blocks(nx, 256)), dim3(256), 0, st, x, s->scratch, nx);
+            SUR_TRY(s, hipGetLastError());
+            x = s->scratch;
+        } else {
+            fused = false;
+        }
+    }
+    if (fused) {   // the activations stay on chip
         PassArgs a = pass_args(s, PASS_FORWARD, n);
         a.x = x;
         a.out = out;
@@ -1019,7 +1047,10 @@ ARBO_API int arbo_sur_input_grad(ArboSurrogate* s, uint32_t n, const float* x, c
     if (!s || !x || !dout || !dx || n == 0) return ARBO_E_INVALID;
     if (n > s->max_batch) return fail(s, ARBO_E_CAPACITY, "more rows than max_batch");
     SUR_TRY(s, hipSetDevice(s->device));
-    if (s->pin) return pass_host_rows<PASS_INPUT>(s, n, x, dout, out, dx);
+    const size_t wx = s->w[0], wy = s->w[s->L];
+    if (s->pin && rows_apart(x, wx, dx, wx, n) && rows_apart(dout, wy, dx, wx, n) &&
+        (!out || (rows_apart(x, wx, out, wy, n) && rows_apart(dout, wy, out, wy, n) && rows_apart(out, wy, dx, wx, n))))
+        return pass_host_rows<PASS_INPUT>(s, n, x, dout, out, dx);
     if (int rc = upload_x(s, n, x)) return rc;
     const uint64_t no = (uint64_t)n * s->w[s->L];
     if (s->fused) {

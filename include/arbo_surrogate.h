@@ -10,7 +10,8 @@
  * Every matrix product runs on the bfloat16 MFMA units with float32
  * accumulation, each float32 operand split into two bfloat16 halves (three
  * products per step: about 16 significant bits per operand); parameters,
- * activations, gradients and the optimiser state are float32.
+ * outputs, gradients and the optimiser state are float32, and so are the
+ * activations, or kept as the two halves that the next product reads.
  * Host buffers are row-major float32: inputs [n * width_0], outputs
  * [n * width_last].  Parameters flatten layer by layer as W [width_{l+1} x
  * width_l] (row-major) then b [width_{l+1}].
@@ -43,7 +44,8 @@ ARBO_API int arbo_sur_shape(const ArboSurrogate* s, uint32_t* inputs, uint32_t* 
 ARBO_API int arbo_sur_get_params(ArboSurrogate* s, float* out);
 ARBO_API int arbo_sur_set_params(ArboSurrogate* s, const float* in);
 
-/* out = f(x) for n rows. */
+/* out = f(x) for n rows.  The host calls read all of their inputs before they
+ * write a result over them: out and dx may overlap x and dout. */
 ARBO_API int arbo_sur_forward(ArboSurrogate* s, uint32_t n, const float* x, float* out);
 
 /* out = f(x) for n rows on device buffers, allocating nothing.  No
@@ -51,12 +53,17 @@ ARBO_API int arbo_sur_forward(ArboSurrogate* s, uint32_t n, const float* x, floa
  * memory (code under HIP graph capture, tight serving loops).  x and out are
  * device pointers (x [n * width_0] float32, out [n * width_last] float32);
  * the work is queued on `stream` (a hipStream_t; NULL: the surrogate's own
- * stream) and the call returns without waiting.  The activations between
- * layers live in a fixed 8 MiB scratch array of the library on each GPU
- * (two buffers of 2^20 float32), so n x (the widest hidden layer) must not
- * exceed 2^20 (4,096 rows of a 256-wide network), else ARBO_E_CAPACITY;
- * every call on one GPU shares that array, so calls that overlap on one GPU
- * race.  The results are those of arbo_sur_forward, bit for bit. */
+ * stream) and the call returns without waiting.  The library has a fixed
+ * 8 MiB scratch array on each GPU (two buffers of 2^20 float32), and n x (the
+ * widest hidden layer) must not exceed 2^20 (4,096 rows of a 256-wide
+ * network), else ARBO_E_CAPACITY.  Networks with a layer above 512, or too
+ * deep for a CU's LDS, keep the activations between layers there; the others
+ * keep them on chip and use it only where x and out overlap, for a copy of x.
+ * Every call on one GPU shares that array, so calls that use it and overlap in
+ * time on one GPU race.  out may overlap x (networks of two layers or more).
+ * The results are those of arbo_sur_forward, bit for bit; only where the two
+ * overlap, n x width_0 exceeds 2^21 and the activations would stay on chip are
+ * they rounded otherwise. */
 ARBO_API int arbo_sur_forward_noalloc(ArboSurrogate* s, uint32_t n, const float* x, float* out, void* stream);
 
 /* out = f(x) and dx = (d f / d x)^T dout, row by row. */

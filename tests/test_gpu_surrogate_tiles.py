@@ -11,6 +11,8 @@ them: 10 * 1.2e-5 * 4 = 5e-4, tested at 1e-3.  An Adam update from zero
 moments is lr * sign(g) to leading order, so entries within the gradient's
 error of zero may take either sign: a fraction below 1e-3 of them, each
 twice the update, sqrt(4 * 1e-3) = 0.063 of the update's norm, tested at 0.1."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -180,3 +182,69 @@ def test_epochs_take_their_own_row_orders(hip_lib, widths):
         got.append(s.get_params())
         s.close()
     assert np.array_equal(got[0], got[1])
+
+
+def _place(kind, n_in, n_out):
+    """Element offsets of an input and an output of n_in and n_out elements
+    that overlap, and the buffer's size."""
+    at = {"output first": (n_out // 3, 0), "input first": (0, n_in // 2), "same start": (0, 0)}[kind]
+    return *at, max(at[0] + n_in, at[1] + n_out)
+
+
+OVERLAPS = ["output first", "input first", "same start"]
+
+
+@pytest.mark.parametrize("kind", OVERLAPS)
+@pytest.mark.parametrize("widths,n", [([6, 64, 64, 20], 4000), ([20, 33, 20], 2500), ([200, 16, 16, 30], 12000),
+                                      ([6, 520, 30], 300)],
+                         ids=lambda w: "-".join(map(str, w)) if isinstance(w, list) else None)
+def test_results_over_the_inputs(hip_lib, widths, n, kind):
+    """Calls whose results lie over their inputs give what they give apart
+    from them: rows of several chunks, of one width and of two, and more
+    inputs than the scratch holds (products of other rounding)."""
+    print(f"[tiles] overlap {kind} {widths}", flush=True)
+    hip = Hip()
+    f32p = ctypes.POINTER(ctypes.c_float)
+    s = Surrogate(widths, max_batch=n, seed=7, lib=hip_lib)
+    rng = np.random.default_rng(8)
+    x = rng.normal(size=(n, widths[0])).astype(np.float32)
+    dout = rng.normal(size=(n, widths[-1])).astype(np.float32)
+    want, want_dx = s.input_grad(x, dout)
+    at_x, at_o, size = _place(kind, x.size, want.size)
+
+    def ptr(a, at):
+        return a[at:].ctypes.data_as(f32p)
+    buf = np.zeros(size, np.float32)
+    buf[at_x:at_x + x.size] = x.ravel()
+    assert s.lib.arbo_sur_forward(s._h, n, ptr(buf, at_x), ptr(buf, at_o)) == 0
+    assert np.array_equal(buf[at_o:at_o + want.size], want.ravel())
+
+    dev = hip.upload(np.concatenate([np.zeros(at_x, np.float32), x.ravel(),
+                                     np.zeros(size - at_x - x.size, np.float32)]))
+    base = dev.value
+    assert s.lib.arbo_sur_forward_noalloc(s._h, n, ctypes.c_void_p(base + 4 * at_x), ctypes.c_void_p(base + 4 * at_o), None) == 0
+    hip.check(hip.lib.hipDeviceSynchronize(), "hipDeviceSynchronize")
+    got = hip.download(dev, (size,))[at_o:at_o + want.size]
+    if n * widths[0] > 1 << 21 and not (at_x == at_o and widths[0] == widths[-1]):
+        assert rel(got, want) < 1e-4
+    else:
+        assert np.array_equal(got, want.ravel())
+    hip.check(hip.lib.hipFree(dev), "hipFree")
+
+    # the gradient in the inputs' place and the outputs in dout's, outputs over
+    # the inputs, the gradient over dout
+    buf = np.zeros(size, np.float32)
+    buf[at_x:at_x + x.size] = x.ravel()
+    y = dout.ravel().copy()
+    assert s.lib.arbo_sur_input_grad(s._h, n, ptr(buf, at_x), ptr(y, 0), ptr(y, 0), ptr(buf, at_x)) == 0
+    assert np.array_equal(y, want.ravel()) and np.array_equal(buf[at_x:at_x + x.size], want_dx.ravel())
+    buf[at_x:at_x + x.size] = x.ravel()
+    dx = np.empty_like(x)
+    assert s.lib.arbo_sur_input_grad(s._h, n, ptr(buf, at_x), ptr(dout.ravel(), 0), ptr(buf, at_o), ptr(dx.ravel(), 0)) == 0
+    assert np.array_equal(buf[at_o:at_o + want.size], want.ravel()) and np.array_equal(dx, want_dx)
+    at_y, at_d, size = _place(kind, want.size, x.size)
+    buf = np.zeros(size, np.float32)
+    buf[at_y:at_y + want.size] = dout.ravel()
+    assert s.lib.arbo_sur_input_grad(s._h, n, ptr(x.ravel(), 0), ptr(buf, at_y), None, ptr(buf, at_d)) == 0
+    assert np.array_equal(buf[at_d:at_d + x.size], want_dx.ravel())
+    s.close()
