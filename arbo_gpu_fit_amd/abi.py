@@ -114,6 +114,8 @@ PROTOTYPES = {
     "arbo_tuning_candidates": (C.c_int, [C.POINTER(Tuning), _u32, _u32p]),
     "arbo_set_tuning": (C.c_int, [EnginePtr, C.POINTER(Tuning)]),
     "arbo_get_tuning": (C.c_int, [EnginePtr, C.POINTER(Tuning)]),
+    "arbo_update_tuning": (C.c_int, [EnginePtr, C.POINTER(Tuning), _u32]),
+    "arbo_launch_shape": (C.c_int, [EnginePtr, _u32p, _u32p]),
     "arbo_autotune": (C.c_int, [EnginePtr, _u32, C.POINTER(Tuning), C.POINTER(C.c_double)]),
     "arbo_destroy": (None, [EnginePtr]),
     "arbo_last_error": (C.c_char_p, [EnginePtr]),

@@ -201,7 +201,7 @@ struct Tuning {
     uint32_t ld_split;   // long-distance kernel: workgroups per simulation
     uint32_t wps;        // demography: 0 the compiler's register budget, 8 eight waves per SIMD
     uint32_t nw;         // demography: waves per community (1, 2, 4)
-    bool chosen;         // set or autotuned; the default leaves a small batch's waves per community to the launch
+    bool chosen;         // nw was set, or found on a small batch; else a small batch's is left to the launch
 };
 constexpr uint32_t kDemographyShapes[][2] = {{4, 4}, {4, 2}, {8, 4}, {2, 2}};   // (unroll, early_m)
 constexpr uint32_t kOccShapes[][2] = {{4, 2}, {2, 2}};   // shapes also built for 8 waves per SIMD
@@ -234,6 +234,7 @@ hipError_t launch_life_tables(uint32_t* pool, const HumanTable* humans, uint32_t
                               const MosquitoTable* mosq, uint32_t n_mosq, uint32_t max_rows, const double* scales,
                               hipStream_t st);
 hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st);
+uint32_t demography_waves(const EngineView& v, const Tuning& tu);   // waves per community that it launches
 hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_longdist(const EngineView& v, const Tuning& tu, hipStream_t st);

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <map>
 #include <string>
@@ -652,9 +653,34 @@ int arbo_tuning_candidates(ArboTuning* out, uint32_t cap, uint32_t* n) {
     return ARBO_OK;
 }
 
-int arbo_set_tuning(ArboEngine* e, const ArboTuning* t) {
+constexpr uint32_t kTuningFields = sizeof(ArboTuning) / sizeof(uint32_t);
+constexpr uint32_t kWavesField = 1u << (offsetof(ArboTuning, waves_per_comm) / sizeof(uint32_t));
+
+int arbo_update_tuning(ArboEngine* e, const ArboTuning* t, uint32_t fields) {
     if (!e || !t) return ARBO_E_INVALID;
-    return apply_tuning(e, from_abi(*t));
+    if (fields >> kTuningFields) return fail(e, ARBO_E_INVALID, "no such member of the tuning");
+    uint32_t now[kTuningFields], given[kTuningFields];
+    ArboTuning all = to_abi(e->tuning);
+    std::memcpy(now, &all, sizeof all);
+    std::memcpy(given, t, sizeof all);
+    for (uint32_t i = 0; i < kTuningFields; ++i)
+        if ((fields >> i) & 1u) now[i] = given[i];
+    std::memcpy(&all, now, sizeof all);
+    Tuning tu = from_abi(all);
+    tu.chosen = e->tuning.chosen || (fields & kWavesField) != 0;
+    return apply_tuning(e, tu);
+}
+
+int arbo_set_tuning(ArboEngine* e, const ArboTuning* t) {
+    return arbo_update_tuning(e, t, (1u << kTuningFields) - 1u);
+}
+
+int arbo_launch_shape(const ArboEngine* e, uint32_t* small_batch, uint32_t* waves_per_comm) {
+    if (!e) return ARBO_E_INVALID;
+    if (!e->ready) return ARBO_E_STATE;
+    if (small_batch) *small_batch = e->view.small;
+    if (waves_per_comm) *waves_per_comm = demography_waves(e->view, e->tuning);
+    return ARBO_OK;
 }
 
 int arbo_get_tuning(const ArboEngine* e, ArboTuning* out) {
@@ -679,6 +705,7 @@ int arbo_autotune(ArboEngine* e, uint32_t days_each, ArboTuning* chosen, double*
     // bracket the demography kernel and the rest of the day; the demography
     // knobs come from the candidate with the least demography time, the event
     // kernel's order bit from the one with the least rest-of-day time.
+    const Tuning before = e->tuning;
     const uint32_t ne = 3 * n;
     std::vector<hipEvent_t> ev(ne, nullptr);
     int rc = ARBO_OK;
@@ -721,11 +748,37 @@ int arbo_autotune(ArboEngine* e, uint32_t days_each, ArboTuning* chosen, double*
         (void)rc2;
         return rc;
     }
+    double best = ta[ka] + tb[kb];
     Tuning keep = from_abi(cand[ka]);
     keep.xcd = (keep.xcd & 1u) | (cand[kb].xcd_order & 2u);
+    keep.chosen = before.chosen;   // what suits a large batch says nothing of a small one's waves
+    if (e->view.small) {
+        // Only the waves per community differ: the candidates that share them
+        // are one kernel, timed together, and their other knobs stay as they
+        // were.  With one number of waves for all (bitmaps that need eight)
+        // there is nothing to choose.
+        std::map<uint32_t, std::pair<double, uint32_t>> by_waves;   // time and candidates
+        double rest = 0.0;
+        for (uint32_t k = 0; k < n; ++k) {
+            auto& w = by_waves[demography_waves(e->view, from_abi(cand[k]))];
+            w.first += ta[k];
+            w.second++;
+            rest += tb[k];
+        }
+        auto mean = [](const std::pair<double, uint32_t>& w) { return w.first / w.second; };
+        uint32_t waves = by_waves.begin()->first;
+        for (const auto& w : by_waves)
+            if (mean(w.second) < mean(by_waves[waves])) waves = w.first;
+        best = mean(by_waves[waves]) + rest / n;
+        keep = before;
+        if (by_waves.size() > 1) {
+            keep.chosen = true;
+            for (uint32_t k = 0; k < n && demography_waves(e->view, keep) != waves; ++k) keep = from_abi(cand[k]);
+        }
+    }
     if ((rc = apply_tuning(e, keep))) return rc;
     if (chosen) *chosen = to_abi(keep);
-    if (ms_per_day) *ms_per_day = (ta[ka] + tb[kb]) / days_each;
+    if (ms_per_day) *ms_per_day = best / days_each;
     return ARBO_OK;
 }
 

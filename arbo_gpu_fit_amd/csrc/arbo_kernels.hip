@@ -2005,12 +2005,15 @@ hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
 // better than four up to 400 communities and slower from 484 on.
 constexpr uint32_t kWideCommunities = 1024;
 
+uint32_t demography_waves(const EngineView& v, const Tuning& tu) {
+    if (v.max_words > kWaveWords * tu.nw) return kMaxWaves;   // a community's bitmap needs more than the tuning's
+    return v.small && !tu.chosen && v.n_comm <= kWideCommunities ? 4u : tu.nw;
+}
+
 template <bool HIST>
 static hipError_t launch_demography_small(const EngineView& v, const Tuning& tu, hipStream_t st) {
     const size_t lds = (size_t)v.death_m_lds * 4;
-    uint32_t nw = tu.nw;
-    if (v.max_words > kWaveWords * nw) nw = kMaxWaves;   // a community's bitmap needs more waves than the tuning's
-    else if (!tu.chosen && v.n_comm <= kWideCommunities) nw = 4;
+    const uint32_t nw = demography_waves(v, tu);
     const dim3 grid(v.n_comm), block(kWave * nw);
     if (nw == 1) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 1, true>), grid, block, lds, st, v);
     else if (nw == 2) hipLaunchKernelGGL((k_day_demography<4, 2, false, HIST, 0, 2, true>), grid, block, lds, st, v);
@@ -2026,7 +2029,7 @@ static hipError_t launch_demography_small(const EngineView& v, const Tuning& tu,
 template <bool XCD, bool HIST>
 static hipError_t launch_demography_xh(const EngineView& v, const Tuning& tu, hipStream_t st) {
     const size_t lds = (size_t)v.death_m_lds * 4;
-    if (v.max_words > kWaveWords * tu.nw) {   // a community's bitmap needs more waves than the tuning's
+    if (demography_waves(v, tu) == kMaxWaves) {
         hipLaunchKernelGGL((k_day_demography<2, 2, false, HIST, 0, kMaxWaves>), dim3(v.n_comm),
                            dim3(kWave * kMaxWaves), lds, st, v);
         return hipGetLastError();

@@ -266,13 +266,19 @@ class Engine:
         return [t.as_dict() for t in arr]
 
     def set_tuning(self, **knobs):
-        """Set launch knobs (census_unroll, early_mosq, xcd_order, ld_split);
-        unnamed knobs keep their values.  Results never depend on them."""
-        t = abi.Tuning()
-        self._check(self.lib.arbo_get_tuning(self._h, C.byref(t)))
-        for k, v in knobs.items():
-            setattr(t, k, v)
-        self._check(self.lib.arbo_set_tuning(self._h, C.byref(t)))
+        """Set launch knobs (census_unroll, early_mosq, xcd_order, ld_split,
+        waves_per_simd, waves_per_comm); unnamed knobs keep their values, or
+        stay the engine's to choose.  Results never depend on them."""
+        t = abi.Tuning(**knobs)
+        fields = sum(1 << i for i, (name, _) in enumerate(t._fields_) if name in knobs)
+        self._check(self.lib.arbo_update_tuning(self._h, C.byref(t), fields))
+
+    def launch_shape(self) -> dict:
+        """Whether the batch is a small one, and the waves per community of its
+        demography kernel."""
+        small, waves = C.c_uint32(), C.c_uint32()
+        self._check(self.lib.arbo_launch_shape(self._h, C.byref(small), C.byref(waves)))
+        return {"small_batch": bool(small.value), "waves_per_comm": waves.value}
 
     def tuning(self) -> dict:
         t = abi.Tuning()

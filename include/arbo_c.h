@@ -281,9 +281,9 @@ ARBO_API int arbo_scan_counts(ArboEngine* e, uint64_t* human_vectors, uint64_t* 
  * event), never by workgroup or lane, so runs under any tuning are
  * bit-identical.  Small batches (up to 4,096 communities, 512 in a simulation)
  * have one kernel shape per waves_per_comm, no long-distance kernel and no
- * order: only waves_per_comm acts there, and until a tuning is set the engine
- * gives communities of such a batch four waves where that is the faster.  No
- * counterpart in the reference, whose launch shapes come from the device
+ * order: only waves_per_comm acts there, and until it is set, or found by
+ * arbo_autotune on a small batch, the engine gives communities of such a batch
+ * four waves where that is the faster.  No counterpart in the reference, whose launch shapes come from the device
  * properties (cudaidentities.h:14-37). */
 typedef struct ArboTuning {
     uint32_t census_unroll;   /* demography kernel: 16-byte census loads in flight per lane (2, 4, 8) */
@@ -304,12 +304,19 @@ ARBO_API int arbo_tuning_candidates(ArboTuning* out, uint32_t cap, uint32_t* n);
  * combination the library was not built with. */
 ARBO_API int arbo_set_tuning(ArboEngine* e, const ArboTuning* t);
 ARBO_API int arbo_get_tuning(const ArboEngine* e, ArboTuning* out);
+/* Set the members of *t whose bit is set in `fields` (bit i: member i, from 0)
+ * and leave the others as they are, set or not. */
+ARBO_API int arbo_update_tuning(ArboEngine* e, const ArboTuning* t, uint32_t fields);
+/* What the batch's days launch under the tuning: whether it is a small batch
+ * (0 or 1), and the waves of a community in the demography kernel, 8 where its
+ * bitmap needs them.  Either may be NULL; ARBO_E_STATE before arbo_batch_init. */
+ARBO_API int arbo_launch_shape(const ArboEngine* e, uint32_t* small_batch, uint32_t* waves_per_comm);
 /* Time every candidate on the engine's own batch for days_each days each
  * (those days are simulated: the run advances by candidates x days_each days,
  * with the same results as under any fixed tuning; the candidates take turns
  * a day at a time, forward and backward in alternate rounds) and keep the
- * fastest demography knobs and the fastest event-kernel order; ms_per_day
- * gets the sum of their day times.  chosen and ms_per_day may be NULL. */
+ * fastest demography knobs and the fastest event-kernel order (small batches:
+ * the fastest waves_per_comm); ms_per_day gets the sum of their day times.  chosen and ms_per_day may be NULL. */
 ARBO_API int arbo_autotune(ArboEngine* e, uint32_t days_each, ArboTuning* chosen, double* ms_per_day);
 
 ARBO_API void arbo_destroy(ArboEngine* e);

@@ -1135,6 +1135,27 @@ int arbo_set_tuning(ArboEngine* e, const ArboTuning* t) {
     return ARBO_OK;
 }
 
+int arbo_update_tuning(ArboEngine* e, const ArboTuning* t, uint32_t fields) {
+    if (!e || !t || fields > 63u) return ARBO_E_INVALID;
+    ArboTuning all = e->tuning;
+    uint32_t* const to[6] = {&all.census_unroll, &all.early_mosq, &all.xcd_order,
+                             &all.ld_split, &all.waves_per_simd, &all.waves_per_comm};
+    const uint32_t from[6] = {t->census_unroll, t->early_mosq, t->xcd_order,
+                              t->ld_split, t->waves_per_simd, t->waves_per_comm};
+    for (int i = 0; i < 6; ++i)
+        if ((fields >> i) & 1u) *to[i] = from[i];
+    return arbo_set_tuning(e, &all);
+}
+
+// No launches here: one thread's view of a large batch.
+int arbo_launch_shape(const ArboEngine* e, uint32_t* small_batch, uint32_t* waves_per_comm) {
+    if (!e) return ARBO_E_INVALID;
+    if (!e->ready) return ARBO_E_STATE;
+    if (small_batch) *small_batch = 0;
+    if (waves_per_comm) *waves_per_comm = 1;
+    return ARBO_OK;
+}
+
 int arbo_get_tuning(const ArboEngine* e, ArboTuning* out) {
     if (!e || !out) return ARBO_E_INVALID;
     *out = e->tuning;

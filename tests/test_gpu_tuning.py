@@ -5,11 +5,13 @@ mosquito loads, XCD-contiguous community order, 8 waves per SIMD, several
 waves per community) and the extremes of the
 long-distance split give the oracle's census and series bit for bit, and an
 autotuned run, graph replay included, equals an untuned one."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from arbo_gpu_fit_amd import abi
-from arbo_gpu_fit_amd.engine import Engine
+from arbo_gpu_fit_amd import abi, configs
+from arbo_gpu_fit_amd.engine import Engine, SimSpec
 from tests.cases import CASES
 from tests.test_gpu_parity import _compare_series, _compare_state
 
@@ -120,4 +122,69 @@ def test_large_communities_under_every_tuning(hip_lib, oracle_lib, flags):
             assert np.array_equal(gpu.spatial(0), kept[0])
             assert np.array_equal(gpu.history(0), kept[1])
             assert np.array_equal(gpu.aoi(0), kept[2])
+    gpu.close()
+
+
+def _lattice(grids, seed=40):
+    p = configs.base_params(beta_hm=0.7, beta_mh=0.7, seed_frac_h=0.05, seed_frac_m=0.05)
+    return [SimSpec(w, h, np.full(w * h, 9, np.uint32), p, seed + i) for i, (w, h) in enumerate(grids)]
+
+
+SMALL, LARGE = [(32, 16)], [(27, 19)]   # 512 communities in a simulation, and one more
+
+
+def test_waves_stay_the_engines_until_they_are_set(hip_lib):
+    """A small batch's communities keep their four waves through a tuning
+    that names other knobs, and through one found on a large batch; a named
+    number of waves holds."""
+    gpu = Engine(hip_lib, flags=abi.F_GRAPH)
+    with pytest.raises(RuntimeError):
+        gpu.launch_shape()   # no batch yet
+
+    def shape(grids):
+        gpu.init(_lattice(grids), 60)
+        return gpu.launch_shape()
+    four, one = ({"small_batch": True, "waves_per_comm": n} for n in (4, 1))
+    assert shape(SMALL) == four
+    gpu.set_tuning(ld_split=4, xcd_order=3)
+    assert gpu.launch_shape() == four and gpu.tuning()["ld_split"] == 4
+    assert shape(SMALL) == four
+    assert shape(LARGE) == {"small_batch": False, "waves_per_comm": 1}
+    chosen, _ = gpu.autotune(2)
+    assert gpu.launch_shape()["waves_per_comm"] == chosen["waves_per_comm"]
+    if chosen["waves_per_comm"] == 1:
+        assert shape(SMALL) == four
+    gpu.set_tuning(census_unroll=4, early_mosq=2, waves_per_simd=0, waves_per_comm=1)
+    assert shape(SMALL) == one
+    gpu.set_tuning(ld_split=8)
+    assert shape(SMALL) == one
+    assert shape([(32, 16), (32, 16), (1, 1)]) == one
+    gpu.close()
+    gpu = Engine(hip_lib)
+    assert shape([(32, 16), (32, 16)]) == four
+    assert shape([(32, 16), (32, 16), (1, 1)]) == one
+    gpu.set_tuning(**gpu.tuning())   # all of them named
+    assert shape(SMALL) == one
+    with pytest.raises(RuntimeError):
+        gpu.set_tuning(waves_per_comm=0)
+    assert gpu.lib.arbo_update_tuning(gpu._h, ctypes.byref(abi.Tuning()), 64) == abi.E_INVALID
+    gpu.close()
+
+
+def test_autotuning_a_small_batch_compares_its_waves(hip_lib):
+    """Candidates that are one kernel in a small batch leave the other knobs
+    as they were; a batch whose bitmaps need eight waves has nothing to
+    choose."""
+    gpu = Engine(hip_lib)
+    gpu.init(_lattice(SMALL), 60)
+    gpu.set_tuning(ld_split=16, xcd_order=1)
+    before = gpu.tuning()
+    chosen, ms = gpu.autotune(2)
+    assert chosen == gpu.tuning() and ms > 0 and gpu.day == 2 * len(gpu.tuning_candidates())
+    assert gpu.launch_shape()["waves_per_comm"] == chosen["waves_per_comm"]
+    assert chosen["waves_per_comm"] > 1 or chosen == before
+    gpu.set_tuning(**before)
+    gpu.init([SimSpec(1, 1, np.array([40000], np.uint32), configs.base_params(), 3, mosq_slots=np.array([65535], np.uint32))], 60)
+    assert gpu.launch_shape() == {"small_batch": True, "waves_per_comm": 8}
+    assert gpu.autotune(1)[0] == before
     gpu.close()
