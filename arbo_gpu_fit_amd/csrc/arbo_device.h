@@ -32,7 +32,17 @@ constexpr uint32_t kPartWords = 24;
 // Communities of a batch: a launch holds fewer than 2^32 threads, and the day
 // kernels take at least 64 a community.
 constexpr uint64_t kMaxCommunities = (1ull << 26) - 1;
-constexpr uint32_t kCountComms = 32;      // communities of a workgroup of k_day_counts
+// Communities of a workgroup of k_day_counts: 32, or fewer (4, 8, 16) while that
+// makes no more than kCountBlocks workgroups.  The 256 threads share their
+// communities' events, so fewer communities shorten an epidemic's days, and
+// the idle workgroups of quiet days cost about 11 ns each.  One simulation,
+// transmission rates 0.7, us a day with 32, 16, 8 and 4: 529 communities of
+// 2,500 humans 108.6, 93.8, 86.1, 82.3, 1,024 of 1,000 humans 70.0, 62.4,
+// 59.0, 57.5, 2,500 81.0, 75.1, 72.7, 72.7, 4,096 91.8, 86.4, 85.1, 87.2,
+// 6,400 120.4, 117.4, 116.4, 123.4; rates 0.15 and no epidemic: 1,024 36.0,
+// 35.8, 36.5, 38.0, 2,500 48.3, 48.9, 50.6, 54.7, 4,096 56.0, 57.0, 60.1, 67.3.
+constexpr uint32_t kCountComms = 32;
+constexpr uint32_t kCountBlocks = 320;
 constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this
 

@@ -323,6 +323,8 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     std::map<std::vector<float>, uint32_t> seen_f32;
     uint64_t h_tot = 0, m_tot = 0, ser_tot = 0, spa_tot = 0;
     uint32_t aoi_blocks = 0;
+    uint32_t count_comms = 4;   // communities of a workgroup of the event counts
+    while (count_comms < kCountComms && communities > (uint64_t)count_comms * kCountBlocks) count_comms *= 2;
     uint32_t max_n = 0, max_cap = 0, death_m_lds = 1;
     for (uint32_t i = 0; i < n_sims; ++i) {
         const SimTables& t = tabs[i];
@@ -441,8 +443,8 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
             max_n = std::max(max_n, cd.n);
             max_cap = std::max(max_cap, cd.cap);
         }
-        for (uint32_t c = 0; c < t.C; c += kCountComms) {
-            const uint32_t n = std::min(kCountComms, t.C - c), row = row_base + t.row_ptr[c];
+        for (uint32_t c = 0; c < t.C; c += count_comms) {
+            const uint32_t n = std::min(count_comms, t.C - c), row = row_base + t.row_ptr[c];
             count_map.push_back(CountBlock{i, c, sh.comm_off + c, n, row, t.row_ptr[c + n] - t.row_ptr[c]});
         }
         sd.aoi_block = aoi_blocks;

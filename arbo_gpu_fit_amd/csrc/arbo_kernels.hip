@@ -1707,7 +1707,7 @@ __global__ __launch_bounds__(256) void k_day_longdist(EngineView v, uint32_t spl
     longdist_part(v, sim, *v.day + v.day_offset, part, split, threadIdx.x);
 }
 
-// The communities of a day as sources, kCountComms of one simulation a
+// The communities of a day as sources, up to kCountComms of one simulation a
 // workgroup, and the sums of their partials.  Eight lanes a community draw its
 // event counts (direction and serotype each), the workgroup spreads all its
 // events' quads over its threads and pushes the counts into the destinations'
@@ -1774,7 +1774,7 @@ __global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
     }
     const bool some = __syncthreads_or((int)(sc.n | sc.stay)) != 0;
     if (some) {
-        for (uint32_t i = tid; i < kCountComms * kCntPerComm; i += 256) (&s_hist[0][0])[i] = 0u;
+        for (uint32_t i = tid; i < cb.n * kCntPerComm; i += 256) (&s_hist[0][0])[i] = 0u;
         // quads of the workgroup's segments
         uint32_t wtot;
         uint32_t q0 = wave_exclusive_scan((sc.n + 3) >> 2, wtot);

@@ -223,3 +223,19 @@ def test_first_census_of_many_communities(hip_lib, oracle_lib, grid):
             gpu.init([spec] * 4, 1)
     gpu.close()
     orc.close()
+
+
+@pytest.mark.parametrize("grids", [[(1277, 1), (1, 3)], [(1277, 1), (2, 2)], [(33, 77), (7, 1), (4, 3)], [(32, 80), (1, 1)],
+                                   [(64, 79), (32, 1), (8, 4)], [(64, 79), (5, 13)], [(3, 1), (33, 1), (31, 9), (641, 19)]])
+def test_event_counts_of_few_and_many_communities(hip_lib, oracle_lib, grids):
+    """1,280, 2,560 and 5,120 communities, up to which a workgroup of the
+    event counts takes 4, 8 and 16, and one more: blocks that end with a
+    simulation, days without and with events in them."""
+    print(f"[edges] counts {grids}", flush=True)
+    specs = []
+    for i, (w, h) in enumerate(grids):
+        over = dict(count_law=abi.COUNT_STOCH_ROUND, no_distance=0.3) if i % 2 else {}
+        p = configs.base_params(beta_hm=0.7, beta_mh=0.7, seed_frac_h=0.05 if i != 1 else 0.0, seed_frac_m=0.01,
+                                long_distance=0.05, **over)
+        specs.append(SimSpec(w, h, np.where(np.arange(w * h) % 5 == 3, 150, 6).astype(np.uint32), p, 70 + i))
+    _both(hip_lib, oracle_lib, specs, 20, checks=(2, 9))
