@@ -189,17 +189,29 @@ struct EngineView {
 };
 
 // Batches whose event kernel sums the series and draws the long-distance
-// events itself (EngineView.small).  Every community's wave then reads its
-// simulation's C partials and draws all its long-distance events, so C is
-// bounded, and so is what a simulation may send a day: about a tenth of
-// omega x humans at an epidemic's peak.  All waves have to run side by side
-// for the repeated work to cost only its latency: 4,096 communities are half
-// of the device's 8,192 one-wave slots.  A day of 100 communities takes 34.5
-// us with it for 40.2, of 289 (rings kept) 32 for 36.3, of 16 x 144 37.5 for
-// 42.6.
+// events itself (EngineView.small), which spares the day two launches.  Every
+// community's wave then reads its simulation's C partials and draws all its
+// long-distance events, so all of these are bounded; us a day with it and
+// without:
+//  * C (the sums): one simulation of 484 communities of 200 and of 1,000
+//    humans 33.1 and 34.8, 43.4 and 52.8; 529 34.7 and 35.4, 44.6 and 52.8; 676
+//    36.6 and 36.0, 47.0 and 53.8; 1,024 41.1 and 36.9, 53.4 and 55.8;
+//  * communities in all, whose waves have to run side by side for the repeated
+//    work to cost only its latency: 28 simulations of 144 communities of 200 and
+//    of 1,000 humans (4,032) 41.4 and 43.5, 68.7 and 71.2; 36 (5,184) 48.0 and
+//    48.7, 80.4 and 79.6; 44 (6,336) 55.7 and 54.1, 93.9 and 89.8;
+//  * the long-distance events: in proportion to omega, the transmission rates
+//    and the mosquitoes, sent = omega x slots x (beta_hm + beta_mh), a wave's
+//    share of them where a community has several, and times the waves per SIMD
+//    that redraw them.  100 communities of 1,000 humans at 21,000 sent 46.7 and
+//    50.3, 36,000 50.1 and 51.6, 84,000 70.4 and 51.9; 484 at 8,700 51.1 and
+//    56.2, 20,300 54.1 and 53.8, 43,600 60.8 and 56.3; 16 x 144 at 13,600 67.9
+//    and 70.7, 23,300 71.6 and 73.6, 29,200 73.8 and 74.1, 68,000 83.3 and 71.6;
+//    10 x 400 at 14,100 50.0 and 48.7, 28,100 88.9 and 84.2, 65,600 93.4 and 82.5.
 constexpr uint32_t kSmallCommunities = 4096;
 constexpr uint32_t kSmallSimulation = 512;
-constexpr float kSmallSent = 32768.0f;
+constexpr float kSmallSent = 24000.0f;
+constexpr uint32_t kSimds = 1024;   // of the device: 256 CUs of four
 
 // Launch knobs of the day kernels.  None of them changes a result: every
 // random draw is keyed by model entities, never by workgroup or lane.
@@ -246,6 +258,7 @@ hipError_t launch_life_tables(uint32_t* pool, const HumanTable* humans, uint32_t
 hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st);
 uint32_t demography_waves(const EngineView& v, const Tuning& tu);   // waves per community that it launches
 hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t st);
+uint32_t event_waves(const EngineView& v);   // waves per community of the event kernel
 hipError_t launch_events(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_longdist(const EngineView& v, const Tuning& tu, hipStream_t st);
 hipError_t launch_advance(uint32_t* day, uint32_t n, hipStream_t st);

@@ -575,9 +575,16 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     {
         uint32_t max_c = 1;
         for (const SimHost& sh : e->sims) max_c = std::max(max_c, sh.C);
-        float sent = 0.0f;   // omega x humans of the simulation that may send most
-        for (uint32_t i = 0; i < n_sims; ++i)
-            sent = std::max(sent, e->sim_desc[i].omega * (float)e->sims[i].n_humans);
+        float sent = 0.0f;   // of the simulation that may send most
+        for (uint32_t i = 0; i < n_sims; ++i) {
+            const SimDesc& sd = e->sim_desc[i];
+            float beta = sd.climate ? 0.0f : sd.beta_hm + sd.beta_mh;
+            const std::vector<float>& clim = tabs[i].clim;   // with a climate, its days' rates
+            for (size_t d = 0; d < clim.size(); d += 3) beta = std::max(beta, clim[d] + clim[d + 1]);
+            sent = std::max(sent, sd.omega * (float)e->sims[i].n_slots * beta);
+        }
+        v.small = 1u;
+        sent *= std::max(1.0f, (float)e->n_comm / (float)kSimds) / (float)event_waves(v);
         v.small = e->n_comm <= kSmallCommunities && max_c <= kSmallSimulation && sent <= kSmallSent ? 1u : 0u;
     }
 

@@ -2103,6 +2103,8 @@ hipError_t launch_demography(const EngineView& v, const Tuning& tu, hipStream_t 
 // 33.9 us a day instead of 32.0 and 4,000 of them 89.7 instead of 62.2.
 constexpr uint32_t kEventWaves = 8;
 
+uint32_t event_waves(const EngineView& v) { return v.small && v.max_words > kWaveWords ? kEventWaves : 1u; }
+
 template <bool HIST>
 static void launch_events_h(const EngineView& v, const Tuning& tu, hipStream_t st) {
     const dim3 grid(v.n_comm + (v.small ? v.n_sims : 0u)), block(kWave);
@@ -2110,7 +2112,7 @@ static void launch_events_h(const EngineView& v, const Tuning& tu, hipStream_t s
         // A small batch's large communities: eight waves each.  With one, 49
         // cities of 3,000 to 21,000 humans took 44 us a day (a chain of
         // 256-event chunks); with four 29.8, with eight 26.9.
-        if (v.small)
+        if (event_waves(v) == kEventWaves)
             hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, true, kEventWaves>), grid,
                                dim3(kEventWaves * kWave), 0, st, v);
         else hipLaunchKernelGGL((k_day_events<false, HIST, kMaxWaves, false>), grid, block, 0, st, v);

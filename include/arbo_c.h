@@ -279,9 +279,9 @@ ARBO_API int arbo_scan_counts(ArboEngine* e, uint64_t* human_vectors, uint64_t* 
 /* Launch knobs of the day kernels.  No knob changes a result: every random
  * draw is keyed by model entities (simulation, community, individual, day,
  * event), never by workgroup or lane, so runs under any tuning are
- * bit-identical.  Small batches (up to 4,096 communities, 512 in a simulation)
- * have one kernel shape per waves_per_comm, no long-distance kernel and no
- * order: only waves_per_comm acts there, and until it is set, or found by
+ * bit-identical.  Small batches (up to 4,096 communities, 512 in a simulation,
+ * and few long-distance events a day) have one kernel shape per
+ * waves_per_comm, no long-distance kernel and no order: only waves_per_comm acts there, and until it is set, or found by
  * arbo_autotune on a small batch, the engine gives communities of such a batch
  * four waves where that is the faster.  No counterpart in the reference, whose launch shapes come from the device
  * properties (cudaidentities.h:14-37). */

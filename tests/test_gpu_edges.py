@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from arbo_gpu_fit_amd import abi, configs
-from arbo_gpu_fit_amd.engine import Engine, SimSpec
+from arbo_gpu_fit_amd.engine import Engine, SimSpec, climate_day
 from tests.test_gpu_parity import _compare_series, _compare_state
 
 pytestmark = pytest.mark.gpu
@@ -239,3 +239,40 @@ def test_event_counts_of_few_and_many_communities(hip_lib, oracle_lib, grids):
                                 long_distance=0.05, **over)
         specs.append(SimSpec(w, h, np.where(np.arange(w * h) % 5 == 3, 150, 6).astype(np.uint32), p, 70 + i))
     _both(hip_lib, oracle_lib, specs, 20, checks=(2, 9))
+
+
+@pytest.mark.parametrize("grids,humans,big", [([(10, 10)], 300, 0), ([(32, 16)], 40, 0), ([(32, 16)] * 5 + [(3, 1)], 9, 0),
+                                              ([(2, 2)], 2000, 12000)])
+@pytest.mark.parametrize("climate", [False, True])
+def test_small_batches_by_what_they_send(hip_lib, oracle_lib, grids, humans, big, climate):
+    """omega x slots x the transmission rates, times the waves per SIMD that
+    draw the events or over the waves of a community that share them, up to
+    24,000 and above it; with a climate the days' largest rates count."""
+    T = 15
+    cl = configs.seasonal_climate(T + 1, biting_rate=6.0) if climate else None
+    n_comm = sum(w * h for w, h in grids)
+
+    def specs(omega):
+        out = []
+        for i, (w, h) in enumerate(grids):
+            n = np.full(w * h, humans, np.uint32)
+            n[0] += big
+            p = configs.base_params(beta_hm=2.0, beta_mh=1.5, seed_frac_h=0.05, seed_frac_m=0.05, long_distance=omega)
+            out.append(SimSpec(w, h, n, p, 60 + i, climate=cl))
+        return out
+    gpu = Engine(hip_lib)
+    gpu.init(specs(0.0), T)
+    beta = 3.5
+    if climate:
+        beta = max(sum(climate_day(cl, r, oracle_lib)[:2]) for r in range(1, T + 1))
+    waves = 8 if gpu.launch_shape()["waves_per_comm"] == 8 else 1
+    assert waves == (8 if big else 1) and gpu.launch_shape()["small_batch"]
+    slots = max(gpu.sizes(i)[2] for i in range(len(grids)))
+    limit = 24000.0 * waves / (slots * beta * max(1.0, n_comm / 1024))
+    print(f"[edges] sends {grids[:2]} {climate} omega {limit:.3f}", flush=True)
+    assert limit * 1.01 < 1.0
+    for omega, small in ((limit * 0.99, True), (limit * 1.01, False)):
+        gpu.init(specs(omega), T)
+        assert gpu.launch_shape()["small_batch"] == small
+        _both(hip_lib, oracle_lib, specs(omega), T, checks=(4,))
+    gpu.close()
