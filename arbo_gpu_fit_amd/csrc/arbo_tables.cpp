@@ -81,11 +81,17 @@ static std::string validate_climate(const ArboClimate& c, uint32_t max_days) {
     return std::string();
 }
 
-// The first age from 1 whose threshold is 2^24, at most the table's last.
-template <class Cdf>
-static uint32_t first_certain(Cdf cdf) {
-    uint32_t a = 1;
-    while (a < kMosqAgeTable - 1 && fixed24(cdf((double)a)) < kOne24) ++a;
+// The first age from 1 whose threshold under a Weibull scale is 2^24, at most
+// the table's last: where the hazard (a / scale)^shape takes exp(-hazard)
+// below the last bit of 1, at 54 log 2, `ratio` scales; the ages about there
+// are evaluated.
+static uint32_t certain_age(double scale, double shape, double ratio) {
+    const uint32_t last = kMosqAgeTable - 1;
+    auto certain = [&](uint32_t a) { return fixed24(weibull_cdf((double)a, scale, shape)) >= kOne24; };
+    const double guess = ratio * scale;
+    uint32_t a = guess < (double)last ? std::max(1u, (uint32_t)guess) : last;
+    while (a > 1 && certain(a - 1)) --a;
+    while (a < last && !certain(a)) ++a;
     return a;
 }
 
@@ -266,24 +272,36 @@ static void build_network(const ArboParams& p, SimTables& t) {
 // F(a; scale(b + a)) reaches its PLE (mdemographic.cu:72 with the day's
 // mScaleLifeExpectancy); the running maximum over a of those thresholds turns
 // that first passage into a search of a monotone row.  Days past the run use
-// the last day's scale.  Every such row reaches 2^24 no later than F of the
-// run's largest scale does; one more day covers the rounding of F.
+// the last day's scale.  A row reaches 2^24 on the first day d whose certain
+// age the mosquito has by then, d - b >= age(d); since d - age(d) >= b + 1
+// implies >= b, that day never falls from one b to the next, so one walk over
+// the days finds them all.  The largest such age sizes the rows, which every
+// community stages in LDS daily: the certain age of the run's largest scale is
+// no more than a bound (2,047 days for 1,400 under the seasonal climate's 37 to
+// 74 days, exponential lifetimes).
 static void size_mosquito_rows(const ArboShape& sh, const ArboParams& p, uint32_t max_days, SimTables& t) {
     t.m_rows = 1;
-    t.death_m_max = first_certain([&](double a) { return mosq_cdf(p, a); });
+    const double shape = (double)p.m_shape, ratio = powd(37.43, 1.0 / shape);   // 54 log 2
+    t.death_m_max = certain_age((double)p.m_scale, shape, ratio);
     t.scale.clear();
     if (!t.climate) return;
     t.m_rows = max_days + 1;
     t.scale.resize(max_days);
-    double smax = 0.0;
+    std::vector<uint32_t> age(max_days);
     for (uint32_t d = 0; d < max_days; ++d) {
         double x[4];
         climate_day(*sh.climate, d + 1, x);
         t.scale[d] = x[3];
-        smax = std::max(smax, x[3]);
+        age[d] = certain_age(x[3], shape, ratio);
     }
-    const uint32_t last = first_certain([&](double a) { return weibull_cdf(a, smax, (double)p.m_shape); });
-    t.death_m_max = std::max(t.death_m_max, std::min(last + 1, kMosqAgeTable - 1));
+    const uint32_t end = max_days - 1;
+    uint32_t d = 0, most = 1;
+    for (uint32_t b = 0; b < max_days; ++b) {
+        d = std::max(d, b + 1);
+        while (d < end && d - b < age[d]) ++d;
+        most = std::max(most, d < end ? d - b : std::max(d - b, age[end]));
+    }
+    t.death_m_max = std::max(t.death_m_max, std::min(most, kMosqAgeTable - 1));
 }
 
 void build_tables(const ArboShape& sh, const ArboParams& p, uint64_t seed, uint32_t max_days,
