@@ -74,9 +74,50 @@ int main() {
 """
 
 
-def test_rows_are_as_long_as_their_ages(tmp_path):
+# Scales whose certain age lies at a whole day, and the floats about them.
+WHOLE_DAYS = r"""
+#include <cmath>
+#include <cstdio>
+#include "arbo_tables.h"
+#include "arbo_rng.h"
+using namespace arbo;
+
+int main() {
+    int checked = 0, bad = 0;
+    ArboParams p{};
+    p.n_serotypes = 1; p.neighbourhood = 4; p.include_self = 1; p.iip_min = 4; p.iip_max = 7;
+    p.recovery = 5.0f; p.eip = 10.0f; p.h_scale = 27000.0f; p.h_shape = 6.0f; p.m_ratio = 2.0f;
+    const uint32_t humans[1] = {10};
+    ArboShape sh{};
+    sh.grid_w = sh.grid_h = 1; sh.humans = humans;
+    for (float shape : {0.04f, 0.1f, 0.6f, 1.0f, 4.0f, 11.0f, 99.0f, 400.0f})
+        for (uint32_t age : {1u, 2u, 3u, 17u, 150u, 1000u, 2045u, 2046u, 2047u, 2048u, 5000u}) {
+            float scale = (float)(age / pow(54.0 * log(2.0), 1.0 / (double)shape));
+            for (int k = 0; k < 4; ++k) scale = nextafterf(scale, 0.0f);
+            for (int k = -4; k <= 4; ++k, scale = nextafterf(scale, 1e30f)) {
+                if (!(scale > 0.0f)) continue;
+                p.m_shape = shape;
+                p.m_scale = scale;
+                SimTables t;
+                build_tables(sh, p, 1, 1, t);
+                uint32_t want = 1;
+                while (want < kMosqAgeTable - 1 && fixed24(weibull_cdf((double)want, (double)scale, (double)shape)) < kOne24) ++want;
+                ++checked;
+                if (t.death_m_max != want) {
+                    ++bad;
+                    printf("shape %g scale %.9g: %u, tabulated %u\n", shape, scale, t.death_m_max, want);
+                }
+            }
+        }
+    printf("%d checked, %d differ\n", checked, bad);
+    return bad != 0;
+}
+"""
+
+
+def _run(tmp_path, program):
     src, exe = tmp_path / "rows.cpp", tmp_path / "rows"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     csrc = os.path.join(ROOT, "arbo_gpu_fit_amd", "csrc")
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(build.hipcc())))
     subprocess.run(["g++", "-std=c++17", "-O2", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"),
@@ -85,3 +126,11 @@ def test_rows_are_as_long_as_their_ages(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     print(out.stdout)
     assert out.returncode == 0, out.stdout
+
+
+def test_rows_are_as_long_as_their_ages(tmp_path):
+    _run(tmp_path, PROGRAM)
+
+
+def test_ages_certain_at_a_whole_day(tmp_path):
+    _run(tmp_path, WHOLE_DAYS)
