@@ -376,7 +376,8 @@ struct Buf {
 // surrogate is created there.
 constexpr size_t kScratchElems = size_t(1) << 20;
 constexpr size_t kPinBytes = size_t(16) << 20;   // pinned host rows of a surrogate, at most
-constexpr uint32_t kPinChunk = 1024;             // rows of a host call's pass: results are copied out a chunk behind
+constexpr size_t kPinChunkBytes = size_t(1) << 20;   // of the wider of a chunk's inputs and outputs (chunk_rows)
+constexpr size_t kCopyBytes = size_t(2) << 20;   // inputs of a forward call that are copied to the device (see there)
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) float scratch[2 * kScratchElems];
 
@@ -750,11 +751,21 @@ bool rows_apart(const float* in, size_t in_width, const float* out, size_t out_w
     return a + n * in_width * 4 <= b || b + n * out_width * 4 <= a || (a == b && in_width == out_width);
 }
 
+// Rows of a host call's pass: results are copied out a chunk behind.  Every
+// chunk costs a launch and a wait, so its size goes by its bytes: with 1,024
+// rows whatever their width, 16,384 rows of 6-256-256-20 took 245 us and
+// 65,536 of 2-16-16-3 631, in chunks of 1 MB 97 and 89 (before host rows were
+// pinned 212 and 132).
+uint32_t chunk_rows(const ArboSurrogate* s) {
+    const size_t widest = std::max(s->w[0], s->w[s->L]);
+    return (uint32_t)(kPinChunkBytes / (4 * widest) / kFuseRows * kFuseRows);   // 512 or more: kFuseWidth
+}
+
 // Outputs, and with dout the input gradients, of n host rows.  The kernel
 // reads and writes pinned copies of the rows in place: a 64-row forward call
 // took 47.9 us through two hipMemcpyAsync of pageable rows (11 and 13 us) and
-// takes 34.8, its input gradient 105.7 and 54.9.  Beyond kPinChunk rows the
-// host copies a chunk out while the next one runs: 4,096 rows 352.8 -> 212,
+// takes 34.8, its input gradient 105.7 and 54.9.  Beyond a chunk of rows the
+// host copies a chunk out while the next one runs: 4,096 rows 352.8 -> 205,
 // of which the copy of 4.3 MB that the device has just written is the most
 // (one chunk of all rows, two streams, or outputs kept on the device and
 // copied a chunk at a time: 228 to 253).
@@ -762,12 +773,13 @@ template <uint32_t MODE>
 int pass_host_rows(ArboSurrogate* s, uint32_t n, const float* x, const float* dout, float* out, float* dx) {
     const Staging h = staging(s);
     const size_t in = s->w[0], no = s->w[s->L];
+    const uint32_t chunk = chunk_rows(s);
     PassArgs a = pass_args(s, MODE, 0);
     for (uint32_t b0 = 0; b0 < n; b0 += s->pin_rows) {   // blocks of the pinned rows
-        const uint32_t nb = std::min(s->pin_rows, n - b0), chunks = blocks(nb, kPinChunk);
+        const uint32_t nb = std::min(s->pin_rows, n - b0), chunks = blocks(nb, chunk);
         for (uint32_t c = 0; c <= chunks; ++c) {
             if (c < chunks) {
-                const size_t r0 = (size_t)c * kPinChunk, r = std::min<size_t>(kPinChunk, nb - r0);
+                const size_t r0 = (size_t)c * chunk, r = std::min<size_t>(chunk, nb - r0);
                 std::memcpy(h.x + r0 * in, x + (b0 + r0) * in, r * in * 4);
                 if (MODE == PASS_INPUT) std::memcpy(h.y + r0 * no, dout + (b0 + r0) * no, r * no * 4);
                 a.n = (uint32_t)r;
@@ -779,7 +791,7 @@ int pass_host_rows(ArboSurrogate* s, uint32_t n, const float* x, const float* do
                 if (chunks > 1) SUR_TRY(s, hipEventRecord(s->chunk_done[c & 1u], s->stream));
             }
             if (c == 0) continue;
-            const size_t r0 = (size_t)(c - 1) * kPinChunk, r = std::min<size_t>(kPinChunk, nb - r0);
+            const size_t r0 = (size_t)(c - 1) * chunk, r = std::min<size_t>(chunk, nb - r0);
             SUR_TRY(s, chunks > 1 ? hipEventSynchronize(s->chunk_done[(c - 1) & 1u]) : hipStreamSynchronize(s->stream));
             if (out) std::memcpy(out + (b0 + r0) * no, h.out + r0 * no, r * no * 4);
             if (MODE == PASS_INPUT) std::memcpy(dx + (b0 + r0) * in, h.dx + r0 * in, r * in * 4);
@@ -973,7 +985,16 @@ ARBO_API int arbo_sur_forward(ArboSurrogate* s, uint32_t n, const float* x, floa
     if (!s || !x || !out || n == 0) return ARBO_E_INVALID;
     if (n > s->max_batch) return fail(s, ARBO_E_CAPACITY, "more rows than max_batch");
     SUR_TRY(s, hipSetDevice(s->device));
-    if (s->pin && rows_apart(x, s->w[0], out, s->w[s->L], n))
+    // Long inputs with few outputs are copied to the device, which the runtime
+    // does faster than one thread fills pinned rows and the pass reads them:
+    // 8,192 rows of 512-256-256-3 took 814 us in pinned rows (chunks of 1 MB)
+    // and take 520.  With a quarter as many outputs or more, or less than 2 MB,
+    // pinned rows are the faster or as fast: 65,536 of 64-256-256-20 850 and
+    // copied 884, 4,096 of 300-256-256-100 266 and 273, 1,024 of 300-256-256-3
+    // 83% of the copied call's time.
+    const size_t in = s->w[0], no = s->w[s->L];
+    const bool copied = in > 4 * no && n * in * sizeof(float) >= kCopyBytes;
+    if (s->pin && !copied && rows_apart(x, in, out, no, n))
         return pass_host_rows<PASS_FORWARD>(s, n, x, nullptr, out, nullptr);
     if (int rc = upload_x(s, n, x)) return rc;
     if (s->fused) {

@@ -248,3 +248,26 @@ def test_results_over_the_inputs(hip_lib, widths, n, kind):
     assert s.lib.arbo_sur_input_grad(s._h, n, ptr(x.ravel(), 0), ptr(buf, at_y), None, ptr(buf, at_d)) == 0
     assert np.array_equal(buf[at_d:at_d + x.size], want_dx.ravel())
     s.close()
+
+
+@pytest.mark.parametrize("widths,rows", [([6, 16, 4], (43679, 43680, 43681, 87365)), ([20, 16, 260], (1007, 1009, 2017)),
+                                         ([300, 33, 74], (1747, 1748, 2500)), ([300, 33, 75], (1748,)),
+                                         ([301, 33, 1], (869, 870, 871, 1741, 1742, 6000))],
+                         ids=lambda w: "-".join(map(str, w)) if isinstance(w, list) else None)
+def test_host_rows_in_chunks_of_bytes(hip_lib, widths, rows):
+    """Host calls around the rows of a 1 MB chunk (2^20 / (4 x the wider of
+    inputs and outputs), a multiple of 16), and around the 2 MB of inputs from
+    which a forward call of few outputs copies them: every row as in calls of
+    fewer rows."""
+    s = Surrogate(widths, max_batch=rows[-1], seed=6, lib=hip_lib)
+    rng = np.random.default_rng(7)
+    x = rng.normal(size=(rows[-1], widths[0])).astype(np.float32)
+    dout = rng.normal(size=(rows[-1], widths[-1])).astype(np.float32)
+    parts = [s.input_grad(x[i:i + 800], dout[i:i + 800]) for i in range(0, rows[-1], 800)]
+    out, dx = (np.concatenate([p[k] for p in parts]) for k in (0, 1))
+    for n in rows:
+        print(f"[tiles] host chunks widths={widths} rows={n}", flush=True)
+        assert np.array_equal(s.forward(x[:n]), out[:n])
+        got_out, got_dx = s.input_grad(x[:n], dout[:n])
+        assert np.array_equal(got_out, out[:n]) and np.array_equal(got_dx, dx[:n])
+    s.close()
