@@ -705,15 +705,22 @@ hipError_t launch_wgrad(ArboSurrogate* s, uint32_t n, bool adam, float lr, float
     return hipGetLastError();
 }
 
-// The packed halves of every layer's weights from the parameters.
+// The packed halves of every layer's weights from the parameters, and zero moments.
 hipError_t launch_pack(ArboSurrogate* s) {
+    PackArgs g{};
+    g.L = s->L;
+    g.n = (uint32_t)s->n_params;   // at most 8 layers of 512 x 513
+    g.P = s->P.p;
+    g.M = s->Mo.p;
+    g.V = s->Vo.p;
+    g.pack = s->pack.p;
     for (uint32_t l = 0; l < s->L; ++l) {
         const uint32_t N = s->w[l + 1], K = s->w[l];
-        hipLaunchKernelGGL(k_pack, dim3(blocks((uint64_t)N * ((K + 1) / 2), 256)), dim3(256), 0, s->stream, s->P.p + s->woff[l], N,
-                           K, s->foff[l], (N + 15) / 16, s->boffk[l], (K + 15) / 16, s->pack.p);
-        if (hipError_t e = hipGetLastError()) return e;
+        g.l[l] = PackLayer{g.pairs, N, K, s->foff[l], s->boffk[l], s->woff[l]};
+        g.pairs += N * ((K + 1) / 2);
     }
-    return hipSuccess;
+    hipLaunchKernelGGL(k_pack, dim3(blocks(g.n, 256)), dim3(256), 0, s->stream, g);
+    return hipGetLastError();
 }
 
 // The pinned rows' arrays: inputs, targets or dout, outputs, input gradients.
@@ -970,12 +977,15 @@ ARBO_API int arbo_sur_set_params(ArboSurrogate* s, const float* in) {
     if (!s || !in) return ARBO_E_INVALID;
     SUR_TRY(s, hipSetDevice(s->device));
     SUR_TRY(s, hipMemcpyAsync(s->P.p, in, s->n_params * 4, hipMemcpyHostToDevice, s->stream));
-    hipLaunchKernelGGL(k_zero_f32, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->Mo.p,
-                       (uint64_t)s->n_params);
-    hipLaunchKernelGGL(k_zero_f32, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->Vo.p,
-                       (uint64_t)s->n_params);
-    SUR_TRY(s, hipGetLastError());
-    if (s->fused) SUR_TRY(s, launch_pack(s));
+    if (s->fused) {
+        SUR_TRY(s, launch_pack(s));
+    } else {
+        hipLaunchKernelGGL(k_zero_f32, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->Mo.p,
+                           (uint64_t)s->n_params);
+        hipLaunchKernelGGL(k_zero_f32, dim3(blocks(s->n_params, 256)), dim3(256), 0, s->stream, s->Vo.p,
+                           (uint64_t)s->n_params);
+        SUR_TRY(s, hipGetLastError());
+    }
     s->adam_t = 0;
     SUR_TRY(s, hipStreamSynchronize(s->stream));
     return ARBO_OK;

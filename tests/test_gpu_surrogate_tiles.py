@@ -271,3 +271,26 @@ def test_host_rows_in_chunks_of_bytes(hip_lib, widths, rows):
         got_out, got_dx = s.input_grad(x[:n], dout[:n])
         assert np.array_equal(got_out, out[:n]) and np.array_equal(got_dx, dx[:n])
     s.close()
+
+
+@pytest.mark.parametrize("widths", [[1, 1], [6, 33, 12], [5, 17, 300, 64, 7], [6, 520, 9]], ids=lambda w: "-".join(map(str, w)))
+def test_new_parameters_start_afresh(hip_lib, widths):
+    """set_params after a training: its weights are the ones the next calls
+    read, and the next training starts from zero moments, as a surrogate's
+    first one does."""
+    rng = np.random.default_rng(14)
+    x = rng.normal(size=(40, widths[0])).astype(np.float32)
+    y = rng.poisson(2.0, size=(40, widths[-1])).astype(np.float32)
+    p = flatten(random_layers(widths, 15))
+    got = []
+    for before in (False, True):
+        s = Surrogate(widths, max_batch=64, seed=16, lib=hip_lib)
+        if before:
+            s.train(x, y, epochs=2, batch=16, lr=1e-2, seed=17)
+        s.set_params(p)
+        out = s.forward(x)
+        s.train(x, y, epochs=1, batch=16, lr=1e-3, seed=18)
+        got.append((out, s.get_params(), s.forward(x)))
+        s.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
