@@ -192,12 +192,23 @@ __global__ __launch_bounds__(kFuseThreads) void k_mlp(PassArgs g) {
         for (uint32_t l = 0; l < ARBO_SUR_MAX_LAYERS; ++l) b[l] = l < g.L && tid < g.bias[l].n ? g.bias[l].p[tid] : 0.0f;
         const uint32_t r = tid >> 5, kp = g.st[0].groups * kGroupK;
         const uint64_t xr = r < left ? (g.rows ? g.rows[row0 + r] : row0 + r) : 0u;
-        for (uint32_t c = tid & 31u; c < kp; c += 32) {
-            const float v = r < left && c < g.w0 ? g.x[xr * g.w0 + c] : 0.0f;
-            uint16_t hi, lo;
-            split_bf16(v, hi, lo);
-            s_act[r * g.ldk + c] = hi;
-            s_act[plane + r * g.ldk + c] = lo;
+        // Eight loads of a row in flight where the inputs are many (one at a
+        // time: 262,144 rows of 512-2-3 449 us for 252); columns past the last
+        // read the first's, so that no branch waits for a load.
+        const float* x = g.x + xr * g.w0;
+#pragma unroll 4
+        for (uint32_t c0 = tid & 31u; c0 < kp; c0 += 64) {   // kp is a multiple of 64
+            float v[2];
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) v[u] = x[c0 + 32 * u < g.w0 ? c0 + 32 * u : 0u];
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const uint32_t c = c0 + 32 * u;
+                uint16_t hi, lo;
+                split_bf16(r < left && c < g.w0 ? v[u] : 0.0f, hi, lo);
+                s_act[r * g.ldk + c] = hi;
+                s_act[plane + r * g.ldk + c] = lo;
+            }
         }
 #pragma unroll
         for (uint32_t l = 0; l < ARBO_SUR_MAX_LAYERS; ++l)

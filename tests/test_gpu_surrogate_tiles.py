@@ -294,3 +294,21 @@ def test_new_parameters_start_afresh(hip_lib, widths):
         s.close()
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("inputs", [1, 31, 32, 33, 63, 64, 65, 255, 256, 257, 319, 320, 511, 512])
+def test_rows_of_any_width_are_read(hip_lib, inputs):
+    """Input widths around the columns that a row's loads take at once; a NaN
+    in a row's first column, which loads past the last column read, stays in
+    its row."""
+    print(f"[tiles] inputs={inputs}", flush=True)
+    layers = random_layers([inputs, 24, 9], 23)
+    s = Surrogate([inputs, 24, 9], max_batch=64, seed=24, lib=hip_lib)
+    s.set_params(flatten(layers))
+    x = np.random.default_rng(25).normal(size=(37, inputs)).astype(np.float32)
+    out = s.forward(x)
+    assert rel(out, forward64(layers, x)[0]) < 1e-4
+    x[5, 0] = np.nan
+    bad = s.forward(x)
+    assert np.all(np.isnan(bad[5])) and np.array_equal(np.delete(bad, 5, 0), np.delete(out, 5, 0))
+    s.close()
