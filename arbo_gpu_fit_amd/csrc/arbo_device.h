@@ -23,7 +23,7 @@ constexpr uint32_t kHumanAlign = 4;       // humans per 16-byte vector
 constexpr uint32_t kMosqAlign = 128;      // mosquito slots per 16-byte group of alive-bitmap words
 constexpr uint32_t kAoiRecord = 5000;     // ages per age-of-infection ring
 // Per-community partials of a day, written by the demography kernel and
-// summed per simulation by k_day_counts: word 0 mosquitoes alive after the
+// summed by k_day_counts: word 0 mosquitoes alive after the
 // births, 1 humans, 2-3 infectious humans (two 16-bit serotype pairs), 4-5
 // E->I onsets (pairs), 6-7 the 16-byte census vectors of humans and of
 // mosquitoes the day's scan read, 8-9 infectious mosquitoes (pairs); in small
@@ -34,23 +34,37 @@ constexpr uint32_t kPartWords = 24;
 constexpr uint64_t kMaxCommunities = (1ull << 26) - 1;
 // Communities of a workgroup of k_day_counts: 32, or fewer (4, 8, 16) while that
 // makes no more than kCountBlocks workgroups.  The 256 threads share their
-// communities' events, so fewer communities shorten an epidemic's days, and
-// the idle workgroups of quiet days cost about 11 ns each.  One simulation,
-// transmission rates 0.7, us a day with 32, 16, 8 and 4: 529 communities of
-// 2,500 humans 108.6, 93.8, 86.1, 82.3, 1,024 of 1,000 humans 70.0, 62.4,
-// 59.0, 57.5, 2,500 81.0, 75.1, 72.7, 72.7, 4,096 91.8, 86.4, 85.1, 87.2,
-// 6,400 120.4, 117.4, 116.4, 123.4; rates 0.15 and no epidemic: 1,024 36.0,
-// 35.8, 36.5, 38.0, 2,500 48.3, 48.9, 50.6, 54.7, 4,096 56.0, 57.0, 60.1, 67.3.
+// communities' events, so fewer communities shorten an epidemic's days; on
+// quiet days a workgroup more costs 2 ns.  One simulation, transmission rates
+// 0.7, us a day with 32, 16, 8 and 4: 529 communities of 2,500 humans 126.2,
+// 107.4, 98.1, 93.7, 1,024 of 1,000 humans 79.2, 69.6, 65.6, 63.0, 2,500 92.3,
+// 84.9, 81.0, 80.2, 4,096 104.2, 96.5, 94.1, 93.4, 10,000 176.5, 171.2, 167.9,
+// 174.1, 25,600 428.3, 426.3, 430.0, 444.0; rates 0.15 and no epidemic: 1,024
+// 31.4, 30.8, 31.3, 30.7, 2,500 36.8, 37.0, 36.5, 37.4, 4,096 41.5, 40.8, 41.2,
+// 42.1, 10,000 62.1, 62.8, 63.1, 66.8, 25,600 120.9, 123.6, 126.5, 133.3.
 constexpr uint32_t kCountComms = 32;
 constexpr uint32_t kCountBlocks = 320;
 constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together
 constexpr uint32_t kAoiWindow = 3650;     // rings record the days t with max_days - t <= this
 
 // A workgroup of k_day_counts: n communities of one simulation from community
-// c0, global index `first`, whose CSR rows are entries [row, row + rows).
+// c0, global index `first`, whose CSR rows are entries [row, row + rows); its
+// sums go to record `total`.
 struct CountBlock {
-    uint32_t sim, c0, first, n, row, rows;
+    uint32_t sim, c0, first, n, row, rows, total;
 };
+
+// Sums of a day over communities of one simulation, added by k_day_counts and
+// read by the long-distance kernel: words (u64) 0-7 the long-distance rates in
+// 2^-24 units (Poisson counts) or event counts (stochastic rounding), then as
+// u32 humans, mosquitoes, infectious humans[4], onsets[4], census vectors read
+// (humans, mosquitoes).  Integer atomics of different workgroups on one line
+// follow each other 9 ns apart, so a simulation has a record per kTotalBlocks
+// workgroups, up to kTotalRecords: with one, a quiet day of 480 x 480
+// communities (7,200 workgroups) spent 63 of its 94 us in k_day_counts on them.
+constexpr uint32_t kTotalWords = 16;
+constexpr uint32_t kTotalBlocks = 64;
+constexpr uint32_t kTotalRecords = 16;
 
 struct CommDesc {
     uint64_t h_off;       // global offset of the first human
@@ -93,6 +107,7 @@ struct SimDesc {
     float no_distance;            // fraction of events staying at the source (communities with kCommStay)
     uint64_t series_off;          // this simulation's block in the series array
     uint64_t spatial_off;         // its block [(T+1)][S][C] of the per-community series (if kept)
+    uint32_t total, totals;       // its records of the day's sums
     uint32_t aoi_block;           // its first block of kAoiBlock communities (age-of-infection rings)
     uint32_t aoi_blocks;
     uint32_t climate;             // 1: per-day beta/eip at clim_off and per-birth-day lifetime rows
@@ -150,12 +165,12 @@ struct EngineView {
     uint32_t* hsum;                // [G][4] summary: earliest day any human has an event (0 = unknown),
                                    // infectious humans by serotype (two 16-bit pairs), mosquito scan
                                    // limit + 1 in 8-slot vectors (0 = unknown)
-    unsigned long long* lam;       // [2 parity][n_sims][8] long-distance events of the day: the rate in
-                                   // 2^-24 units (Poisson counts) or the count (stochastic rounding)
+    unsigned long long* totals;    // [2 parity][n_totals][kTotalWords] sums of days of that parity
+    uint32_t n_totals;
     uint32_t* series;
     uint32_t* part;                // [G][kPartWords] per-community partials of the day (see kPartWords)
     unsigned long long* scanned;   // [n_sims][2] census vectors read by the demography kernel (humans,
-                                   // mosquitoes), summed over days by k_day_counts
+                                   // mosquitoes), summed over days
     uint32_t* spatial;             // per-community infectious humans [(T+1)][S][C] per simulation, or null
     int32_t* hist;                 // per human 4 infection-history words (one per serotype), or null
     uint8_t* aoi_mark;             // per human: 1 + ring when a mosquito event infected it today

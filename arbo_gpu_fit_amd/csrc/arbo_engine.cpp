@@ -65,7 +65,7 @@ struct ArboEngine {
     DevBuf<uint8_t> aoi_mark;
     DevBuf<uint32_t> aoi, aoi_pos, aoi_cnt, aoi_sum;
     DevBuf<CountBlock> count_map;
-    DevBuf<unsigned long long> lam, scanned;
+    DevBuf<unsigned long long> totals, scanned;
     DevBuf<uint32_t> part;   // per-community partials of the day
     DevBuf<float> dens;
     DevBuf<double> scales;         // daily mosquito scales of the climates (lifetime tables)
@@ -134,7 +134,7 @@ void free_batch(ArboEngine* e) {
     dev_free(e->h_word); dev_free(e->alive); dev_free(e->cnt); dev_free(e->nld); dev_free(e->active); dev_free(e->hsum); dev_free(e->series); dev_free(e->spatial); dev_free(e->csr_thr); dev_free(e->csr_inbox);
     dev_free(e->in_edge); dev_free(e->in_slot); dev_free(e->tables); dev_free(e->day_ctr);
     dev_free(e->h_next); dev_free(e->m_word); dev_free(e->m_next); dev_free(e->h_birth); dev_free(e->hist); dev_free(e->aoi_mark); dev_free(e->aoi); dev_free(e->aoi_pos); dev_free(e->aoi_cnt); dev_free(e->aoi_sum); dev_free(e->count_map);
-    dev_free(e->lam); dev_free(e->scanned); dev_free(e->dens); dev_free(e->part);
+    dev_free(e->totals); dev_free(e->scanned); dev_free(e->dens); dev_free(e->part);
     dev_free(e->scales); dev_free(e->life_h); dev_free(e->life_m);
     e->ready = false;
 }
@@ -322,7 +322,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     std::map<std::vector<uint32_t>, uint32_t> seen_u32;
     std::map<std::vector<float>, uint32_t> seen_f32;
     uint64_t h_tot = 0, m_tot = 0, ser_tot = 0, spa_tot = 0;
-    uint32_t aoi_blocks = 0;
+    uint32_t aoi_blocks = 0, n_totals = 0;
     uint32_t count_comms = 4;   // communities of a workgroup of the event counts
     while (count_comms < kCountComms && communities > (uint64_t)count_comms * kCountBlocks) count_comms *= 2;
     uint32_t max_n = 0, max_cap = 0, death_m_lds = 1;
@@ -443,9 +443,14 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
             max_n = std::max(max_n, cd.n);
             max_cap = std::max(max_cap, cd.cap);
         }
-        for (uint32_t c = 0; c < t.C; c += count_comms) {
-            const uint32_t n = std::min(count_comms, t.C - c), row = row_base + t.row_ptr[c];
-            count_map.push_back(CountBlock{i, c, sh.comm_off + c, n, row, t.row_ptr[c + n] - t.row_ptr[c]});
+        const uint32_t count_blocks = (t.C + count_comms - 1) / count_comms;
+        sd.total = n_totals;
+        sd.totals = std::min(kTotalRecords, (count_blocks + kTotalBlocks - 1) / kTotalBlocks);
+        n_totals += sd.totals;
+        for (uint32_t b = 0; b < count_blocks; ++b) {
+            const uint32_t c = b * count_comms, n = std::min(count_comms, t.C - c), row = row_base + t.row_ptr[c];
+            count_map.push_back(CountBlock{i, c, sh.comm_off + c, n, row, t.row_ptr[c + n] - t.row_ptr[c],
+                                           sd.total + b % sd.totals});
         }
         sd.aoi_block = aoi_blocks;
         sd.aoi_blocks = (t.C + kAoiBlock - 1) / kAoiBlock;
@@ -488,7 +493,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
         (rc = dev_alloc(e, e->aoi_sum, (e->flags & ARBO_F_AOI) ? (size_t)aoi_blocks * 8 : 0)) || (rc = dev_alloc(e, e->m_word, m_tot)) ||
         (rc = dev_alloc(e, e->m_next, m_tot)) || (rc = dev_alloc(e, e->alive, m_tot / 32)) || (rc = dev_alloc(e, e->cnt, comm.size() * kInboxEdges * 8)) || (rc = dev_alloc(e, e->nld, comm.size() * 8)) ||
         (rc = dev_alloc(e, e->hsum, comm.size() * 4)) || (rc = dev_alloc(e, e->active, comm.size())) ||
-        (rc = dev_alloc(e, e->lam, (size_t)2 * n_sims * 8)) || (rc = dev_alloc(e, e->scanned, (size_t)2 * n_sims)) || (rc = dev_alloc(e, e->part, comm.size() * kPartWords)) || (rc = dev_alloc(e, e->series, ser_tot)) || (rc = dev_alloc(e, e->spatial, spa_tot)) ||
+        (rc = dev_alloc(e, e->totals, (size_t)2 * n_totals * kTotalWords)) || (rc = dev_alloc(e, e->scanned, (size_t)2 * n_sims)) || (rc = dev_alloc(e, e->part, comm.size() * kPartWords)) || (rc = dev_alloc(e, e->series, ser_tot)) || (rc = dev_alloc(e, e->spatial, spa_tot)) ||
         (rc = dev_alloc(e, e->csr_thr, csr_thr.size())) || (rc = dev_alloc(e, e->csr_inbox, csr_inbox.size())) || (rc = dev_alloc(e, e->in_edge, in_edge.size())) ||
         (rc = dev_alloc(e, e->in_slot, in_slot.size())) || (rc = dev_alloc(e, e->tables, pool_words)) || (rc = dev_alloc(e, e->count_map, count_map.size())) || (rc = dev_alloc(e, e->scales, scales.size())) ||
         (rc = dev_alloc(e, e->life_h, life_h.size())) || (rc = dev_alloc(e, e->life_m, life_m.size())) ||
@@ -512,7 +517,7 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
                                   max_rows, e->scales.p, e->stream));
     HIP_TRY(e, launch_fill(e->series.p, ser_tot, 0u, e->stream));
     if (spa_tot) HIP_TRY(e, launch_fill(e->spatial.p, spa_tot, 0u, e->stream));
-    HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->lam.p), (uint64_t)2 * n_sims * 8 * 2, 0u, e->stream));
+    HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->totals.p), (uint64_t)2 * n_totals * kTotalWords * 2, 0u, e->stream));
     HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->scanned.p), (uint64_t)2 * n_sims * 2, 0u, e->stream));
     HIP_TRY(e, launch_fill(e->day_ctr.p, 1, 0u, e->stream));
     HIP_TRY(e, launch_fill(e->nld.p, comm.size() * 8, 0u, e->stream));
@@ -545,7 +550,8 @@ int arbo_batch_init(ArboEngine* e, uint32_t n_sims, const ArboShape* shapes, con
     v.active = e->active.p;
     v.cnt = e->cnt.p;
     v.nld = e->nld.p;
-    v.lam = e->lam.p;
+    v.totals = e->totals.p;
+    v.n_totals = n_totals;
     v.part = e->part.p;
     v.scanned = e->scanned.p;
     v.series = e->series.p;
@@ -932,7 +938,7 @@ int arbo_set_day(ArboEngine* e, uint32_t day) {
         }
     }
     HIP_TRY(e, hipMemcpy(e->series.p, blk.data(), blk.size() * 4, hipMemcpyHostToDevice));
-    HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->lam.p), (uint64_t)e->lam.n * 2, 0u, e->stream));
+    HIP_TRY(e, launch_fill(reinterpret_cast<uint32_t*>(e->totals.p), (uint64_t)2 * e->view.n_totals * kTotalWords * 2, 0u, e->stream));
     HIP_TRY(e, launch_fill(e->hsum.p, e->hsum.n, 0u, e->stream));
     if (e->flags & ARBO_F_AOI) {   // the rings go on where they stand, whichever the new day's parity
         const size_t n = (size_t)e->n_sims * 4;

@@ -21,8 +21,9 @@
 //  k_day_counts      (nepidemic.cu:49-136)
 //     draws the Poisson event counts of the communities as sources, spreads
 //     the local events over their CSR rows with the alias tables into LDS
-//     histograms and adds the partials into the series row of the next day
-//     (small batches: in the demography and event kernels).
+//     histograms and sums the partials; the long-distance kernel writes them
+//     to the series row of the next day (small batches: the counts in the
+//     demography kernel, the series in the event kernel).
 //
 //  k_day_events      mepidemic.cu:143-246 (nmTransmission) +
 //                    nepidemic.cu:146-319 (mnTransmission)
@@ -1671,7 +1672,8 @@ __global__ __launch_bounds__(kWave * NW) void k_day_events(EngineView v) {
 // direction and serotype the events are L ~ Poisson(summed long-distance rate
 // of all sources); event l lands on community mulhi(Philox(l), C).  Only the
 // number landing on each destination matters (their targets are drawn at the
-// destination), so the destinations are counted with integer atomics.
+// destination), so the destinations are counted with integer atomics.  Part 0
+// also writes the day's sums to series row t + 1.
 // Part `part` of `split` of simulation `sim`'s long-distance events of day t
 // (all 256 threads of the workgroup call it).
 __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim, uint32_t t, uint32_t part,
@@ -1679,8 +1681,12 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
     const SimDesc sd = v.sims[sim];
     const Key key{sd.k0, sd.k1};
     __shared__ uint32_t s_L[8];
+    // the simulation's sums of today, by k_day_counts
+    const unsigned long long* tot = v.totals + ((size_t)(t & 1u) * v.n_totals + sd.total) * kTotalWords;
     if (tid < 8) {
-        const unsigned long long fx = v.lam[((size_t)(t & 1u) * v.n_sims + sim) * 8 + tid];   // summed by k_day_counts
+        unsigned long long fx = 0;
+#pragma unroll 4
+        for (uint32_t r = 0; r < sd.totals; ++r) fx += tot[r * kTotalWords + tid];
         const uint32_t L = longdist_count(sd, key, t, tid, fx);
         s_L[tid] = L;
     }
@@ -1697,8 +1703,22 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
         atomicAdd(&v.nld[(size_t)(sd.comm_off + d) * 8 + k], 1u);
         v.active[sd.comm_off + d] = 1u;
     }
-    // the long-distance sums of the next day start at zero
-    if (part == 0 && tid < 8) v.lam[((size_t)((t + 1) & 1u) * v.n_sims + sim) * 8 + tid] = 0ull;
+    if (part != 0) return;
+    if (tid >= 64 && tid < 76) {   // the series row (datacollect.cu:79-189)
+        const uint32_t k = tid - 64, S = sd.S, row = t + 1;
+        uint32_t n = 0;
+#pragma unroll 4
+        for (uint32_t r = 0; r < sd.totals; ++r) n += reinterpret_cast<const uint32_t*>(tot + r * kTotalWords + 8)[k];
+        const SeriesIdx si = series_index(sd.series_off, v.max_days, S);
+        if (k == 0) v.series[si.n_count + row] = n;
+        else if (k == 1) v.series[si.m_count + row] = n;
+        else if (k < 6) { if (k - 2 < S) v.series[si.n_inf + (size_t)row * S + (k - 2)] = n; }
+        else if (k < 10) { if (k - 6 < S) v.series[si.n_inc + (size_t)row * S + (k - 6)] = n; }
+        else v.scanned[2 * (size_t)sim + (k - 10)] += n;
+    }
+    // tomorrow's sums start at zero
+    unsigned long long* next = v.totals + ((size_t)((t + 1) & 1u) * v.n_totals + sd.total) * kTotalWords;
+    for (uint32_t i = tid; i < sd.totals * kTotalWords; i += 256) next[i] = 0ull;
 }
 
 __global__ __launch_bounds__(256) void k_day_longdist(EngineView v, uint32_t split) {
@@ -1711,8 +1731,7 @@ __global__ __launch_bounds__(256) void k_day_longdist(EngineView v, uint32_t spl
 // workgroup, and the sums of their partials.  Eight lanes a community draw its
 // event counts (direction and serotype each), the workgroup spreads all its
 // events' quads over its threads and pushes the counts into the destinations'
-// inboxes; integer atomics add the workgroup's sums to the series row t + 1
-// (datacollect.cu:79-189, zero until then) and to the long-distance totals
+// inboxes; integer atomics add the workgroup's sums to its record of the day
 // (zeroed by the previous day's long-distance kernel).
 // Why here: the demography kernel issues a vector instruction on 9 of 10
 // cycles during an epidemic, and the counts took it 500 of 2,400 a wave with
@@ -1838,21 +1857,14 @@ __global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
         s_fx[wv][k] = fx;
     }
     __syncthreads();
-    const uint32_t S = sd.S, row = t + 1;
-    const SeriesIdx si = series_index(sd.series_off, v.max_days, S);
+    unsigned long long* tot = v.totals + ((size_t)(t & 1u) * v.n_totals + cb.total) * kTotalWords;
     if (tid < 12) {
         const uint32_t n = s_cnt[0][tid] + s_cnt[1][tid] + s_cnt[2][tid] + s_cnt[3][tid];
-        uint32_t* dst = nullptr;
-        if (tid == 0) dst = &v.series[si.n_count + row];
-        else if (tid == 1) dst = &v.series[si.m_count + row];
-        else if (tid < 6) { if (tid - 2 < S) dst = &v.series[si.n_inf + (size_t)row * S + (tid - 2)]; }
-        else if (tid < 10) { if (tid - 6 < S) dst = &v.series[si.n_inc + (size_t)row * S + (tid - 6)]; }
-        else if (n) atomicAdd(&v.scanned[2 * (size_t)cb.sim + (tid - 10)], (unsigned long long)n);
-        if (dst && n) atomicAdd(dst, n);
+        if (n) atomicAdd(reinterpret_cast<uint32_t*>(tot + 8) + tid, n);
     }
     if (tid >= 64 && tid < 72) {
         const unsigned long long n = s_fx[0][tid - 64] + s_fx[1][tid - 64] + s_fx[2][tid - 64] + s_fx[3][tid - 64];
-        if (n) atomicAdd(&v.lam[((size_t)(t & 1u) * v.n_sims + cb.sim) * 8 + (tid - 64)], n);
+        if (n) atomicAdd(tot + (tid - 64), n);
     }
 }
 

@@ -276,3 +276,37 @@ def test_small_batches_by_what_they_send(hip_lib, oracle_lib, grids, humans, big
         assert gpu.launch_shape()["small_batch"] == small
         _both(hip_lib, oracle_lib, specs(omega), T, checks=(4,))
     gpu.close()
+
+
+@pytest.mark.parametrize("grids,law", [([(16, 16), (20, 13), (27, 19)], 0), ([(128, 256), (1, 1)], 0), ([(181, 183), (9, 9)], 1)])
+def test_day_sums_of_many_workgroups(hip_lib, oracle_lib, grids, law):
+    """Simulations of 64 and 65 workgroups of event counts (one record of the
+    day's sums and two), and of 1,024 and more (the most records): the series
+    and the first day's scan counts, and days of either parity done again."""
+    print(f"[edges] sums {grids} {law}", flush=True)
+    specs = [SimSpec(w, h, np.where(np.arange(w * h) % 3 == 1, 9, 4).astype(np.uint32),
+                     configs.base_params(beta_hm=0.8, beta_mh=0.8, seed_frac_h=0.1, seed_frac_m=0.05, long_distance=0.1, count_law=law),
+                     90 + i) for i, (w, h) in enumerate(grids)]
+    gpu, orc = Engine(hip_lib), Engine(oracle_lib, threads=8)
+    for e in (gpu, orc):
+        e.init(specs, 12)
+    assert not gpu.launch_shape()["small_batch"]
+    for e in (gpu, orc):
+        e.step(1)
+    assert gpu.scan_counts() == orc.scan_counts()   # on day 0 both read everything
+    for e in (gpu, orc):
+        e.step(4)
+    kept = [orc.state(i) for i in range(len(specs))]
+    for e in (gpu, orc):
+        e.step(4)
+    for day in (5, 6):
+        for e in (gpu, orc):
+            for i, s in enumerate(kept):
+                e.write_state(i, s)
+            e.set_day(day)
+            e.step(12 - day)
+        for i in range(len(specs)):
+            _compare_state(gpu.state(i), orc.state(i), f"sim {i}")
+            _compare_series(gpu.series(i), orc.series(i), f"sim {i}")
+    gpu.close()
+    orc.close()
