@@ -7,11 +7,12 @@
 // workgroup keeps its rows' activations in LDS and a pass is one launch; a
 // product per launch costs 4.3 us of the stream for the launch alone, and took
 // 17-20 us here: 64 x 64 tiles gave a 64-row pass four workgroups, each with a
-// load latency per 64 k in series.  What is left is the weights: every
-// workgroup reads all of them once per pass, 1.05 MB forward for the
-// 6-256^4-260 network, at the 38 B/clk that one CU draws from L2 whatever is
-// kept in flight (32 to 256 KB a CU measured the same; the same loads hitting
-// L1 end 5 us earlier): 11.6 us at 2.4 GHz of a pass's 14.5.  Hence:
+// load latency per 64 k in series.  What is left is one workgroup's chain:
+// it reads all the weights once per pass, 1.1 MB forward for the 6-256^4-260
+// network, through six dependent stages of about 3 us each.  The reads alone
+// are 7 us of the pass's 18.6 (a CU draws 64 B/clk out of L2, 52 with all of
+// them reading), and the same loads hitting L1 end 5 us earlier; more of them
+// in flight (32 to 256 KB a CU) measured the same.  Hence:
 //  * the weights are kept a second time, split into bf16 halves (hi, lo) and
 //    laid out in MFMA fragment order, once for the forward products and once
 //    transposed for the backward ones: a lane's operand is one coalesced
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256) void k_pack(PackArgs g) {
 struct GradLayer {
     uint32_t N, K;             // outputs, inputs
     uint32_t first, tx;        // its first workgroup and tiles along the inputs
-    const uint16_t* dz;        // dZ and inputs as operands (frag_of_row)
+    const uint16_t* dz;        // dZ and inputs as operands (store_operand)
     const uint16_t* h;
     uint64_t w, b;             // weights and biases in the parameter arrays
     uint32_t foff, boff;       // in the packed weights (bytes)
@@ -475,7 +476,7 @@ __device__ __forceinline__ float adam_update(const GradArgs& g, uint64_t at, con
 constexpr uint32_t kGradWaves = 8;
 
 // [dW | db] = dZ^T [X | 1] of every layer in one launch, a 32 x 32 tile of dW
-// a workgroup (273 tiles for 6-256^4-260, about one per CU).  The batch is the
+// a workgroup (272 tiles for 6-256^4-260, about one per CU).  The batch is the
 // reduction: its 16-row steps are dealt to the eight waves in turn, so a
 // minibatch of 512 is four steps a wave, all sixteen loads of them in flight
 // at once, and the waves' partial tiles are added in LDS.  The bias gradient
