@@ -36,8 +36,8 @@ day, against HBM bandwidth.
     `achieved` divides them by the kernel's mean launch time, measured with
     HIP events on the engine's stream.
   * `traffic` is the kernel's HBM bytes per launch from rocprofv3's
-    FETCH_SIZE and WRITE_SIZE passes over this same command (calibrated
-    against a plain copy), read from the committed profile; `traffic_frac`
+    FETCH_SIZE and WRITE_SIZE passes over the same days, both at the default
+    tuning (calibrated against a plain copy), read from the committed profile; `traffic_frac`
     is that rate over the peak.  `full_scan_bytes` prices a scan of every
     member every day (4 B per human, 4 B per slot, 32 B per community and
     serotype) for comparison.
