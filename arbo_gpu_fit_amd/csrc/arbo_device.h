@@ -36,12 +36,12 @@ constexpr uint64_t kMaxCommunities = (1ull << 26) - 1;
 // makes no more than kCountBlocks workgroups.  The 256 threads share their
 // communities' events, so fewer communities shorten an epidemic's days; on
 // quiet days a workgroup more costs 2 ns.  One simulation, transmission rates
-// 0.7, us a day with 32, 16, 8 and 4: 529 communities of 2,500 humans 126.2,
-// 107.4, 98.1, 93.7, 1,024 of 1,000 humans 79.2, 69.6, 65.6, 63.0, 2,500 92.3,
-// 84.9, 81.0, 80.2, 4,096 104.2, 96.5, 94.1, 93.4, 10,000 176.5, 171.2, 167.9,
-// 174.1, 25,600 428.3, 426.3, 430.0, 444.0; rates 0.15 and no epidemic: 1,024
-// 31.4, 30.8, 31.3, 30.7, 2,500 36.8, 37.0, 36.5, 37.4, 4,096 41.5, 40.8, 41.2,
-// 42.1, 10,000 62.1, 62.8, 63.1, 66.8, 25,600 120.9, 123.6, 126.5, 133.3.
+// 0.7, us a day with 32, 16, 8 and 4: 529 communities of 2,500 humans 127.4,
+// 108.0, 97.3, 92.3, 1,024 of 1,000 humans 77.3, 67.4, 62.5, 59.8, 2,500 89.4,
+// 81.1, 77.3, 77.0, 4,096 102.6, 93.9, 90.7, 92.5, 10,000 177.7, 171.9, 170.4,
+// 177.8, 25,600 439.2, 437.9, 442.5, 459.1; rates 0.15 and no epidemic: 1,024
+// 33.0, 32.5, 33.1, 32.3, 2,500 38.0, 38.1, 37.7, 38.5, 4,096 42.2, 41.5, 41.8,
+// 43.4, 10,000 62.9, 63.5, 64.2, 68.1, 25,600 121.7, 124.1, 127.2, 134.5.
 constexpr uint32_t kCountComms = 32;
 constexpr uint32_t kCountBlocks = 320;
 constexpr uint32_t kAoiBlock = 256;       // communities whose age-of-infection records are summed together

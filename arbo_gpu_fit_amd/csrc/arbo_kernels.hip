@@ -550,21 +550,81 @@ __device__ __forceinline__ uint32_t human_states_packed(const EngineView& v, con
 
 // Events of a community as a source in direction k / 4 and of serotype k % 4
 // (nepidemic.cu:49-136): n dispersed locally, `stay` that stay, and the
-// long-distance rate (2^-24 units) or count.
+// long-distance rate (2^-24 units) or count.  Every lane of a wave calls it,
+// those without a source with I = 0.
 struct SourceCount {
     uint32_t n, stay;
     unsigned long long fx;
 };
+
+__device__ __forceinline__ double lane_double(double x, uint32_t lane) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)b, (int)lane, kWave);
+    const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(b >> 32), (int)lane, kWave);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+// poisson(mu, st) of every lane of the wave (all of them call; the same key).
+// A rejection trial is 2 us of dependent double arithmetic and the lane that
+// needs most of them holds up the wave, its workgroup and, in a batch of a few
+// workgroups a CU, the kernel.  The trials of a lane are therefore tried side
+// by side: as many at once as there are lanes for each lane still without a
+// result, the first accepted one taken.  A day at an epidemic's height: 12
+// simulations of 324 communities of 500 humans 69.4 -> 60.8 us, 11 of 100 to
+// 484 of 1,000 89.0 -> 80.5, one of 1,024 of 1,000 66.6 -> 53.3, one of 100
+// 47.9 -> 41.4; quiet days within 0.3.
+__device__ __forceinline__ uint32_t wave_poisson(double mu, const Stream& st, uint32_t lane) {
+    const bool reject = mu >= 10.0;
+    uint32_t out = 0u;
+    if (reject) out = (uint32_t)floor(mu);   // the result where no trial is accepted
+    else if (mu > 0.0) out = poisson_inversion(mu, stream_draw(st, 0));
+    uint64_t left = __builtin_amdgcn_ballot_w64(reject);
+    if (left == 0ull) return out;
+    const Ptrs mine = ptrs(reject ? mu : 10.0);
+    for (uint32_t it0 = 0; left != 0ull && it0 < POIS_PTRS_MAXIT;) {   // wave-uniform
+        const uint32_t n = (uint32_t)__popcll(left), per = kWave / n, slot = lane / per;
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(left >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u));
+        const bool pending = (left >> lane) & 1ull;
+        // the lane whose trial this one takes, the slot-th that is left: each
+        // sends its number to the lane of its rank (the others to the last
+        // lane, no lane's rank while there are any)
+        const uint32_t sent = (uint32_t)__builtin_amdgcn_ds_permute((int)(4u * (pending ? rank : kWave - 1u)), (int)lane);
+        const uint32_t owner = (uint32_t)__shfl((int)sent, (int)slot, kWave);
+        const uint32_t it = it0 + lane % per;
+        const Ptrs p{lane_double(mine.mu, owner), lane_double(mine.loglam, owner), lane_double(mine.b, owner),
+                     lane_double(mine.a, owner), lane_double(mine.invalpha, owner), lane_double(mine.vr, owner)};
+        const Stream s{st.key, (uint32_t)__shfl((int)st.x0, (int)owner, kWave), st.x1,
+                       (uint32_t)__shfl((int)st.x2, (int)owner, kWave)};
+        const PtrsTrial x = ptrs_trial(p, stream_draw(s, it));
+        const bool valid = slot < n && it < POIS_PTRS_MAXIT;
+        // the long test only for trials with no accepted one before them
+        uint64_t acc = __builtin_amdgcn_ballot_w64(valid && x.sure);
+        const uint64_t before = (1ull << lane) - 1ull, group = ~0ull << (slot * per);
+        const bool open = valid && x.open && (acc & before & group) == 0ull;
+        if (__builtin_amdgcn_ballot_w64(open)) acc |= __builtin_amdgcn_ballot_w64(open && ptrs_accept(p, x));
+        const uint64_t own = pending ? (acc >> (rank * per)) & (~0ull >> (kWave - per)) : 0ull;   // of this lane's trials
+        const uint32_t from = own ? rank * per + (uint32_t)__ffsll((unsigned long long)own) - 1u : 0u;
+        const uint32_t k = (acc >> lane) & 1ull ? (uint32_t)x.kf : 0u;
+        const uint32_t got = (uint32_t)__shfl((int)k, (int)from, kWave);
+        if (own) out = got;
+        left &= ~__builtin_amdgcn_ballot_w64(own != 0ull);
+        it0 += per;
+    }
+    return out;
+}
+
 __device__ __forceinline__ SourceCount source_count(const SimDesc& sd, const float* dens, Key key, uint32_t c,
                                                     uint32_t flags, uint32_t t, uint32_t k, uint32_t I, uint32_t Mc,
                                                     uint32_t humans) {
     SourceCount o{0u, 0u, 0ull};
     const uint32_t dir = k >> 2, s = k & 3u;
-    if (s >= sd.S || I == 0) return o;
+    const bool none = s >= sd.S || I == 0;
+    if (__builtin_amdgcn_ballot_w64(!none) == 0ull) return o;
     const DayParams dp = day_params(sd, dens, t);
     const float lam = dir == DIR_HM ? (float)Mc / (float)humans * dp.beta_hm * (float)I : dp.beta_mh * (float)I;
     const bool staying = (flags & kCommStay) != 0;
     if (sd.count_law == ARBO_COUNT_STOCH_ROUND) {   // nepidemic.cu:67-104
+        if (none) return o;
         const U4 r = draw(key, c, t, ctr_tag(P_NSR, dir, s, 0), 0);
         uint32_t all = stoch_round(lam, r.x);
         if (staying) o.stay = stoch_round((float)all * sd.no_distance, r.y);
@@ -578,11 +638,12 @@ __device__ __forceinline__ SourceCount source_count(const SimDesc& sd, const flo
         const float mu_ld = go * sd.omega;
         o.fx = (unsigned long long)floor((double)mu_ld * 16777216.0);
         const Stream st{key, c, t, ctr_tag(P_NLOC, dir, s, 0)};
-        o.n = poisson((double)mu_loc, st);
-        if (staying) {
-            const Stream ss{key, c, t, ctr_tag(P_NSTAY, dir, s, 0)};
-            o.stay = poisson((double)(lam * sd.no_distance), ss);
-        }
+        const Stream ss{key, c, t, ctr_tag(P_NSTAY, dir, s, 0)};
+        const uint32_t lane = threadIdx.x & (kWave - 1);
+        if (none) o.fx = 0ull;
+        o.n = wave_poisson(none ? 0.0 : (double)mu_loc, st, lane);
+        if (__builtin_amdgcn_ballot_w64(staying))
+            o.stay = wave_poisson(none || !staying ? 0.0 : (double)(lam * sd.no_distance), ss, lane);
     }
     return o;
 }
@@ -1116,15 +1177,17 @@ void k_day_demography(EngineView v) {
     // ---- event counts of this community as a source ----
     // Small batches draw and spread them here, others in k_day_counts.
     if (SMALL) {
-        if (tid < 8) {
-            const uint32_t dir = tid >> 2, s = tid & 3u;
-            const uint32_t I = dir == DIR_HM ? unpack_pair(ih01, ih23, s) : unpack_pair(im01, im23, s);
-            const SourceCount sc = source_count(sd, v.dens, key, cd.c, cd.flags, t, tid, I, Mc, cd.n);
-            // staying events join the count of the source's own column
-            if (sc.stay) atomicAdd(&s_hist[tid * 9 + ((cd.flags >> kCommSelfShift) & 15u)], sc.stay);
-            s_n[tid] = sc.n;
-            // read by every community of the simulation (no same-address atomics)
-            reinterpret_cast<unsigned long long*>(v.part + (size_t)g * kPartWords + 8)[tid] = sc.fx;
+        if (NW == 1 || wv == 0) {   // one wave, all of its lanes
+            const uint32_t k = lane & 7u, s = lane & 3u;
+            const uint32_t I = lane >= 8 ? 0u : k < 4 ? unpack_pair(ih01, ih23, s) : unpack_pair(im01, im23, s);
+            const SourceCount sc = source_count(sd, v.dens, key, cd.c, cd.flags, t, k, I, Mc, cd.n);
+            if (lane < 8) {
+                // staying events join the count of the source's own column
+                if (sc.stay) atomicAdd(&s_hist[lane * 9 + ((cd.flags >> kCommSelfShift) & 15u)], sc.stay);
+                s_n[lane] = sc.n;
+                // read by every community of the simulation (no same-address atomics)
+                reinterpret_cast<unsigned long long*>(v.part + (size_t)g * kPartWords + 8)[lane] = sc.fx;
+            }
         }
         __syncthreads();
         // Destinations: event i of source segment k takes word i%4 of Philox
@@ -1743,7 +1806,7 @@ __global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
     static_assert(kSeg == 256 && kRows <= 2 * 256, "one segment, at most two CSR entries per thread");
     const CountBlock cb = v.count_map[blockIdx.x];
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-    const uint32_t j = tid >> 3, k = tid & 7u;
+    const uint32_t j = wv + 4u * (lane >> 3), k = tid & 7u;   // dealt to the waves in turn
     __shared__ uint32_t s_hist[kCountComms][kCntPerComm];
     __shared__ uint32_t s_row[kRows], s_box[kRows];   // the communities' CSR rows, one behind the other
     __shared__ uint8_t s_own[kRows];                  // community of each entry
@@ -1786,11 +1849,8 @@ __global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
             s_rl[j] = rl;
         }
     }
-    SourceCount sc{0u, 0u, 0ull};
-    if (in) {
-        const uint32_t I = k < 4 ? unpack_pair(pa.z, pa.w, k) : unpack_pair(pm.x, pm.y, k & 3u);
-        sc = source_count(sd, v.dens, key, c, flags, t, k, I, pa.x, pa.y);
-    }
+    const uint32_t I = k < 4 ? unpack_pair(pa.z, pa.w, k) : unpack_pair(pm.x, pm.y, k & 3u);
+    const SourceCount sc = source_count(sd, v.dens, key, c, flags, t, k, in ? I : 0u, pa.x, pa.y);
     const bool some = __syncthreads_or((int)(sc.n | sc.stay)) != 0;
     if (some) {
         for (uint32_t i = tid; i < cb.n * kCntPerComm; i += 256) (&s_hist[0][0])[i] = 0u;
@@ -1817,7 +1877,7 @@ __global__ __launch_bounds__(256) void k_day_counts(EngineView v) {
                 const uint32_t mid = (lo + hi + 1) >> 1;
                 if (s_q[mid] <= q) lo = mid; else hi = mid - 1;
             }
-            const uint32_t jj = lo >> 3, kk = lo & 7u;
+            const uint32_t jj = (lo >> 6) + 4u * ((lo >> 3) & 7u), kk = lo & 7u;
             spread_quad(key, cb.c0 + jj, t, kk, q - s_q[lo], s_n[lo], s_row + s_off[jj], s_rl[jj], &s_hist[jj][kk * 9]);
         }
         __syncthreads();

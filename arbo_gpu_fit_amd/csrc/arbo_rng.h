@@ -302,7 +302,56 @@ ARBO_HD U4 stream_draw(const Stream& s, uint32_t i) {
 constexpr uint32_t POIS_INV_MAX = 200;     // inversion search cap (mu < 10)
 constexpr uint32_t POIS_PTRS_MAXIT = 256;  // rejection loop cap (mu >= 10)
 
-// Poisson(mu).  mu < 10: sequential-search inversion of one 53-bit uniform.
+// PTRS's constants for a mean mu >= 10.
+struct Ptrs { double mu, loglam, b, a, invalpha, vr; };
+ARBO_HD Ptrs ptrs(double mu) {
+    Ptrs p;
+    p.mu = mu;
+    p.loglam = dlog(mu);
+    const double slam = dexp(0.5 * p.loglam);
+    p.b = 0.931 + 2.53 * slam;
+    p.a = -0.059 + 0.02483 * p.b;
+    p.invalpha = 1.1239 + 1.1328 / (p.b - 3.4);
+    p.vr = 0.9277 - 3.6224 / (p.b - 2.0);
+    return p;
+}
+// One trial: accepted or rejected by the squeeze, or left to ptrs_accept.
+struct PtrsTrial { double kf, us, V; bool sure, open; };
+ARBO_HD PtrsTrial ptrs_trial(const Ptrs& p, const U4& r) {
+    PtrsTrial x;
+    const double U = u53(r.x, r.y) - 0.5;
+    x.V = u53(r.z, r.w);
+    x.us = 0.5 - (U < 0.0 ? -U : U);
+    x.kf = -1.0;
+    x.sure = x.open = false;
+    if (!(x.us > 0.0)) return x;
+    x.kf = floor((2.0 * p.a / x.us + p.b) * U + p.mu + 0.43);
+    const bool in = x.us >= 0.07 && x.V <= p.vr;
+    x.sure = in && !(x.kf < 0.0);
+    x.open = !in && !(x.kf < 0.0 || (x.us < 0.013 && x.V > x.us)) && !(x.kf > 4.0e9);
+    return x;
+}
+ARBO_HD bool ptrs_accept(const Ptrs& p, const PtrsTrial& x) {
+    const double lhs = dlog(x.V) + dlog(p.invalpha) - dlog(p.a / (x.us * x.us) + p.b);
+    const double rhs = -p.mu + x.kf * p.loglam - dlogfact(x.kf);
+    return lhs <= rhs;
+}
+
+// Poisson(mu), 0 < mu < 10: sequential-search inversion of one 53-bit uniform.
+ARBO_HD uint32_t poisson_inversion(double mu, const U4& r) {
+    const double u = u53(r.x, r.y);
+    double p = dexp(-mu);
+    double F = p;
+    uint32_t k = 0;
+    while (u >= F && k < POIS_INV_MAX) {
+        k += 1u;
+        p = p * mu / (double)k;
+        F = F + p;
+    }
+    return k;
+}
+
+// Poisson(mu).  mu < 10: inversion.
 // mu >= 10: PTRS, the transformed rejection with squeeze of W. Hoermann,
 // "The transformed rejection method for generating Poisson random variables",
 // Insurance: Mathematics and Economics 12 (1993), one Philox block per trial.
@@ -310,41 +359,11 @@ constexpr uint32_t POIS_PTRS_MAXIT = 256;  // rejection loop cap (mu >= 10)
 // bit-identical on every platform that runs this code.
 ARBO_HD uint32_t poisson(double mu, const Stream& st) {
     if (!(mu > 0.0)) return 0u;
-    if (mu < 10.0) {
-        const U4 r = stream_draw(st, 0);
-        const double u = u53(r.x, r.y);
-        double p = dexp(-mu);
-        double F = p;
-        uint32_t k = 0;
-        while (u >= F && k < POIS_INV_MAX) {
-            k += 1u;
-            p = p * mu / (double)k;
-            F = F + p;
-        }
-        return k;
-    }
-    const double loglam = dlog(mu);
-    const double slam = dexp(0.5 * loglam);
-    const double b = 0.931 + 2.53 * slam;
-    const double a = -0.059 + 0.02483 * b;
-    const double invalpha = 1.1239 + 1.1328 / (b - 3.4);
-    const double vr = 0.9277 - 3.6224 / (b - 2.0);
+    if (mu < 10.0) return poisson_inversion(mu, stream_draw(st, 0));
+    const Ptrs p = ptrs(mu);
     for (uint32_t it = 0; it < POIS_PTRS_MAXIT; ++it) {
-        const U4 r = stream_draw(st, it);
-        const double U = u53(r.x, r.y) - 0.5;
-        const double V = u53(r.z, r.w);
-        const double us = 0.5 - (U < 0.0 ? -U : U);
-        if (!(us > 0.0)) continue;
-        const double kf = floor((2.0 * a / us + b) * U + mu + 0.43);
-        if (us >= 0.07 && V <= vr) {
-            if (kf < 0.0) continue;
-            return (uint32_t)kf;
-        }
-        if (kf < 0.0 || (us < 0.013 && V > us)) continue;
-        if (kf > 4.0e9) continue;
-        const double lhs = dlog(V) + dlog(invalpha) - dlog(a / (us * us) + b);
-        const double rhs = -mu + kf * loglam - dlogfact(kf);
-        if (lhs <= rhs) return (uint32_t)kf;
+        const PtrsTrial x = ptrs_trial(p, stream_draw(st, it));
+        if (x.sure || (x.open && ptrs_accept(p, x))) return (uint32_t)x.kf;
     }
     return (uint32_t)floor(mu);
 }

@@ -241,6 +241,28 @@ def test_event_counts_of_few_and_many_communities(hip_lib, oracle_lib, grids):
     _both(hip_lib, oracle_lib, specs, 20, checks=(2, 9))
 
 
+@pytest.mark.parametrize("grids,small", [([(1, 1)], True), ([(5, 3), (1, 2)], True), ([(23, 23)], False),
+                                         ([(36, 36), (3, 2)], False), ([(51, 51)], False), ([(72, 72)], False)])
+@pytest.mark.parametrize("serotypes,staying", [(1, 0.0), (4, 0.4)])
+def test_event_counts_on_both_sides_of_the_inversion(hip_lib, oracle_lib, grids, small, serotypes, staying):
+    """Mean event counts from below 1 to several hundred in one wave, so that
+    from one to all of its lanes draw by rejection and share the others' lanes
+    for their trials: in small batches, and in workgroups of 4, 8, 16 and 32
+    communities."""
+    print(f"[edges] rejection {grids} {serotypes} {staying}", flush=True)
+    specs = []
+    for i, (w, h) in enumerate(grids):
+        humans = np.array([1, 3, 17, 60, 400, 9, 130], np.uint32)[(np.arange(w * h) + 4) % 7]
+        p = configs.base_params(n_serotypes=serotypes, beta_hm=0.6, beta_mh=0.5, seed_frac_h=0.15, seed_frac_m=0.1,
+                                long_distance=0.002, no_distance=staying)
+        specs.append(SimSpec(w, h, humans, p, 90 + i))
+    gpu = Engine(hip_lib)
+    gpu.init(specs, 2)
+    assert gpu.launch_shape()["small_batch"] == small
+    gpu.close()
+    _both(hip_lib, oracle_lib, specs, 8, checks=(1, 3))
+
+
 @pytest.mark.parametrize("grids,humans,big", [([(10, 10)], 300, 0), ([(32, 16)], 40, 0), ([(32, 16)] * 5 + [(3, 1)], 9, 0),
                                               ([(2, 2)], 2000, 12000)])
 @pytest.mark.parametrize("climate", [False, True])
