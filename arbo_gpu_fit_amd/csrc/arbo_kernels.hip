@@ -564,7 +564,10 @@ __device__ __forceinline__ double lane_double(double x, uint32_t lane) {
     return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// poisson(mu, st) of every lane of the wave (all of them call; the same key).
+// Poisson(mu) of every lane of the wave (all of them call; the same key):
+// mu < 10 by inversion, else PTRS, one Philox block of the stream per trial.
+// Both are a fixed sequence of IEEE operations, so the result is bit-identical
+// on every platform.
 // A rejection trial is 2 us of dependent double arithmetic and the lane that
 // needs most of them holds up the wave, its workgroup and, in a batch of a few
 // workgroups a CU, the kernel.  The trials of a lane are therefore tried side
@@ -1318,13 +1321,14 @@ static_assert(ARBO_MAX_COMMUNITY_SLOTS + ARBO_MAX_COMMUNITY_HUMANS <= (1u << kKe
               "mosquito and human claim keys fit the key field");
 
 // Number of long-distance events of direction k / 4 and serotype k % 4 from
-// their summed rate (2^-24 units) or count.
+// their summed rate (2^-24 units) or count.  Every lane of a wave calls it,
+// those past the eight pairs with fx = 0.
 __device__ __forceinline__ uint32_t longdist_count(const SimDesc& sd, Key key, uint32_t t, uint32_t k,
                                                    unsigned long long fx) {
-    if ((k & 3u) >= sd.S) return 0u;
+    if ((k & 3u) >= sd.S) fx = 0ull;
     if (sd.count_law == ARBO_COUNT_STOCH_ROUND) return (uint32_t)fx;   // the sources' own long-distance counts
     const Stream st{key, INIT_DAY, t, ctr_tag(P_NLD, k >> 2, k & 3u, 0)};
-    return poisson((double)fx * 0x1p-24, st);
+    return wave_poisson((double)fx * 0x1p-24, st, threadIdx.x & (kWave - 1));
 }
 
 // Community event l of direction k / 4 and serotype k % 4 lands on.
@@ -1420,11 +1424,8 @@ __global__ __launch_bounds__(kWave * NW) void k_day_events(EngineView v) {
         for (uint32_t c = lane >> 3; c < sd.C; c += 8) fx += rate[(size_t)c * (kPartWords / 2)];
 #pragma unroll
         for (uint32_t d = 8; d < kWave; d <<= 1) fx += __shfl_xor(fx, d, kWave);
-        uint32_t L = 0;
-        if (lane < 8) {
-            s_nld[lane] = 0u;
-            L = longdist_count(sd, key, t, lane, fx);
-        }
+        if (lane < 8) s_nld[lane] = 0u;
+        const uint32_t L = longdist_count(sd, key, t, lane & 7u, lane < 8 ? fx : 0ull);
         uint32_t pre[9];
         pre[0] = 0;
 #pragma unroll
@@ -1746,12 +1747,14 @@ __device__ __forceinline__ void longdist_part(const EngineView& v, uint32_t sim,
     __shared__ uint32_t s_L[8];
     // the simulation's sums of today, by k_day_counts
     const unsigned long long* tot = v.totals + ((size_t)(t & 1u) * v.n_totals + sd.total) * kTotalWords;
-    if (tid < 8) {
+    if (tid < kWave) {
         unsigned long long fx = 0;
+        if (tid < 8) {
 #pragma unroll 4
-        for (uint32_t r = 0; r < sd.totals; ++r) fx += tot[r * kTotalWords + tid];
-        const uint32_t L = longdist_count(sd, key, t, tid, fx);
-        s_L[tid] = L;
+            for (uint32_t r = 0; r < sd.totals; ++r) fx += tot[r * kTotalWords + tid];
+        }
+        const uint32_t L = longdist_count(sd, key, t, tid & 7u, fx);
+        if (tid < 8) s_L[tid] = L;
     }
     __syncthreads();
     uint32_t pre[9];

@@ -302,7 +302,10 @@ ARBO_HD U4 stream_draw(const Stream& s, uint32_t i) {
 constexpr uint32_t POIS_INV_MAX = 200;     // inversion search cap (mu < 10)
 constexpr uint32_t POIS_PTRS_MAXIT = 256;  // rejection loop cap (mu >= 10)
 
-// PTRS's constants for a mean mu >= 10.
+// PTRS, the transformed rejection with squeeze of W. Hoermann, "The
+// transformed rejection method for generating Poisson random variables",
+// Insurance: Mathematics and Economics 12 (1993): the constants for a mean
+// mu >= 10.
 struct Ptrs { double mu, loglam, b, a, invalpha, vr; };
 ARBO_HD Ptrs ptrs(double mu) {
     Ptrs p;
@@ -349,23 +352,6 @@ ARBO_HD uint32_t poisson_inversion(double mu, const U4& r) {
         F = F + p;
     }
     return k;
-}
-
-// Poisson(mu).  mu < 10: inversion.
-// mu >= 10: PTRS, the transformed rejection with squeeze of W. Hoermann,
-// "The transformed rejection method for generating Poisson random variables",
-// Insurance: Mathematics and Economics 12 (1993), one Philox block per trial.
-// Both branches are a fixed sequence of IEEE operations, so the result is
-// bit-identical on every platform that runs this code.
-ARBO_HD uint32_t poisson(double mu, const Stream& st) {
-    if (!(mu > 0.0)) return 0u;
-    if (mu < 10.0) return poisson_inversion(mu, stream_draw(st, 0));
-    const Ptrs p = ptrs(mu);
-    for (uint32_t it = 0; it < POIS_PTRS_MAXIT; ++it) {
-        const PtrsTrial x = ptrs_trial(p, stream_draw(st, it));
-        if (x.sure || (x.open && ptrs_accept(p, x))) return (uint32_t)x.kf;
-    }
-    return (uint32_t)floor(mu);
 }
 
 }  // namespace arbo
