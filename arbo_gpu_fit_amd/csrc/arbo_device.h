@@ -209,20 +209,22 @@ struct EngineView {
 // long-distance events, so all of these are bounded; us a day with it and
 // without:
 //  * C (the sums): one simulation of 484 communities of 200 and of 1,000
-//    humans 33.1 and 34.8, 43.4 and 52.8; 529 34.7 and 35.4, 44.6 and 52.8; 676
-//    36.6 and 36.0, 47.0 and 53.8; 1,024 41.1 and 36.9, 53.4 and 55.8;
+//    humans 32.0 and 32.6, 39.1 and 44.6; 529 33.2 and 33.5, 40.3 and 44.7; 676
+//    35.5 and 34.2, 42.3 and 45.9; 1,024 40.8 and 34.9, 47.8 and 46.3;
 //  * communities in all, whose waves have to run side by side for the repeated
 //    work to cost only its latency: 28 simulations of 144 communities of 200 and
-//    of 1,000 humans (4,032) 41.4 and 43.5, 68.7 and 71.2; 36 (5,184) 48.0 and
-//    48.7, 80.4 and 79.6; 44 (6,336) 55.7 and 54.1, 93.9 and 89.8;
+//    of 1,000 humans (4,032) 41.0 and 41.0, 62.8 and 63.5; 36 (5,184) 48.0 and
+//    47.0, 74.5 and 75.2; 44 (6,336) 55.1 and 52.1, 89.6 and 86.8;
 //  * the long-distance events: in proportion to omega, the transmission rates
 //    and the mosquitoes, sent = omega x slots x (beta_hm + beta_mh), a wave's
 //    share of them where a community has several, and times the waves per SIMD
-//    that redraw them.  100 communities of 1,000 humans at 21,000 sent 46.7 and
-//    50.3, 36,000 50.1 and 51.6, 84,000 70.4 and 51.9; 484 at 8,700 51.1 and
-//    56.2, 20,300 54.1 and 53.8, 43,600 60.8 and 56.3; 16 x 144 at 13,600 67.9
-//    and 70.7, 23,300 71.6 and 73.6, 29,200 73.8 and 74.1, 68,000 83.3 and 71.6;
-//    10 x 400 at 14,100 50.0 and 48.7, 28,100 88.9 and 84.2, 65,600 93.4 and 82.5.
+//    that redraw them.  At rates of 0.7, 100 communities of 1,000 humans at
+//    12,600 sent 47.4 and 53.7, 25,200 54.2 and 54.5, 42,000 62.8 and 54.8; 484
+//    at 10,200 52.8 and 55.8, 18,300 57.3 and 56.3, 24,400 60.6 and 56.3; 16 x
+//    144 at 6,800 71.5 and 73.2, 13,600 73.8 and 73.1, 27,200 78.5 and 73.0; at
+//    0.15, without an epidemic, 22.0 and 28.5, 27.6 and 30.8, 33.4 and 36.2.  10
+//    x 400 of 400 humans, the most sums that the limits admit, 68.3 and 63.3
+//    at 2,600 sent, 34.8 and 33.1 without an epidemic.
 constexpr uint32_t kSmallCommunities = 4096;
 constexpr uint32_t kSmallSimulation = 512;
 constexpr float kSmallSent = 24000.0f;

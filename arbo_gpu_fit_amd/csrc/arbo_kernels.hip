@@ -2074,10 +2074,10 @@ hipError_t launch_init(const EngineView& v, uint32_t largest, hipStream_t st) {
 // of so few communities and their registers make no difference).  A tuning
 // that nobody set leaves the number to the batch: up to 1,024 communities get
 // four waves, a SIMD's four then being one community's.  One wave and four, us
-// a day: 100 communities of 1,000 humans 35.5 and 32.0, 484 43.7 and 40.3,
-// 1,000 42.4 and 39.7; 2,304 of 400 humans 36.7 and 44.0, 4,000 of 1,000
-// humans 62.2 and 78.1; 100 of 200 humans 23.2 and 22.9.  Eight waves are no
-// better than four up to 400 communities and slower from 484 on.
+// a day: 100 communities of 1,000 humans 35.4 and 30.8, 484 43.8 and 39.1,
+// 1,000 (10 simulations) 40.1 and 36.9; 2,304 of 400 humans 39.2 and 48.7,
+// 4,000 of 1,000 humans 68.0 and 91.3; 100 of 200 humans 27.3 and 27.0.  Eight
+// waves are no better than four up to 400 communities and slower from 484 on.
 constexpr uint32_t kWideCommunities = 1024;
 
 uint32_t demography_waves(const EngineView& v, const Tuning& tu) {
